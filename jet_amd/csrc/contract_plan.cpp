@@ -498,3 +498,16 @@ void layout_workspace(ContractionDesc &d)
 }
 
 } // namespace jet_hip
+    d.slices = 1;
+    if ((d.gemm_kernel == kGemmBf16x4m || d.gemm_kernel == kGemmF16x4m) && d.chunks == 1) {
+        const int64_t n = x4m_slices(d.M, d.N, d.K, d.batch, d.gemm_variant);
+        const size_t bytes = align256(eb * (size_t)n * (size_t)d.size_c);
+        // a plan that fits the no-allocation scratch array keeps doing so
+        const bool fits = off > JET_HIP_NOALLOC_SCRATCH_BYTES ||
+                          off + bytes <= JET_HIP_NOALLOC_SCRATCH_BYTES;
+        if (n > 1 && fits) {
+            d.slices = n;
+            d.off_slices = off;
+            off += bytes;
+        }
+    }

@@ -53,6 +53,8 @@ struct ContractionDesc {
     size_t off_rmax_a = 0, off_scale_a = 0, off_rmax_b = 0, off_scale_b = 0;
     int64_t split_a_plane = 0, split_b_plane = 0;
     size_t workspace = 0;
+    int64_t slices = 1;    // slices of k of a 4M split GEMM (x4m_slices)
+    size_t off_slices = 0; // their results (slices > 1)
     double flops = 0; // 8 * batch * M * N * K
 };
 

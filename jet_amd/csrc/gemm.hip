@@ -1179,7 +1179,7 @@ template <> struct Mfma16<_Float16> {
 template <class E, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void cgemm_x4m_kernel(
     SplitOperand a, SplitOperand b, float2 *__restrict__ Cout, int64_t M,
-    int64_t N, int64_t ldc, int64_t sC, int a_bcast, int b_bcast)
+    int64_t N, int64_t ldc, int64_t sC, int a_bcast, int b_bcast, int slice_kt, int64_t slice_stride)
 {
     using vec = typename Mfma16<E>::vec;
     typedef __attribute__((address_space(3))) void lds_void;
@@ -1224,6 +1224,8 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_x4m_kernel(
                                              (lds_void *)(as + (wave * A_IN + i) * 64), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < B_IN; i++)
+// blockIdx.y takes slice_kt k tiles each and writes its own result at
+// slice_stride (x4m_slices).
             __builtin_amdgcn_global_load_lds((const void *)(Bt + uint64_t(offb[i] + kb)),
                                              (lds_void *)(bs + (wave * B_IN + i) * 64), 16, 0, 0);
     };
@@ -1280,11 +1282,12 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_x4m_kernel(
     // vmcnt(0) (expcnt and lgkmcnt left at their maximum): this wave's
     // direct-to-LDS loads have landed; the barrier then covers all waves.
     constexpr int kWaitLoads = 0x0f70;
-    const int nk = int(a.k_p / KT);
-    issue(0, As0, Bs0);
+    const int kt0 = int(blockIdx.y) * slice_kt;
+    const int nk = min(int(a.k_p / KT), kt0 + slice_kt);
+    issue(kt0, As0, Bs0);
     __builtin_amdgcn_s_waitcnt(kWaitLoads);
     __syncthreads();
-    for (int kt = 0; kt < nk; kt += 2) {
+    for (int kt = kt0; kt < nk; kt += 2) {
         if (kt + 1 < nk) issue(kt + 1, As1, Bs1);
         compute(As0, Bs0);
         __builtin_amdgcn_s_waitcnt(kWaitLoads);
@@ -1296,7 +1299,7 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_x4m_kernel(
         __syncthreads();
     }
 
-    float2 *C = Cout + bz * sC;
+    float2 *C = Cout + bz * sC + int64_t(blockIdx.y) * slice_stride;
     const float *sa = a.scale ? a.scale + (a_bcast ? 0 : bz) * a.rows_p : nullptr;
     const float *sb = b.scale ? b.scale + (b_bcast ? 0 : bz) * b.rows_p : nullptr;
 #pragma unroll
@@ -2019,7 +2022,7 @@ constexpr int kX4mWideN = 4096;
 template <class E>
 void launch_x4m(const SplitOperand &a, const SplitOperand &b, void *C, int64_t M, int64_t N,
                 int64_t ldc, int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
-                hipStream_t stream, int variant)
+                hipStream_t stream, int variant, int64_t slices)
 {
     constexpr int BM = 128, WM = 2, WN = 4;
     JH_REQUIRE(a.k_p <= kX4mMaxK, "k exceeds the 4M split kernels' limit (2^21).");
@@ -2052,7 +2055,7 @@ void launch_x4m(const SplitOperand &a, const SplitOperand &b, void *C, int64_t M
         JH_HIP(hipGetLastError());
         return;
     }
-    const int BN = variant == 1 ? 128 : variant == 2 ? 192 : N >= kX4mWideN ? 192 : 128;
+    const int BN = variant == 1 || slices > 1 ? 128 : variant == 2 ? 192 : N >= kX4mWideN ? 192 : 128;
     JH_REQUIRE(ceil_div(M, BM) * ceil_div(N, BN) <= 0x7fffffff, "Too many tiles.");
     dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), 1, (unsigned)batch);
     if (BN == 192) {
@@ -2063,30 +2066,32 @@ void launch_x4m(const SplitOperand &a, const SplitOperand &b, void *C, int64_t M
     else
         hipLaunchKernelGGL((cgemm_x4m_kernel<E, BM, 128, WM, WN>), grid, dim3(64 * WM * WN), 0,
                            stream, a, b, static_cast<float2 *>(C), M, N, ldc, sC,
-                           a_bcast ? 1 : 0, b_bcast ? 1 : 0);
+                           a_bcast ? 1 : 0, b_bcast ? 1 : 0,
+                           int(ceil_div(a.k_p / kSplitKPad, slices)), batch * M * N);
     JH_HIP(hipGetLastError());
 }
 
 void launch_gemm_f16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K_true,
                         void *C, int64_t M, int64_t N, int64_t ldc,
                         int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
-                        hipStream_t stream, int variant)
+                        hipStream_t stream, int variant, int64_t slices)
 {
     JH_REQUIRE(a.k_p == b.k_p, "Split operands disagree on k.");
     JH_REQUIRE(a.planes == 4 && b.planes == 4 && a.interleaved && b.interleaved && a.scale &&
+    JH_REQUIRE(slices == 1 || variant <= 1, "Only the 128x128 form takes slices of k.");
                    b.scale,
                "The split-FP16 kernel needs four interleaved planes and row scales.");
     JH_REQUIRE(batch <= 65535, "Batch count exceeds 65535.");
     const double K = double(K_true);
     prof::Scope ps(prof::kGemmF16x4m, stream, 8.0 * double(batch) * double(M) * double(N) * K,
                    8.0 * double(batch) * (double(M) * K + double(N) * K + double(M) * double(N)));
-    launch_x4m<_Float16>(a, b, C, M, N, ldc, sC, batch, a_bcast, b_bcast, stream, variant);
+    launch_x4m<_Float16>(a, b, C, M, N, ldc, sC, batch, a_bcast, b_bcast, stream, variant, slices);
 }
 
 void launch_gemm_bf16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K_true,
                          void *C, int64_t M, int64_t N, int64_t ldc,
                          int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
-                         hipStream_t stream, int variant)
+                         hipStream_t stream, int variant, int64_t slices)
 {
     JH_REQUIRE(a.k_p == b.k_p, "Split operands disagree on k.");
     JH_REQUIRE(a.planes == 4 && b.planes == 4 && a.interleaved && b.interleaved,
@@ -2096,7 +2101,7 @@ void launch_gemm_bf16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K
     const double K = double(K_true);
     prof::Scope ps(prof::kGemmBf16x4m, stream, 8.0 * double(batch) * double(M) * double(N) * K,
                    8.0 * double(batch) * (double(M) * K + double(N) * K + double(M) * double(N)));
-    launch_x4m<__bf16>(a, b, C, M, N, ldc, sC, batch, a_bcast, b_bcast, stream, variant);
+    launch_x4m<__bf16>(a, b, C, M, N, ldc, sC, batch, a_bcast, b_bcast, stream, variant, slices);
 }
 
 void launch_fused_small(const FusedSmall &f, int elem_bytes, const void *a, const void *b,
@@ -2144,7 +2149,7 @@ void launch_gemm_bf16x3(const SplitOperand &a, const SplitOperand &b, int64_t K_
                "The 3M kernel needs six planar planes.");
     JH_REQUIRE(batch <= 65535, "Batch count exceeds 65535.");
     JH_REQUIRE(ceil_div(M, BM) * ceil_div(N, BN) <= 0x7fffffff, "Too many tiles.");
-    dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), 1, (unsigned)batch);
+    dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), (unsigned)slices, (unsigned)batch);
     const double K = double(K_true);
     prof::Scope ps(prof::kGemmBf16x3, stream, 8.0 * double(batch) * double(M) * double(N) * K,
                    8.0 * double(batch) * (double(M) * K + double(N) * K + double(M) * double(N)));

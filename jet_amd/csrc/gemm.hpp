@@ -77,6 +77,19 @@ inline int64_t splitk_partials(int64_t outputs, int64_t K)
 constexpr int kSplitRowPad = 16;
 constexpr int kSplitKPad = 32;
 // Longest padded k of the 4M split kernels: their per-lane load offsets
+// 4M split products with few 128x128 tiles: slices of k (at least 256 each)
+// that fill the 256 CUs, each slice a result of its own, summed afterwards in
+// FP64 (launch_sum_chunks).  One slice where half the CUs have a tile
+// already, or for the other tile forms (variant > 1).
+inline int64_t x4m_slices(int64_t M, int64_t N, int64_t K, int64_t batch, int variant)
+{
+    const int64_t tiles = ceil_div(M, 128) * ceil_div(N, 128) * batch;
+    const int64_t kt = ceil_div(K, 32);
+    if (variant > 1 || tiles > 128 || kt < 16) return 1;
+    const int64_t want = 256 / tiles < kt / 8 ? 256 / tiles : kt / 8;
+    return ceil_div(kt, ceil_div(kt, want)); // no slice empty
+}
+
 // within a tile of up to 192 operand rows stay below 2^32 bytes.
 constexpr int64_t kX4mMaxK = int64_t(1) << 21;
 
@@ -162,7 +175,7 @@ void launch_split_bf16(const void *src, int64_t rows, int64_t k, int64_t ld,
 void launch_gemm_bf16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K_true,
                          void *C, int64_t M, int64_t N, int64_t ldc,
                          int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
-                         hipStream_t stream, int variant = 0);
+                         hipStream_t stream, int variant = 0, int64_t slices = 1);
 // Row maxima then the scaled fp16 planes of a split-FP16 operand.
 void launch_split_f16(const void *src, int64_t rows, int64_t k, int64_t ld,
                       int64_t s, int64_t batch, const SplitOperand &dst,
@@ -173,7 +186,15 @@ void launch_split_f16_gather(const void *src, const SplitGather &g, const SplitO
 void launch_gemm_f16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K_true,
                         void *C, int64_t M, int64_t N, int64_t ldc,
                         int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
-                        hipStream_t stream, int variant = 0);
+                        hipStream_t stream, int variant = 0, int64_t slices = 1);
+// n_blocks consecutive blocks of one group; `pointers` is the device table
+// that their slots index.
+void launch_grouped_small(const GroupBlock *blocks, int n_blocks, const void *const *pointers,
+                          int elem_bytes, double flops, hipStream_t stream);
+// pointers[first + i] = values[i] on the device, in stream order (the values
+// travel as kernel arguments).
+void launch_set_pointers(const void **pointers, const void *const *values, int n,
+                         hipStream_t stream);
 void launch_gemm_bf16x3(const SplitOperand &a, const SplitOperand &b, int64_t K_true,
                         void *C, int64_t M, int64_t N, int64_t ldc,
                         int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,

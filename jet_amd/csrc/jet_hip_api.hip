@@ -156,9 +156,11 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
         Bt = ws + d.off_bt;
     }
     void *Ct = d.need_c ? static_cast<void *>(ws + d.off_ct) : c;
-    // K split into batched chunks: the GEMM writes each chunk's result,
-    // then they are summed into Ct.
-    void *Cg = d.chunks > 1 ? static_cast<void *>(ws + d.off_chunks) : Ct;
+    // K split into batched chunks or slices: the GEMM writes each one's
+    // result, then they are summed into Ct.
+    void *Cg = d.chunks > 1   ? static_cast<void *>(ws + d.off_chunks)
+               : d.slices > 1 ? static_cast<void *>(ws + d.off_slices)
+                              : Ct;
     if (d.gemm_kernel == kGemmBf16x3 || d.gemm_kernel == kGemmBf16x4m ||
         d.gemm_kernel == kGemmF16x4m) {
         const int planes = d.gemm_kernel == kGemmBf16x3 ? 6 : 4;
@@ -182,7 +184,7 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
             else
                 launch_split_f16(Bt, d.N, d.K, d.K, d.N * d.K, d.batch, sb, s);
             launch_gemm_f16x4m(sa, sb, d.K, Cg, d.M, d.N, d.N, d.M * d.N, d.batch, false, false, s,
-                               d.gemm_variant);
+                               d.gemm_variant, d.slices);
         }
         else {
             launch_split_bf16(At, d.M, d.K, d.K, d.M * d.K, d.batch, sa, s);
@@ -192,7 +194,7 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
                                    false, s);
             else
                 launch_gemm_bf16x4m(sa, sb, d.K, Cg, d.M, d.N, d.N, d.M * d.N, d.batch, false,
-                                    false, s, d.gemm_variant);
+                                    false, s, d.gemm_variant, d.slices);
         }
     }
     else {
@@ -213,7 +215,8 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
         g.variant = d.gemm_variant;
         launch_gemm(d.gemm_kernel, eb, g, s, ws + d.off_partials);
     }
-    if (d.chunks > 1) launch_sum_chunks(eb, Cg, Ct, d.size_c, d.chunks, s);
+    if (d.chunks > 1 || d.slices > 1)
+        launch_sum_chunks(eb, Cg, Ct, d.size_c, d.chunks * d.slices, s);
     if (d.need_c) launch_permute(d.pc, eb, Ct, c, s);
 }
 
