@@ -59,7 +59,7 @@ typedef enum {
     JET_HIP_PREC_DEFAULT = 0, /* FP32 for C64, FP64 for C128 (the reference's
                                  CUTENSOR_COMPUTE_32F / _64F,
                                  include/jet/CudaTensor.hpp:494-502)          */
-    JET_HIP_PREC_FP32 = 1,    /* 4M complex GEMM on FP32 MFMA                  */
+    JET_HIP_PREC_FP32 = 1,    /* 4M complex GEMM, FP32 products and sums        */
     JET_HIP_PREC_BF16X3 = 2,  /* 3M complex GEMM, each FP32 operand split into
                                  hi+lo BF16, three BF16 MFMA products per real
                                  product, FP32 accumulation.  C64 only.  Steps
@@ -175,9 +175,12 @@ int jet_hip_contract_noalloc(jet_hip_plan_t plan, const void *a,
  *      cutensorInitContractionPlan, include/jet/CudaTensor.hpp:616-640).
  *
  * Kernel ids (jet_hip_plan_info's gemm_kernel): 0 VALU per output, 1 VALU
- * block reduction, 2 FP32 MFMA, 3 FP64 MFMA, 4 split-BF16 3M, 5 split-BF16
+ * block reduction, 2 FP32 products on the matrix cores (six BF16 MFMA
+ * products of three-piece operands; FP32 MFMA where k, M or N is
+ * below 16), 3 FP64 MFMA, 4 split-BF16 3M, 5 split-BF16
  * 4M, 6 split-K with FP64 partials, 7 split-FP16 4M.  Variants: kernel 2
- * 1 = 128x128 / 2 = 64x128 / 3 = 128x64 block tiles; kernels 5 and 7
+ * 1 = 128x128 / 2 = 64x128 / 3 = 128x64 block tiles of its FP32 MFMA form;
+ * kernels 5 and 7
  * 1 = 128x128 / 2 = 128x192 block tiles / 3 = 128x128 tiles walked by a
  * persistent grid of one work-group per CU / 4 = 192x128 block tiles (long
  * side along M); kernel 0 1 = one thread per output

@@ -24,6 +24,7 @@ LIB = os.path.join(LIBDIR, "libjet_hip.so")
 SOURCES = [
     "permute.hip",
     "gemm.hip",
+    "gemm_f32x6.hip",
     "misc.hip",
     "profiler.hip",
     "network.hip",

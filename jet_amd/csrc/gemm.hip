@@ -21,6 +21,7 @@
 //  * VALU kernels for shapes too small or skinny for MFMA tiles.
 #include "common.hpp"
 #include "gemm.hpp"
+#include "gemm_device.hpp"
 #include "profiler.hpp"
 
 #include <algorithm>
@@ -57,30 +58,6 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
 __device__ __forceinline__ f64x4 mfma4(double a, double b, f64x4 c)
 {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
-// Map the linear work-group id to an output tile.  Work-groups are dispatched
-// round-robin over the 8 XCDs (each with its own L2), so first give every XCD
-// a contiguous range of tile indices, then order tiles in groups of
-// kGroupM tile-rows so that the work-groups resident on one XCD share A and B
-// panels in its L2.
-constexpr int kXcds = 8;
-constexpr int kGroupM = 8;
-
-__device__ __forceinline__ void tile_coords(int64_t id, int64_t tiles_m, int64_t tiles_n,
-                                            int64_t &tm, int64_t &tn)
-{
-    const int64_t total = tiles_m * tiles_n;
-    const int64_t q = total / kXcds, r = total % kXcds;
-    const int64_t x = id % kXcds, k = id / kXcds;
-    const int64_t j = x * q + (x < r ? x : r) + k;
-    const int64_t per_group = int64_t(kGroupM) * tiles_n;
-    const int64_t group = j / per_group;
-    const int64_t first_m = group * kGroupM;
-    const int64_t gsz = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
-    const int64_t w = j % per_group;
-    tm = first_m + w % gsz;
-    tn = w / gsz;
 }
 
 // ---------------------------------------------------------------------------
@@ -344,6 +321,77 @@ __global__ __launch_bounds__(256) void fused_small_red_kernel(const void *Av, co
                    (red_s[1][0] + red_s[1][1]) + (red_s[1][2] + red_s[1][3])};
         __syncthreads();
     }
+}
+
+// Independent small contractions of one dependency level in one launch: a
+// circuit's network has hundreds of steps of a few dozen values, and each as
+// a launch of its own costs 3-4 us of launch and memory latency, one after
+// the other.  The block's record is staged in LDS (one load per thread: read in
+// place, its byte-sized bit positions would be a chain of vector loads), the k offsets are
+// tabulated as in fused_small_kernel, 2^lanes lanes share an output's k and
+// add their sums with shuffles.  Measured: 1556 steps of the 6x6 depth-10
+// loss and gradient 8.9 ms as single launches -> see launch_grouped_small.
+template <class R>
+__global__ __launch_bounds__(256) void grouped_small_kernel(const GroupBlock *__restrict__ blocks,
+                                                            const void *const *__restrict__ ptrs)
+{
+    using C2 = typename Vec<R>::c;
+    __shared__ int32_t record[sizeof(GroupBlock) / 4];
+    const GroupBlock &g = *reinterpret_cast<const GroupBlock *>(record);
+    __shared__ const void *base[3];
+    __shared__ int32_t ka[1 << kGroupMaxLog2K], kb[1 << kGroupMaxLog2K];
+    static_assert(sizeof(GroupBlock) % 4 == 0 && sizeof(GroupBlock) / 4 <= 256, "record");
+    const int tid = threadIdx.x;
+    if (tid < int(sizeof(GroupBlock) / 4))
+        record[tid] = reinterpret_cast<const int32_t *>(blocks + blockIdx.x)[tid];
+    __syncthreads();
+    if (tid < 3) base[tid] = ptrs[tid == 0 ? g.a : tid == 1 ? g.b : g.c];
+    const int K = 1 << g.f.lk;
+    for (int k = tid; k < K; k += 256) {
+        ka[k] = int32_t(fused_offset(g.f.a_k, k));
+        kb[k] = int32_t(fused_offset(g.f.b_k, k));
+    }
+    __syncthreads();
+    const int lanes = g.lanes, G = 1 << lanes;
+    const int idx = g.first + (tid >> lanes);
+    const bool live = idx < 1 << (g.f.lb + g.f.lm + g.f.ln);
+    const int n = idx & ((1 << g.f.ln) - 1);
+    const int m = (idx >> g.f.ln) & ((1 << g.f.lm) - 1);
+    const int b = idx >> (g.f.ln + g.f.lm);
+    R sr = 0, si = 0;
+    if (live) {
+        const C2 *x = static_cast<const C2 *>(base[0]) +
+                      (fused_offset(g.f.a_b, b) | fused_offset(g.f.a_m, m));
+        const C2 *y = static_cast<const C2 *>(base[1]) +
+                      (fused_offset(g.f.b_b, b) | fused_offset(g.f.b_n, n));
+#pragma unroll 4
+        for (int k = tid & (G - 1); k < K; k += G) {
+            const C2 u = x[ka[k]], v = y[kb[k]];
+            sr = fma(u.x, v.x, sr);
+            sr = fma(-u.y, v.y, sr);
+            si = fma(u.x, v.y, si);
+            si = fma(u.y, v.x, si);
+        }
+    }
+    for (int off = G >> 1; off > 0; off >>= 1) {
+        sr += __shfl_xor(sr, off);
+        si += __shfl_xor(si, off);
+    }
+    if (live && (tid & (G - 1)) == 0)
+        static_cast<C2 *>(const_cast<void *>(
+            base[2]))[fused_offset(g.f.c_b, b) | fused_offset(g.f.c_m, m) |
+                      fused_offset(g.f.c_n, n)] = C2{sr, si};
+}
+
+constexpr int kPointersPerLaunch = 448; // 3.5 KiB of kernel arguments
+struct PointerChunk {
+    const void *p[kPointersPerLaunch];
+};
+__global__ __launch_bounds__(kPointersPerLaunch) void set_pointers_kernel(const void **table,
+                                                                          PointerChunk v, int n)
+{
+    const int i = threadIdx.x;
+    if (i < n) table[i] = v.p[i];
 }
 
 // Short-K products (K <= kShortK) with many outputs are bound by writing C.
@@ -1176,6 +1224,8 @@ template <> struct Mfma16<_Float16> {
 // Rows past the padded operand are read from its last row: they only feed
 // output rows or columns that are not stored.  Two LDS buffers (128 KiB):
 // the next k tile streams in while the current one is multiplied.
+// blockIdx.y takes slice_kt k tiles each and writes its own result at
+// slice_stride (x4m_slices).
 template <class E, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void cgemm_x4m_kernel(
     SplitOperand a, SplitOperand b, float2 *__restrict__ Cout, int64_t M,
@@ -1224,8 +1274,6 @@ __global__ __launch_bounds__(64 * WM * WN) void cgemm_x4m_kernel(
                                              (lds_void *)(as + (wave * A_IN + i) * 64), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < B_IN; i++)
-// blockIdx.y takes slice_kt k tiles each and writes its own result at
-// slice_stride (x4m_slices).
             __builtin_amdgcn_global_load_lds((const void *)(Bt + uint64_t(offb[i] + kb)),
                                              (lds_void *)(bs + (wave * B_IN + i) * 64), 16, 0, 0);
     };
@@ -1894,6 +1942,10 @@ void launch_gemm(int kernel, int elem_bytes, const GemmArgs &g,
         JH_REQUIRE(ceil_div(g.M, BM) * ceil_div(g.N, BN) <= 0x7fffffff, "Too many tiles.");
         dim3 grid((unsigned)(ceil_div(g.M, BM) * ceil_div(g.N, BN)), 1, (unsigned)g.batch);
         prof::Scope ps(prof::kGemmF32, stream, gemm_flops(g), gemm_bytes(g, 8));
+        if (f32x6_applies(g)) {
+            launch_f32x6(g, stream);
+            return;
+        }
         if (BN == 64)
             hipLaunchKernelGGL((cgemm_embed_kernel<float, 128, 64, 16, 2, 2>), grid, dim3(256), 0,
                                stream, g);
@@ -2025,6 +2077,7 @@ void launch_x4m(const SplitOperand &a, const SplitOperand &b, void *C, int64_t M
                 hipStream_t stream, int variant, int64_t slices)
 {
     constexpr int BM = 128, WM = 2, WN = 4;
+    JH_REQUIRE(slices == 1 || variant <= 1, "Only the 128x128 form takes slices of k.");
     JH_REQUIRE(a.k_p <= kX4mMaxK, "k exceeds the 4M split kernels' limit (2^21).");
     if (variant == 3) {
         // Persistent 128x128 tiles: one work-group per CU, the grid a
@@ -2057,7 +2110,7 @@ void launch_x4m(const SplitOperand &a, const SplitOperand &b, void *C, int64_t M
     }
     const int BN = variant == 1 || slices > 1 ? 128 : variant == 2 ? 192 : N >= kX4mWideN ? 192 : 128;
     JH_REQUIRE(ceil_div(M, BM) * ceil_div(N, BN) <= 0x7fffffff, "Too many tiles.");
-    dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), 1, (unsigned)batch);
+    dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), (unsigned)slices, (unsigned)batch);
     if (BN == 192) {
         hipLaunchKernelGGL((cgemm_x4m_wide_kernel<E, BM, 192, WM, WN>), grid, dim3(64 * WM * WN),
                            0, stream, a, b, static_cast<float2 *>(C), M, N, ldc, sC,
@@ -2078,7 +2131,6 @@ void launch_gemm_f16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K_
 {
     JH_REQUIRE(a.k_p == b.k_p, "Split operands disagree on k.");
     JH_REQUIRE(a.planes == 4 && b.planes == 4 && a.interleaved && b.interleaved && a.scale &&
-    JH_REQUIRE(slices == 1 || variant <= 1, "Only the 128x128 form takes slices of k.");
                    b.scale,
                "The split-FP16 kernel needs four interleaved planes and row scales.");
     JH_REQUIRE(batch <= 65535, "Batch count exceeds 65535.");
@@ -2138,6 +2190,32 @@ void launch_fused_small(const FusedSmall &f, int elem_bytes, const void *a, cons
     JH_HIP(hipGetLastError());
 }
 
+void launch_grouped_small(const GroupBlock *blocks, int n_blocks, const void *const *pointers,
+                          int elem_bytes, double flops, hipStream_t stream)
+{
+    prof::Scope ps(prof::kGemmSmall, stream, flops, 0.0);
+    if (elem_bytes == 8)
+        hipLaunchKernelGGL(grouped_small_kernel<float>, dim3((unsigned)n_blocks), dim3(256), 0,
+                           stream, blocks, pointers);
+    else
+        hipLaunchKernelGGL(grouped_small_kernel<double>, dim3((unsigned)n_blocks), dim3(256), 0,
+                           stream, blocks, pointers);
+    JH_HIP(hipGetLastError());
+}
+
+void launch_set_pointers(const void **pointers, const void *const *values, int n,
+                         hipStream_t stream)
+{
+    for (int first = 0; first < n; first += kPointersPerLaunch) {
+        PointerChunk v{};
+        const int count = std::min(kPointersPerLaunch, n - first);
+        std::copy(values + first, values + first + count, v.p);
+        hipLaunchKernelGGL(set_pointers_kernel, dim3(1), dim3(kPointersPerLaunch), 0, stream,
+                           pointers + first, v, count);
+    }
+    JH_HIP(hipGetLastError());
+}
+
 void launch_gemm_bf16x3(const SplitOperand &a, const SplitOperand &b, int64_t K_true,
                         void *C, int64_t M, int64_t N, int64_t ldc,
                         int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
@@ -2149,7 +2227,7 @@ void launch_gemm_bf16x3(const SplitOperand &a, const SplitOperand &b, int64_t K_
                "The 3M kernel needs six planar planes.");
     JH_REQUIRE(batch <= 65535, "Batch count exceeds 65535.");
     JH_REQUIRE(ceil_div(M, BM) * ceil_div(N, BN) <= 0x7fffffff, "Too many tiles.");
-    dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), (unsigned)slices, (unsigned)batch);
+    dim3 grid((unsigned)(ceil_div(M, BM) * ceil_div(N, BN)), 1, (unsigned)batch);
     const double K = double(K_true);
     prof::Scope ps(prof::kGemmBf16x3, stream, 8.0 * double(batch) * double(M) * double(N) * K,
                    8.0 * double(batch) * (double(M) * K + double(N) * K + double(M) * double(N)));

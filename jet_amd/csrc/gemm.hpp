@@ -28,7 +28,10 @@ struct GemmArgs {
 enum GemmKernel {
     kGemmSmall = 0,     // VALU, one thread per output element
     kGemmSmallRed = 1,  // VALU, one block per output element (long K)
-    kGemmF32Mfma = 2,   // 4M complex on v_mfma_f32_16x16x4_f32
+    kGemmF32Mfma = 2,   // FP32 products on the matrix cores: three BF16 pieces of
+                        // each value and six products (gemm_f32x6.hip), or 4M
+                        // complex on v_mfma_f32_16x16x4_f32 where that does
+                        // not apply (k, M or N < 16)
     kGemmF64Mfma = 3,   // 4M complex on v_mfma_f64_16x16x4_f64
     kGemmBf16x3 = 4,    // 3M complex, split-BF16, v_mfma_f32_16x16x32_bf16
     kGemmBf16x4m = 5,   // 4M complex, split-BF16, v_mfma_f32_16x16x32_bf16
@@ -40,7 +43,8 @@ enum GemmKernel {
 
 // A GEMM kernel family and its tile (or thread-mapping) variant.  Variant 0
 // lets the launcher pick by shape; the others force one form:
-//   kGemmF32Mfma              1: 128x128  2: 64x128  3: 128x64 block tiles
+//   kGemmF32Mfma              1: 128x128  2: 64x128  3: 128x64 block tiles of
+//                             the FP32 MFMA kernel
 //   kGemmF64Mfma              1: 128x64 block tiles
 //   kGemmBf16x4m, kGemmF16x4m 1: 128x128  2: 128x192 block tiles
 //                             3: 128x128 persistent (one work-group per
@@ -73,10 +77,6 @@ inline int64_t splitk_partials(int64_t outputs, int64_t K)
     return outputs * ceil_div(K, splitk_chunk(K));
 }
 
-// Rows and k of the split-BF16 operand planes are padded to these multiples.
-constexpr int kSplitRowPad = 16;
-constexpr int kSplitKPad = 32;
-// Longest padded k of the 4M split kernels: their per-lane load offsets
 // 4M split products with few 128x128 tiles: slices of k (at least 256 each)
 // that fill the 256 CUs, each slice a result of its own, summed afterwards in
 // FP64 (launch_sum_chunks).  One slice where half the CUs have a tile
@@ -90,6 +90,10 @@ inline int64_t x4m_slices(int64_t M, int64_t N, int64_t K, int64_t batch, int va
     return ceil_div(kt, ceil_div(kt, want)); // no slice empty
 }
 
+// Rows and k of the split-BF16 operand planes are padded to these multiples.
+constexpr int kSplitRowPad = 16;
+constexpr int kSplitKPad = 32;
+// Longest padded k of the 4M split kernels: their per-lane load offsets
 // within a tile of up to 192 operand rows stay below 2^32 bytes.
 constexpr int64_t kX4mMaxK = int64_t(1) << 21;
 
@@ -126,6 +130,19 @@ struct FusedSmall {
     int lb = 0, lm = 0, ln = 0, lk = 0; // log2 of batch, M, N, K
     int red = 0; // 1: one work-group per output, k split over its threads
     FusedBits a_b, a_m, a_k, b_b, b_n, b_k, c_b, c_m, c_n;
+};
+
+// One work-group's share of a group of independent small contractions that
+// run in one launch (grouped_small_kernel): 256 >> lanes outputs of one
+// contraction, from output `first` on, 2^lanes lanes per output.  a, b and c
+// are slots of the pointer table that the launch is given.
+constexpr int kGroupMaxLog2K = 10;       // k offset tables in LDS
+constexpr int kGroupMaxLog2Outputs = 14; // result kept apart from the arena's reuse
+constexpr int kGroupMaxLog2Work = 20;    // outputs * K
+struct GroupBlock {
+    FusedSmall f;
+    int32_t a = 0, b = 0, c = 0;
+    int32_t first = 0, lanes = 0;
 };
 
 // Split-BF16 operand: planes re hi/lo, im hi/lo[, re+im hi/lo].
@@ -168,6 +185,10 @@ int choose_gemm_kernel(int mode, int64_t M, int64_t N, int64_t K,
 // kGemmSplitK.
 void launch_gemm(int kernel, int elem_bytes, const GemmArgs &g,
                  hipStream_t stream, void *partials = nullptr);
+// The FP32 products on the BF16 matrix cores (gemm_f32x6.hip), where they
+// apply to the operands.
+bool f32x6_applies(const GemmArgs &g);
+void launch_f32x6(const GemmArgs &g, hipStream_t stream);
 // src: complex64 [batch][rows][k] with row stride ld and batch stride s.
 void launch_split_bf16(const void *src, int64_t rows, int64_t k, int64_t ld,
                        int64_t s, int64_t batch, const SplitOperand &dst,

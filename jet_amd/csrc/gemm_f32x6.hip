@@ -1,0 +1,461 @@
+// gemm_f32x6.hip -- complex64 GEMM at FP32 accuracy on the BF16 matrix cores
+// (gfx950): the FP32 products of every precision mode.
+//
+// Each FP32 value is the sum of three BF16 pieces, x = h + m + l (rounded to
+// nearest: 3 x 8 significant bits, so the sum is exact), and a real product
+// keeps the six terms hh, hm, mh, hl, lh, mm; the dropped ones are below
+// 2^-24 of it (values under 2^-110 lose their low piece to BF16's smallest
+// normal, an absolute 2^-126).  Four real products make 24 v_mfma_f32_32x32x16_bf16 per 32x32
+// block and 16 k: at BF16's rate (16 times FP32's on the same matrix cores)
+// that is 2.7 times the FP32 MFMA rate.  Measured (TFLOP/s of 8 M N K, FP32
+// MFMA kernel before -> this one): 4096^3 121 -> 227, 4096x4096x1024 119 ->
+// 219, 256x65536x256 113 -> 192, 1024^3 52 -> 158; 512^3 (which the VALU
+// kernel ran) 368 -> 12 us.  Errors against 64 bits (normwise, random
+// operands): 4096^3 1.6e-6 -> 1.4e-6, 1024^3 8.1e-7 -> 1.9e-7, 512^3 5.7e-7
+// -> 9.8e-8, K = 64 7.4e-8 -> 5.6e-8: the accumulator takes fewer roundings
+// per k than the K = 4 steps of the FP32 instruction, and (all tiles but the
+// widest) the terms with a middle or low piece, 2^-8 of the product and
+// less, sum in accumulators of their own, so that the main ones are rounded
+// twice per 16 k.
+//
+// The operands stay FP32 in memory and in LDS (8 bytes per complex value:
+// three pieces of each part would be 12) and are split in registers after
+// the LDS read, about 5.5 VALU instructions per value, issued beside the
+// other wave's MFMAs; there is no operand pass and no workspace.
+#include "common.hpp"
+#include "gemm.hpp"
+#include "gemm_device.hpp"
+#include "profiler.hpp"
+
+#include <algorithm>
+
+namespace jet_hip {
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// Three BF16 pieces of eight consecutive k of one operand row.
+struct Pieces {
+    u32x4 h, m, l;
+};
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+__device__ __forceinline__ float low_bf16(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float high_bf16(uint32_t p)
+{
+    return __uint_as_float(p & 0xffff0000u);
+}
+
+// x = h + m + l, each rounded to nearest: 24 significant bits, so the sum is
+// exact unless l falls below BF16's smallest normal.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l)
+{
+    h = pack_bf16(a, b);
+    const float ra = a - low_bf16(h), rb = b - high_bf16(h);
+    m = pack_bf16(ra, rb);
+    l = pack_bf16(ra - low_bf16(m), rb - high_bf16(m));
+}
+
+__device__ __forceinline__ f32x16 mma(const u32x4 &a, const u32x4 &b, f32x16 c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// BM x BN output tile, WM x WN waves of 32x32 blocks; with WK > 1 the waves
+// also split every stage's k (WK slices of 16, summed through LDS at the
+// end): small products have few tiles, and a tile's time is its k steps'
+// latency.  Stages of 16 WK k come straight from global memory into NS LDS
+// buffers with global_load_lds_dwordx4, two stages ahead with three buffers.
+// Rows past M or N repeat the last row (their outputs are not stored); k past
+// K is zeroed after the LDS read.  DW: dwords per lane of a load, 4, or 1 for
+// rows that are not 16-byte aligned (odd k or strides).
+template <int BM, int BN, int WM, int WN, int WK, int NS, bool DUAL, int DW>
+__global__ __launch_bounds__(64 * WM * WN * WK,
+                             WM * WN * WK / 4) void cgemm_f32x6_kernel(GemmArgs g)
+{
+    typedef __attribute__((address_space(3))) void lds_void;
+    constexpr int NW = WM * WN * WK;
+    constexpr int KT = 16 * WK; // complex k per stage
+    constexpr int WTM = BM / WM, WTN = BN / WN;
+    constexpr int FM = WTM / 32, FN = WTN / 32;
+    constexpr int PER = 4 / DW; // loads per 16-byte chunk
+    constexpr int A_IN = BM * 8 * WK * PER / (64 * NW);
+    constexpr int B_IN = BN * 8 * WK * PER / (64 * NW);
+    constexpr int L = A_IN + B_IN;
+    constexpr int STAGE = (BM + BN) * 8 * WK; // 16-byte chunks
+    static_assert(A_IN * 64 * NW == BM * 8 * WK * PER && B_IN * 64 * NW == BN * 8 * WK * PER,
+                  "tile");
+    static_assert(L < 64, "one stage of loads fits the wait counter");
+    static_assert(NS == 2 || NS == 3, "two or three LDS stages");
+    static_assert((WK - 1) * BM * BN * 8 <= STAGE * 16 * (NS == 2 ? 2 : 1), "wave sums fit");
+    __shared__ f32x4 S0[NS == 2 ? 2 * STAGE : STAGE];
+    __shared__ f32x4 S1x[NS == 2 ? 1 : STAGE], S2x[NS == 2 ? 1 : STAGE];
+    f32x4 *const S1 = NS == 2 ? S0 + STAGE : S1x, *const S2 = NS == 2 ? S0 : S2x;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wmn = wave / WK;
+    const int wm = wmn / WN, wn = wmn % WN;
+    const int64_t bz = blockIdx.z;
+    int64_t tm, tn;
+    tile_coords(blockIdx.x, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, tm, tn);
+    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const int K = int(g.K);
+    const char *At = static_cast<const char *>(g.A) + (bz * g.sA + m0 * g.lda) * 8;
+    const char *Bt = static_cast<const char *>(g.B) + (bz * g.sB + n0 * g.ldb) * 8;
+
+    // One load instruction fills 64 consecutive chunks (or dwords) of a
+    // stage; a stage is [k sixteenth][row of A, then of B][8 chunks], the
+    // chunk of a row in slot chunk ^ (row & 7).
+    uint32_t off[L]; // byte offset of the lane's row, and dword of its value
+    int ck[L];       // the lane's first k
+#pragma unroll
+    for (int i = 0; i < L; i++) {
+        const bool isa = i < A_IN;
+        const int pd = (wave * (isa ? A_IN : B_IN) + (isa ? i : i - A_IN)) * 64 + lane;
+        const int p = pd / PER, sub = (pd % PER) * DW;
+        const int r = (p >> 3) % (isa ? BM : BN), slot = p & 7, kk = (p >> 3) / (isa ? BM : BN);
+        const int64_t rows = isa ? g.M - m0 : g.N - n0;
+        const int64_t rr = r < rows ? r : rows - 1;
+        ck[i] = 16 * kk + 2 * (slot ^ (r & 7)) + sub / 2;
+        off[i] = uint32_t(rr * (isa ? g.lda : g.ldb) * 8) + (sub & 1) * 4;
+    }
+    auto issue = [&](int kt, f32x4 *s) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int k0 = kt * KT;
+#pragma unroll
+        for (int i = 0; i < L; i++) {
+            const int k = k0 + ck[i];
+            const uint32_t o = off[i] + (k < K ? uint32_t(k) * 8u : 0u);
+            const void *src = (i < A_IN ? At : Bt) + uint64_t(o);
+            float *dst = i < A_IN ? reinterpret_cast<float *>(s) + (wave * A_IN + i) * 64 * DW
+                                  : reinterpret_cast<float *>(s + BM * 8 * WK) +
+                                        (wave * B_IN + i - A_IN) * 64 * DW;
+            if constexpr (DW == 4)
+                __builtin_amdgcn_global_load_lds(src, (lds_void *)dst, 16, 0, 0);
+            else
+                __builtin_amdgcn_global_load_lds(src, (lds_void *)dst, 4, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // DUAL: the products with a middle or low piece in sums of their own.
+    constexpr int DM = DUAL ? FM : 1, DN = DUAL ? FN : 1;
+    f32x16 cr[FM][FN], ci[FM][FN], dr[DM][DN], di[DM][DN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            cr[i][j] = f32x16{};
+            ci[i][j] = f32x16{};
+            if (DUAL) {
+                dr[i % DM][j % DN] = f32x16{};
+                di[i % DM][j % DN] = f32x16{};
+            }
+        }
+
+    const int q = lane >> 5, j = lane & 31;
+    // Eight complex values of one row from LDS, as the pieces of their real
+    // and imaginary parts; kv: valid k of this lane's eight.
+    auto fetch = [&](const f32x4 *row, int sw, bool tail, int kv, Pieces &re,
+                     Pieces &im) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            f32x4 v = row[(q * 4 + c) ^ sw];
+            if (tail && 2 * c >= kv) v.x = v.y = 0.f;
+            if (tail && 2 * c + 1 >= kv) v.z = v.w = 0.f;
+            uint32_t h, m, l;
+            split_pair(v.x, v.z, h, m, l);
+            re.h[c] = h, re.m[c] = m, re.l[c] = l;
+            split_pair(v.y, v.w, h, m, l);
+            im.h[c] = h, im.m[c] = m, im.l[c] = l;
+        }
+    };
+    auto compute = [&](const f32x4 *s, bool tail, int kt) __attribute__((always_inline)) {
+        const int kv = K - kt * KT - 16 * wk - 8 * q;
+        Pieces br[FN], bi[FN];
+#pragma unroll
+        for (int fn = 0; fn < FN; fn++) {
+            const int r = wn * WTN + fn * 32 + j;
+            fetch(s + (BM * WK + BN * wk + r) * 8, r & 7, tail, kv, br[fn], bi[fn]);
+        }
+#pragma unroll
+        for (int fm = 0; fm < FM; fm++) {
+            const int r = wm * WTM + fm * 32 + j;
+            Pieces ar, ai, ni;
+            fetch(s + (BM * wk + r) * 8, r & 7, tail, kv, ar, ai);
+            ni.h = ai.h ^ 0x80008000u;
+            ni.m = ai.m ^ 0x80008000u;
+            ni.l = ai.l ^ 0x80008000u;
+#pragma unroll
+            for (int fn = 0; fn < FN; fn++) {
+                f32x16 x = DUAL ? dr[fm % DM][fn % DN] : cr[fm][fn];
+                f32x16 y = DUAL ? di[fm % DM][fn % DN] : ci[fm][fn];
+                x = mma(ar.l, br[fn].h, x);
+                y = mma(ar.l, bi[fn].h, y);
+                x = mma(ni.l, bi[fn].h, x);
+                y = mma(ai.l, br[fn].h, y);
+                x = mma(ar.h, br[fn].l, x);
+                y = mma(ar.h, bi[fn].l, y);
+                x = mma(ni.h, bi[fn].l, x);
+                y = mma(ai.h, br[fn].l, y);
+                x = mma(ar.m, br[fn].m, x);
+                y = mma(ar.m, bi[fn].m, y);
+                x = mma(ni.m, bi[fn].m, x);
+                y = mma(ai.m, br[fn].m, y);
+                x = mma(ar.m, br[fn].h, x);
+                y = mma(ar.m, bi[fn].h, y);
+                x = mma(ni.m, bi[fn].h, x);
+                y = mma(ai.m, br[fn].h, y);
+                x = mma(ar.h, br[fn].m, x);
+                y = mma(ar.h, bi[fn].m, y);
+                x = mma(ni.h, bi[fn].m, x);
+                y = mma(ai.h, br[fn].m, y);
+                if (DUAL) {
+                    dr[fm % DM][fn % DN] = x;
+                    di[fm % DM][fn % DN] = y;
+                    x = cr[fm][fn];
+                    y = ci[fm][fn];
+                }
+                x = mma(ar.h, br[fn].h, x);
+                y = mma(ar.h, bi[fn].h, y);
+                x = mma(ni.h, bi[fn].h, x);
+                y = mma(ai.h, br[fn].h, y);
+                cr[fm][fn] = x;
+                ci[fm][fn] = y;
+            }
+        }
+    };
+
+    const int nk = (K + KT - 1) / KT;
+    // vmcnt(L): the loads of the next stage may stay in flight.
+    constexpr int kWaitPrev = 0x0f70 | (L & 15) | ((L >> 4) << 14);
+    constexpr int kWaitAll = 0x0f70;
+    issue(0, S0);
+    if (NS == 3 && nk > 1) issue(1, S1);
+    // Stage kt is in LDS for every wave once each has waited for its own
+    // loads; every wave is then also past its reads of stage kt - 1, whose
+    // buffer takes stage kt + NS - 1.
+    auto arrive = [&](int kt, f32x4 *next) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (NS == 3 && kt + 1 < nk)
+            __builtin_amdgcn_s_waitcnt(kWaitPrev);
+        else
+            __builtin_amdgcn_s_waitcnt(kWaitAll);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + NS - 1 < nk) issue(kt + NS - 1, next);
+    };
+    const int nfull = K / KT;
+    int kt = 0;
+    if (NS == 3) {
+        for (; kt + 3 <= nfull; kt += 3) {
+            arrive(kt, S2);
+            compute(S0, false, kt);
+            arrive(kt + 1, S0);
+            compute(S1, false, kt + 1);
+            arrive(kt + 2, S1);
+            compute(S2, false, kt + 2);
+        }
+        // At most three stages are left; only the third is still to be issued.
+        for (int b = 0; kt < nk; kt++, b++) {
+            arrive(kt, S2);
+            compute(b == 0 ? S0 : b == 1 ? S1 : S2, true, kt);
+        }
+    }
+    else {
+        for (; kt + 2 <= nfull; kt += 2) {
+            arrive(kt, S1);
+            compute(S0, false, kt);
+            arrive(kt + 1, S0);
+            compute(S1, false, kt + 1);
+        }
+        for (int b = 0; kt < nk; kt++, b++) {
+            arrive(kt, b == 0 ? S1 : S0);
+            compute(b == 0 ? S0 : S1, true, kt);
+        }
+    }
+
+    if (DUAL) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j2 = 0; j2 < FN; j2++) {
+                cr[i][j2] += dr[i % DM][j2 % DN];
+                ci[i][j2] += di[i % DM][j2 % DN];
+            }
+    }
+    if (WK > 1) {
+        // The sums of the K slices, added in slice order by the first.
+        __syncthreads();
+        float2 *sums = reinterpret_cast<float2 *>(S0);
+        constexpr int SUM = FM * FN * 16 * 64;
+        if (wk > 0) {
+#pragma unroll
+            for (int fm = 0; fm < FM; fm++)
+#pragma unroll
+                for (int fn = 0; fn < FN; fn++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        sums[((wk - 1) * WM * WN + wmn) * SUM + ((fm * FN + fn) * 16 + i) * 64 +
+                             lane] = float2{cr[fm][fn][i], ci[fm][fn][i]};
+        }
+        __syncthreads();
+        if (wk > 0) return;
+        for (int w = 0; w < WK - 1; w++)
+#pragma unroll
+            for (int fm = 0; fm < FM; fm++)
+#pragma unroll
+                for (int fn = 0; fn < FN; fn++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const float2 v = sums[(w * WM * WN + wmn) * SUM +
+                                              ((fm * FN + fn) * 16 + i) * 64 + lane];
+                        cr[fm][fn][i] += v.x;
+                        ci[fm][fn][i] += v.y;
+                    }
+    }
+
+    float2 *C = static_cast<float2 *>(g.C) + bz * g.sC;
+    bool bad = false;
+#pragma unroll
+    for (int fm = 0; fm < FM; fm++)
+#pragma unroll
+        for (int fn = 0; fn < FN; fn++) {
+            const int64_t col = n0 + wn * WTN + fn * 32 + j;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int64_t row = m0 + wm * WTM + fm * 32 + 8 * (i / 4) + 4 * q + (i & 3);
+                const float2 v{cr[fm][fn][i], ci[fm][fn][i]};
+                bad |= !(__builtin_isfinite(v.x) && __builtin_isfinite(v.y));
+                if (row < g.M && col < g.N) C[row * g.ldc + col] = v;
+            }
+        }
+    if (!bad) return;
+    // An infinite or NaN input (or a result out of range): the pieces of an
+    // infinity do not multiply as the infinity does, so those outputs are
+    // computed again from the operands.
+    for (int e = 0; e < FM * FN * 16; e++) {
+        const int i = e & 15, fn = (e >> 4) % FN, fm = (e >> 4) / FN;
+        const int64_t col = n0 + wn * WTN + fn * 32 + j;
+        const int64_t row = m0 + wm * WTM + fm * 32 + 8 * (i / 4) + 4 * q + (i & 3);
+        if (row >= g.M || col >= g.N) continue;
+        const float2 v = C[row * g.ldc + col];
+        if (__builtin_isfinite(v.x) && __builtin_isfinite(v.y)) continue;
+        const float2 *a = static_cast<const float2 *>(g.A) + bz * g.sA + row * g.lda;
+        const float2 *b = static_cast<const float2 *>(g.B) + bz * g.sB + col * g.ldb;
+        float sr = 0.f, si = 0.f;
+        for (int k = 0; k < K; k++) {
+            const float2 x = a[k], y = b[k];
+            sr = fmaf(x.x, y.x, sr);
+            sr = fmaf(-x.y, y.y, sr);
+            si = fmaf(x.x, y.y, si);
+            si = fmaf(x.y, y.x, si);
+        }
+        C[row * g.ldc + col] = float2{sr, si};
+    }
+}
+
+// The tile form of a product.  A CU that gets `per_cu` tiles (the fullest)
+// runs them `occ` at a time; a stage of `kt` k takes `alone` us while they
+// wait on latency and `full` us of matrix-core time per tile, and a tile costs
+// `out` us beside its stages (prologue and stores).  Measured on shapes with one tile
+// per CU and with many (predicted / measured us: 1024^3 62, 53, 56 / 65, 54,
+// 55 for the 64x64, 64x32 and 32x32 tiles; 2048^3 337, 353 / 336, 369 for
+// 128x128 and 64x64; 256x65536x256 175, 192 / 178, 193 for 256x128 and
+// 128x128); the choices it makes are within 6% of the best of eleven forms
+// timed on 19 shapes from 64^3 to 4096x4096x1024.
+struct TileForm {
+    int bm, bn, kt, occ;
+    float alone, full, out;
+};
+constexpr TileForm kForms[] = {{256, 128, 16, 1, 3.9f, 4.85f, 10.f},
+                               {128, 128, 16, 1, 2.4f, 2.63f, 6.f},
+                               {64, 64, 16, 3, 0.92f, 0.69f, 1.f},
+                               {64, 32, 32, 2, 1.05f, 0.77f, 0.6f},
+                               {32, 32, 64, 2, 1.1f, 0.8f, 0.4f}};
+constexpr int kCus = 256;
+
+int choose_form(const GemmArgs &g)
+{
+    int best = 0;
+    double best_us = -1.0;
+    for (int i = 0; i < int(sizeof(kForms) / sizeof(kForms[0])); i++) {
+        const TileForm &f = kForms[i];
+        const double per_cu = double(
+            ceil_div(ceil_div(g.M, f.bm) * ceil_div(g.N, f.bn) * g.batch, int64_t(kCus)));
+        const double rounds = double(ceil_div(int64_t(per_cu), f.occ));
+        const double us = double(ceil_div(g.K, f.kt)) *
+                              std::max(f.alone * rounds, f.full * per_cu) + f.out * per_cu;
+        if (best_us < 0.0 || us < best_us) {
+            best_us = us;
+            best = i;
+        }
+    }
+    return best;
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int NS, bool DUAL, int DW = 4>
+void launch_tile(const GemmArgs &g, hipStream_t stream)
+{
+    JH_REQUIRE(ceil_div(g.M, BM) * ceil_div(g.N, BN) <= 0x7fffffff, "Too many tiles.");
+    dim3 grid((unsigned)(ceil_div(g.M, BM) * ceil_div(g.N, BN)), 1, (unsigned)g.batch);
+    hipLaunchKernelGGL((cgemm_f32x6_kernel<BM, BN, WM, WN, WK, NS, DUAL, DW>), grid,
+                       dim3(64 * WM * WN * WK), 0, stream, g);
+    JH_HIP(hipGetLastError());
+}
+
+} // namespace
+
+// The lane offsets are 32 bits (row strides to 2^21); 32x32 blocks of which
+// less than half would be outputs, and one or no k step, are left to the FP32 MFMA kernel.
+bool f32x6_applies(const GemmArgs &g)
+{
+    return g.lda <= (int64_t(1) << 21) && g.ldb <= (int64_t(1) << 21) && g.K >= 16 &&
+           g.M >= 16 && g.N >= 16;
+}
+
+void launch_f32x6(const GemmArgs &g, hipStream_t stream)
+{
+    const bool aligned = reinterpret_cast<uintptr_t>(g.A) % 16 == 0 &&
+                         reinterpret_cast<uintptr_t>(g.B) % 16 == 0 && g.K % 2 == 0 &&
+                         g.lda % 2 == 0 && g.ldb % 2 == 0 &&
+                         (g.batch == 1 || (g.sA % 2 == 0 && g.sB % 2 == 0));
+    const int form = choose_form(g);
+    if (!aligned) { // four times the load instructions: the smaller tiles hide them
+        if (form <= 2)
+            launch_tile<64, 64, 2, 2, 1, 3, true, 1>(g, stream);
+        else
+            launch_tile<32, 32, 1, 1, 4, 2, true, 1>(g, stream);
+        return;
+    }
+    switch (form) {
+    case 0:
+        launch_tile<256, 128, 4, 2, 1, 3, false>(g, stream);
+        break;
+    case 1:
+        launch_tile<128, 128, 2, 2, 1, 3, true>(g, stream);
+        break;
+    case 2:
+        launch_tile<64, 64, 2, 2, 1, 3, true>(g, stream);
+        break;
+    case 3:
+        launch_tile<64, 32, 2, 1, 2, 3, true>(g, stream);
+        break;
+    default:
+        launch_tile<32, 32, 1, 1, 4, 2, true>(g, stream);
+        break;
+    }
+}
+
+} // namespace jet_hip

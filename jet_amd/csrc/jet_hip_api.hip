@@ -35,6 +35,9 @@ struct jet_hip_network_s {
     NetworkPlan plan;
     char *arena = nullptr;
     char *workspace = nullptr;
+    // records of the groups of small steps, and their pointer table
+    GroupBlock *blocks = nullptr;
+    const void **pointers = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
 };
@@ -232,11 +235,24 @@ void run_network(jet_hip_network_s *net, const void *const *leaves, void *out, h
         JH_REQUIRE(leaves[i] != nullptr, "Null leaf tensor.");
         node[i] = leaves[i];
     }
-    for (size_t k = 0; k < np.steps.size(); k++) {
-        const NetworkStep &st = np.steps[k];
-        void *c = st.is_root ? out : static_cast<void *>(net->arena + st.offset);
-        run_contraction(st.desc, node[st.a], node[st.b], c, net->workspace, s);
-        node[np.n_leaves + k] = c;
+    if (!np.blocks.empty()) {
+        std::vector<const void *> given(node.begin(), node.begin() + np.n_leaves);
+        given.push_back(out);
+        launch_set_pointers(net->pointers, given.data(), (int)given.size(), s);
+    }
+    for (size_t k = 0; k < np.steps.size(); k++)
+        node[np.n_leaves + k] = np.steps[k].is_root
+                                    ? out
+                                    : static_cast<void *>(net->arena + np.steps[k].offset);
+    for (const NetworkLaunch &l : np.launches) {
+        if (l.step < 0) {
+            launch_grouped_small(net->blocks + l.first_block, l.n_blocks, net->pointers,
+                                 np.elem_bytes, l.flops, s);
+            continue;
+        }
+        const NetworkStep &st = np.steps[l.step];
+        run_contraction(st.desc, node[st.a], node[st.b],
+                        const_cast<void *>(node[np.n_leaves + l.step]), net->workspace, s);
     }
 }
 
@@ -256,6 +272,38 @@ void *device_alloc(size_t bytes, int device)
     }
     JH_HIP(e);
     return p;
+}
+
+void free_memory(jet_hip_network_s *net)
+{
+    if (net->arena) (void)hipFree(net->arena);
+    if (net->workspace) (void)hipFree(net->workspace);
+    if (net->blocks) (void)hipFree(net->blocks);
+    if (net->pointers) (void)hipFree(net->pointers);
+}
+
+// The arena, the workspace and the records and pointer table of the groups
+// of small steps (the slots of the step results are set here, those of the
+// leaves and the output by every execution).
+void alloc_memory(jet_hip_network_s *net)
+{
+    const NetworkPlan &np = net->plan;
+    const int device = net->ctx->device;
+    if (np.arena_bytes) net->arena = static_cast<char *>(device_alloc(np.arena_bytes, device));
+    if (np.workspace_bytes)
+        net->workspace = static_cast<char *>(device_alloc(np.workspace_bytes, device));
+    if (np.blocks.empty()) return;
+    std::vector<const void *> slots(np.slot(np.n_leaves + (int)np.steps.size()), nullptr);
+    for (size_t k = 0; k < np.steps.size(); k++)
+        if (!np.steps[k].is_root)
+            slots[np.slot(np.n_leaves + (int)k)] = net->arena + np.steps[k].offset;
+    const size_t nb = np.blocks.size() * sizeof(GroupBlock), ns = slots.size() * sizeof(void *);
+    net->blocks = static_cast<GroupBlock *>(device_alloc(nb, device));
+    net->pointers = static_cast<const void **>(device_alloc(ns, device));
+    hipStream_t s = net->ctx->stream;
+    JH_HIP(hipMemcpyAsync(net->blocks, np.blocks.data(), nb, hipMemcpyHostToDevice, s));
+    JH_HIP(hipMemcpyAsync(net->pointers, slots.data(), ns, hipMemcpyHostToDevice, s));
+    JH_HIP(hipStreamSynchronize(s));
 }
 
 void free_graph(jet_hip_network_s *net)
@@ -968,15 +1016,10 @@ int jet_hip_network_create(jet_hip_ctx_t ctx, jet_hip_dtype_t dtype, jet_hip_pre
             n->plan = plan_network(elem_bytes_of(dtype), mode_of(dtype, precision), n_leaves,
                                    leaf_ranks, leaf_modes, leaf_extents, n_steps, path, n_out,
                                    out_modes);
-            if (n->plan.arena_bytes)
-                n->arena = static_cast<char *>(device_alloc(n->plan.arena_bytes, ctx->device));
-            if (n->plan.workspace_bytes)
-                n->workspace =
-                    static_cast<char *>(device_alloc(n->plan.workspace_bytes, ctx->device));
+            alloc_memory(n);
         }
         catch (...) {
-            if (n->arena) (void)hipFree(n->arena);
-            if (n->workspace) (void)hipFree(n->workspace);
+            free_memory(n);
             delete n;
             throw;
         }
@@ -1014,15 +1057,10 @@ int jet_hip_dag_create(jet_hip_ctx_t ctx, jet_hip_dtype_t dtype, jet_hip_precisi
             n->plan = plan_dag(elem_bytes_of(dtype), mode_of(dtype, precision), n_leaves,
                                leaf_ranks, leaf_modes, leaf_extents, n_steps, steps, n_keep,
                                keep);
-            if (n->plan.arena_bytes)
-                n->arena = static_cast<char *>(device_alloc(n->plan.arena_bytes, ctx->device));
-            if (n->plan.workspace_bytes)
-                n->workspace =
-                    static_cast<char *>(device_alloc(n->plan.workspace_bytes, ctx->device));
+            alloc_memory(n);
         }
         catch (...) {
-            if (n->arena) (void)hipFree(n->arena);
-            if (n->workspace) (void)hipFree(n->workspace);
+            free_memory(n);
             delete n;
             throw;
         }
@@ -1223,8 +1261,7 @@ int jet_hip_network_destroy(jet_hip_network_t net)
         set_device(net->ctx);
         JH_HIP(hipDeviceSynchronize());
         free_graph(net);
-        if (net->arena) JH_HIP(hipFree(net->arena));
-        if (net->workspace) JH_HIP(hipFree(net->workspace));
+        free_memory(net);
         delete net;
     });
 }

@@ -15,7 +15,12 @@
 //   * intermediates live in one arena; each is released after its consumer
 //     step and the offsets come from a best-fit simulation of that sequence;
 //   * one workspace, sized for the largest step, serves every step (the
-//     steps run in order on one stream).
+//     steps run in order on one stream);
+//   * small steps (at most 2^14 outputs and 2^20 multiply-adds, extents powers
+//     of two) run in groups of one launch each: all whose operands are ready
+//     at the same dependency level.  Their results have memory of their own,
+//     so their order does not matter to the arena; the other steps keep
+//     their order.
 //
 // Pure C++ so that plans can be checked on the CPU.
 #pragma once
@@ -34,6 +39,16 @@ struct NetworkStep {
     ContractionDesc desc;
     size_t offset = 0;                // arena offset of the result
     bool is_root = false;
+    bool grouped = false;             // runs in a group of small steps
+    FusedSmall small;                 // its offsets then
+};
+
+// One launch of an execution: step `step` alone, or (step < 0) the group of
+// small steps made of `n_blocks` records from `first_block` on.
+struct NetworkLaunch {
+    int step = -1;
+    int first_block = 0, n_blocks = 0;
+    double flops = 0;
 };
 
 struct NetworkPlan {
@@ -48,6 +63,11 @@ struct NetworkPlan {
     size_t workspace_bytes = 0;
     double flops = 0;                 // sum of 8*M*N*K*batch over steps
     PermutePlan root_copy;            // used when there are no steps
+    std::vector<NetworkLaunch> launches;
+    // Records of the groups.  Slots of their pointer table: the leaves, the
+    // caller's output (n_leaves), then the step results.
+    std::vector<GroupBlock> blocks;
+    int slot(int node) const { return node < n_leaves ? node : node + 1; }
     // Contraction DAGs (plan_dag): no root and no output; `kept` marks the
     // step results that stay in the arena (a contiguous region at its end,
     // in the order they were listed) after an execution.
