@@ -26,6 +26,7 @@ SOURCES = [
     "gemm.hip",
     "gemm_f32x6.hip",
     "misc.hip",
+    "stream.hip",
     "profiler.hip",
     "network.hip",
     "jet_hip_api.hip",

@@ -183,6 +183,70 @@ bool plan_fused_small(const std::vector<int32_t> &a, const std::vector<int64_t> 
     return f.lk <= kFusedMaxLog2K;
 }
 
+bool plan_stream_shortk(const std::vector<int32_t> &a, const std::vector<int64_t> &ea,
+                        const std::vector<int32_t> &b, const std::vector<int64_t> &eb,
+                        const std::vector<int32_t> &c, StreamShortK &p)
+{
+    // One entry per address bit of A, B and C: the (mode, bit) it holds,
+    // lowest bit first.
+    typedef std::vector<std::pair<int32_t, int>> Bits;
+    auto bits_of = [](const std::vector<int32_t> &m, const std::vector<int64_t> &e, Bits &out) {
+        for (size_t i = m.size(); i-- > 0;) {
+            if (e[i] < 1 || (e[i] & (e[i] - 1))) return false;
+            for (int t = 0; (int64_t(1) << t) < e[i]; t++) out.push_back({m[i], t});
+        }
+        return out.size() <= 31;
+    };
+    Bits ba, bb, bc;
+    if (!bits_of(a, ea, ba) || !bits_of(b, eb, bb)) return false;
+    std::vector<int64_t> ec;
+    for (int32_t m : c) ec.push_back(find(a, m) >= 0 ? ea[find(a, m)] : eb[find(b, m)]);
+    if (!bits_of(c, ec, bc)) return false;
+    p = StreamShortK{};
+    p.swap = bb.size() > ba.size() ? 1 : 0;
+    const Bits &x = p.swap ? bb : ba, &y = p.swap ? ba : bb;
+    auto at = [](const Bits &v, const std::pair<int32_t, int> &q) {
+        return int(std::find(v.begin(), v.end(), q) - v.begin());
+    };
+    auto in = [&](const Bits &v, const std::pair<int32_t, int> &q) {
+        return at(v, q) < (int)v.size();
+    };
+    for (int i = 0; i < (int)x.size(); i++) {
+        const int yi = at(y, x[i]), ci = at(bc, x[i]);
+        if (!in(bc, x[i])) {
+            if (p.lk == kStreamMaxLog2K) return false;
+            p.xk[p.lk] = int8_t(i);
+            p.yk[p.lk++] = int8_t(yi);
+        }
+        else if (in(y, x[i])) {
+            if (p.lb == kStreamMaxBatch || i < 4 || ci < 4) return false;
+            p.xb[p.lb] = int8_t(i);
+            p.yb[p.lb] = int8_t(yi);
+            p.cb[p.lb++] = int8_t(ci);
+        }
+        else {
+            // lowest C bits belong to rows of one work-group step
+            if (ci < 4 && p.lr >= 8) return false;
+            StreamSegment *s = p.n_segments ? &p.segment[p.n_segments - 1] : nullptr;
+            if (s && s->x + s->len == i && s->c + s->len == ci)
+                s->len++;
+            else {
+                if (p.n_segments == kStreamMaxSegments) return false;
+                p.segment[p.n_segments++] =
+                    StreamSegment{int8_t(p.lr), 1, int8_t(i), int8_t(ci)};
+            }
+            p.lr++;
+        }
+    }
+    for (int i = 0; i < (int)bc.size(); i++)
+        if (!in(x, bc[i])) {
+            if (p.ln == kStreamMaxLog2N) return false;
+            p.yn[p.ln] = int8_t(at(y, bc[i]));
+            p.cn[p.ln++] = int8_t(i);
+        }
+    return p.lr >= 1;
+}
+
 int gemm_variants(int kernel)
 {
     switch (kernel) {
@@ -428,6 +492,19 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
             d.fuse_b = plan_split_gather(B, EB, cat(gemm_batch, right, gemm_common), d.K, d.gb);
     }
 
+    // A small tensor on a few modes of a large one: one pass over the large
+    // one in place.  Up to 16 k and 16 columns the VALU keeps up with memory;
+    // below 2^14 elements the fused small step is a launch as short.
+    if (d.chunks == 1 && std::max(d.size_a, d.size_b) >= (int64_t(1) << 14) &&
+        plan_stream_shortk(A, EA, B, EB, C, d.sk)) {
+        d.stream_shortk = true;
+        d.gemm_kernel = kGemmSmall;
+        d.gemm_variant = 0;
+        d.fuse_a = d.fuse_b = false;
+        layout_workspace(d);
+        return d;
+    }
+
     // Small steps on the one-thread-per-output or the one-block-per-output
     // VALU kernel that would need a permuted operand or result: one fused
     // pass of the same form, no copies.
@@ -448,7 +525,7 @@ void layout_workspace(ContractionDesc &d)
 {
     size_t off = 0;
     const size_t eb = (size_t)d.elem_bytes;
-    if (d.fused_small) { // reads and writes the tensors in place
+    if (d.fused_small || d.stream_shortk) { // reads and writes the tensors in place
         d.workspace = 0;
         return;
     }
@@ -494,10 +571,6 @@ void layout_workspace(ContractionDesc &d)
         d.off_chunks = off;
         off = align256(off + eb * (size_t)d.batch * (size_t)d.M * (size_t)d.N);
     }
-    d.workspace = off;
-}
-
-} // namespace jet_hip
     d.slices = 1;
     if ((d.gemm_kernel == kGemmBf16x4m || d.gemm_kernel == kGemmF16x4m) && d.chunks == 1) {
         const int64_t n = x4m_slices(d.M, d.N, d.K, d.batch, d.gemm_variant);
@@ -511,3 +584,7 @@ void layout_workspace(ContractionDesc &d)
             off += bytes;
         }
     }
+    d.workspace = off;
+}
+
+} // namespace jet_hip

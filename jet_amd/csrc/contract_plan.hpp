@@ -18,6 +18,7 @@
 
 #include "gemm.hpp"
 #include "permute_plan.hpp"
+#include "stream.hpp"
 
 #include <cstddef>
 #include <cstdint>
@@ -39,6 +40,9 @@ struct ContractionDesc {
     // or result need permuting: one fused pass instead (FusedSmall)
     bool fused_small = false;
     FusedSmall fs;
+    // a few k and columns of a large operand: read in place (StreamShortK)
+    bool stream_shortk = false;
+    StreamShortK sk;
     int gemm_kernel = kGemmSmall;
     int gemm_variant = 0; // tile variant of gemm_kernel (GemmChoice)
     // K split into `chunks` pieces that run as a batch of the MFMA GEMM
@@ -49,12 +53,12 @@ struct ContractionDesc {
     // Workspace layout (bytes, 256-aligned offsets).
     size_t off_at = 0, off_bt = 0, off_ct = 0, off_sa = 0, off_sb = 0, off_partials = 0;
     size_t off_chunks = 0; // the GEMM's per-chunk results (chunks > 1)
+    int64_t slices = 1;    // slices of k of a 4M split GEMM (x4m_slices)
+    size_t off_slices = 0; // their results (slices > 1)
     // split-FP16 row maxima and scales of A and B (batch * padded rows each)
     size_t off_rmax_a = 0, off_scale_a = 0, off_rmax_b = 0, off_scale_b = 0;
     int64_t split_a_plane = 0, split_b_plane = 0;
     size_t workspace = 0;
-    int64_t slices = 1;    // slices of k of a 4M split GEMM (x4m_slices)
-    size_t off_slices = 0; // their results (slices > 1)
     double flops = 0; // 8 * batch * M * N * K
 };
 

@@ -148,6 +148,10 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
         launch_fused_small(d.fs, eb, a, b, c, s);
         return;
     }
+    if (d.stream_shortk) {
+        launch_stream_shortk(d.sk, eb, a, b, c, s);
+        return;
+    }
     const void *At = a;
     const void *Bt = b;
     if (d.need_a && !d.fuse_a) {
