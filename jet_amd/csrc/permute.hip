@@ -10,6 +10,41 @@ namespace jet_hip {
 
 namespace {
 
+// The plan's bit positions without a loop, as scalar registers: a loop over
+// them (bits_tile_base) waits for a load of kernel arguments per bit, about 1 us of
+// every tile and 5 us of a launch.  Positions past the last bit are zero
+// and meet zero bits of v.
+template <int N> __device__ __forceinline__ int64_t place_bits(const int8_t *pos, int64_t v)
+{
+    int64_t o = 0;
+#pragma unroll
+    for (int j = 0; j < N; j++) o |= ((v >> j) & 1) << pos[j];
+    return o;
+}
+
+__device__ __forceinline__ void tile_base(const BitPermParams &p, int64_t w, int64_t *bin,
+                                          int64_t *bout)
+{
+    constexpr int FAST = 24;
+    int64_t i = place_bits<FAST>(p.outer_in, w), o = place_bits<FAST>(p.outer_out, w);
+    for (int j = FAST; j < p.nr; j++) {
+        i |= ((w >> j) & 1) << p.outer_in[j];
+        o |= ((w >> j) & 1) << p.outer_out[j];
+    }
+    *bin = i;
+    *bout = o;
+}
+
+__device__ __forceinline__ int64_t tile_in_offset(const BitPermParams &p, int u)
+{
+    return place_bits<kTileMaxBits>(p.tile_in, u);
+}
+__device__ __forceinline__ int64_t tile_out_offset(const BitPermParams &p, int v, int *u)
+{
+    *u = int(place_bits<kTileMaxBits>(p.v2u, v));
+    return place_bits<kTileMaxBits>(p.tile_out, v);
+}
+
 template <class T>
 __global__ __launch_bounds__(kPermThreads) void permute_bits_kernel(
     const T *__restrict__ in, T *__restrict__ out, BitPermParams p,
@@ -28,15 +63,15 @@ __global__ __launch_bounds__(kPermThreads) void permute_bits_kernel(
     for (int e = 0; e < EMAX; e++) {
         const int u = tid + e * kPermThreads;
         int uu = 0;
-        ioff[e] = bits_tile_in_offset(p, u);
-        ooff[e] = bits_tile_out_offset(p, u, &uu);
+        ioff[e] = tile_in_offset(p, u);
+        ooff[e] = tile_out_offset(p, u, &uu);
         lsrc[e] = bits_lds_index(u, (int)sizeof(T));
         ldst[e] = bits_lds_index(uu, (int)sizeof(T));
     }
 
     for (int64_t w = blockIdx.x; w < ntiles; w += gridDim.x) {
         int64_t bin, bout;
-        bits_tile_base(p, w, &bin, &bout);
+        tile_base(p, w, &bin, &bout);
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < EMAX; e++)
@@ -66,9 +101,9 @@ __global__ __launch_bounds__(kPermThreads) void permute_bits_pairs_kernel(
     for (int e = 0; e < PMAX; e++) {
         const int u = 2 * (tid + e * kPermThreads);
         int uu0 = 0, uu1 = 0;
-        ioff[e] = bits_tile_in_offset(p, u);
-        ooff[e] = bits_tile_out_offset(p, u, &uu0);
-        (void)bits_tile_out_offset(p, u + 1, &uu1);
+        ioff[e] = tile_in_offset(p, u);
+        ooff[e] = tile_out_offset(p, u, &uu0);
+        (void)tile_out_offset(p, u + 1, &uu1);
         ls0[e] = bits_lds_index(u, 8);
         ls1[e] = bits_lds_index(u + 1, 8);
         ld0[e] = bits_lds_index(uu0, 8);
@@ -80,7 +115,7 @@ __global__ __launch_bounds__(kPermThreads) void permute_bits_pairs_kernel(
     typedef float f32x4v __attribute__((ext_vector_type(4)));
     for (int64_t w = blockIdx.x; w < ntiles; w += gridDim.x) {
         int64_t bin, bout;
-        bits_tile_base(p, w, &bin, &bout);
+        tile_base(p, w, &bin, &bout);
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < PMAX; e++) {
