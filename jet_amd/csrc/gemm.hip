@@ -326,61 +326,71 @@ __global__ __launch_bounds__(256) void fused_small_red_kernel(const void *Av, co
 // Independent small contractions of one dependency level in one launch: a
 // circuit's network has hundreds of steps of a few dozen values, and each as
 // a launch of its own costs 3-4 us of launch and memory latency, one after
-// the other.  The block's record is staged in LDS (one load per thread: read in
-// place, its byte-sized bit positions would be a chain of vector loads), the k offsets are
-// tabulated as in fused_small_kernel, 2^lanes lanes share an output's k and
-// add their sums with shuffles.  Measured: 1556 steps of the 6x6 depth-10
-// loss and gradient 8.9 ms as single launches -> see launch_grouped_small.
+// the other.  The kernel is a chain of latencies, so the record comes in one
+// scalar load, its bit positions packed in words (a loop over byte positions
+// waits for a load per bit), k offsets are made from them on the scalar unit
+// for the k bits that all lanes share, and there is no barrier.
+__device__ __forceinline__ uint32_t group_word(const uint32_t *w, int i)
+{
+    return (w[i / 6] >> (5 * (i % 6))) & 31u;
+}
+
+template <int BITS> __device__ __forceinline__ uint32_t group_offset(const uint32_t *w, uint32_t v)
+{
+    uint32_t o = 0;
+#pragma unroll
+    for (int i = 0; i < BITS; i++) o |= ((v >> i) & 1u) << group_word(w, i);
+    return o;
+}
+
 template <class R>
 __global__ __launch_bounds__(256) void grouped_small_kernel(const GroupBlock *__restrict__ blocks,
                                                             const void *const *__restrict__ ptrs)
 {
-    using C2 = typename Vec<R>::c;
-    __shared__ int32_t record[sizeof(GroupBlock) / 4];
-    const GroupBlock &g = *reinterpret_cast<const GroupBlock *>(record);
-    __shared__ const void *base[3];
-    __shared__ int32_t ka[1 << kGroupMaxLog2K], kb[1 << kGroupMaxLog2K];
-    static_assert(sizeof(GroupBlock) % 4 == 0 && sizeof(GroupBlock) / 4 <= 256, "record");
-    const int tid = threadIdx.x;
-    if (tid < int(sizeof(GroupBlock) / 4))
-        record[tid] = reinterpret_cast<const int32_t *>(blocks + blockIdx.x)[tid];
-    __syncthreads();
-    if (tid < 3) base[tid] = ptrs[tid == 0 ? g.a : tid == 1 ? g.b : g.c];
-    const int K = 1 << g.f.lk;
-    for (int k = tid; k < K; k += 256) {
-        ka[k] = int32_t(fused_offset(g.f.a_k, k));
-        kb[k] = int32_t(fused_offset(g.f.b_k, k));
-    }
-    __syncthreads();
-    const int lanes = g.lanes, G = 1 << lanes;
-    const int idx = g.first + (tid >> lanes);
-    const bool live = idx < 1 << (g.f.lb + g.f.lm + g.f.ln);
-    const int n = idx & ((1 << g.f.ln) - 1);
-    const int m = (idx >> g.f.ln) & ((1 << g.f.lm) - 1);
-    const int b = idx >> (g.f.ln + g.f.lm);
+    // global-memory pointers (generic ones would make flat loads)
+    typedef R R2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(1))) const R2 *In;
+    typedef __attribute__((address_space(1))) R2 *Out;
+    const GroupBlock g = blocks[blockIdx.x];
+    const uint32_t tid = threadIdx.x, G = 1u << g.lanes;
+    const uint32_t idx = g.first + (tid >> g.lanes), k0 = tid & (G - 1);
+    const bool live = idx < 1u << g.lo;
+    constexpr int OB = kGroupMaxLog2Outputs, KB = kGroupMaxLog2K;
+    const In x = In(ptrs[g.a]) +
+                 (group_offset<OB>(g.oa, idx & g.mask_a) | group_offset<6>(g.ka, k0));
+    const In y = In(ptrs[g.b]) +
+                 (group_offset<OB>(g.ob, idx & g.mask_b) | group_offset<6>(g.kb, k0));
     R sr = 0, si = 0;
+    auto mac = [&](R2 u, R2 v) {
+        sr = fma(u.x, v.x, sr);
+        sr = fma(-u.y, v.y, sr);
+        si = fma(u.x, v.y, si);
+        si = fma(u.y, v.x, si);
+    };
     if (live) {
-        const C2 *x = static_cast<const C2 *>(base[0]) +
-                      (fused_offset(g.f.a_b, b) | fused_offset(g.f.a_m, m));
-        const C2 *y = static_cast<const C2 *>(base[1]) +
-                      (fused_offset(g.f.b_b, b) | fused_offset(g.f.b_n, n));
-#pragma unroll 4
-        for (int k = tid & (G - 1); k < K; k += G) {
-            const C2 u = x[ka[k]], v = y[kb[k]];
-            sr = fma(u.x, v.x, sr);
-            sr = fma(-u.y, v.y, sr);
-            si = fma(u.x, v.y, si);
-            si = fma(u.y, v.x, si);
+        const uint32_t K = 1u << g.lk;
+        if (K >= 4 * G) {
+            for (uint32_t k = 0; k < K; k += 4 * G) {
+                R2 u[4], v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    u[e] = x[group_offset<KB>(g.ka, k + e * G)];
+                    v[e] = y[group_offset<KB>(g.kb, k + e * G)];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++) mac(u[e], v[e]);
+            }
         }
+        else
+            for (uint32_t k = 0; k < K; k += G)
+                mac(x[group_offset<KB>(g.ka, k)], y[group_offset<KB>(g.kb, k)]);
     }
-    for (int off = G >> 1; off > 0; off >>= 1) {
+    for (uint32_t off = G >> 1; off > 0; off >>= 1) {
         sr += __shfl_xor(sr, off);
         si += __shfl_xor(si, off);
     }
-    if (live && (tid & (G - 1)) == 0)
-        static_cast<C2 *>(const_cast<void *>(
-            base[2]))[fused_offset(g.f.c_b, b) | fused_offset(g.f.c_m, m) |
-                      fused_offset(g.f.c_n, n)] = C2{sr, si};
+    const Out z = Out(const_cast<void *>(ptrs[g.c]));
+    if (live && k0 == 0) z[group_offset<OB>(g.oc, idx)] = R2{sr, si};
 }
 
 constexpr int kPointersPerLaunch = 448; // 3.5 KiB of kernel arguments

@@ -135,14 +135,20 @@ struct FusedSmall {
 // One work-group's share of a group of independent small contractions that
 // run in one launch (grouped_small_kernel): 256 >> lanes outputs of one
 // contraction, from output `first` on, 2^lanes lanes per output.  a, b and c
-// are slots of the pointer table that the launch is given.
-constexpr int kGroupMaxLog2K = 10;       // k offset tables in LDS
-constexpr int kGroupMaxLog2Outputs = 14; // result kept apart from the arena's reuse
+// are slots of the pointer table that the launch is given.  An output's index
+// holds its n, m and batch bits, lowest first; bit i goes to the address bit
+// packed as the i-th five-bit field (six to a word) of oc, and of oa (ob)
+// where the operand has it (mask_a, mask_b); k bits likewise in ka and kb.
+constexpr int kGroupMaxLog2K = 10;
+constexpr int kGroupMaxLog2Outputs = 14; // results kept apart from the arena's reuse
 constexpr int kGroupMaxLog2Work = 20;    // outputs * K
 struct GroupBlock {
-    FusedSmall f;
     int32_t a = 0, b = 0, c = 0;
     int32_t first = 0, lanes = 0;
+    int32_t lo = 0, lk = 0; // log2 of outputs and K
+    uint32_t mask_a = 0, mask_b = 0;
+    uint32_t oa[3] = {}, ob[3] = {}, oc[3] = {};
+    uint32_t ka[2] = {}, kb[2] = {};
 };
 
 // Split-BF16 operand: planes re hi/lo, im hi/lo[, re+im hi/lo].
