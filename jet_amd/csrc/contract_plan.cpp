@@ -183,42 +183,57 @@ bool plan_fused_small(const std::vector<int32_t> &a, const std::vector<int64_t> 
     return f.lk <= kFusedMaxLog2K;
 }
 
+namespace {
+
+// One entry per address bit of a row-major tensor, lowest first: the (mode,
+// bit) it holds.  False for extents that are not powers of two and beyond
+// 2^31 elements.
+typedef std::vector<std::pair<int32_t, int>> Bits;
+bool address_bits(const std::vector<int32_t> &m, const std::vector<int64_t> &e, Bits &out)
+{
+    for (size_t i = m.size(); i-- > 0;) {
+        if (e[i] < 1 || (e[i] & (e[i] - 1))) return false;
+        for (int t = 0; (int64_t(1) << t) < e[i]; t++) out.push_back({m[i], t});
+    }
+    return out.size() <= 31;
+}
+
+int bit_at(const Bits &v, const std::pair<int32_t, int> &q)
+{
+    const auto it = std::find(v.begin(), v.end(), q);
+    return it == v.end() ? -1 : int(it - v.begin());
+}
+
+bool result_bits(const std::vector<int32_t> &a, const std::vector<int64_t> &ea,
+                 const std::vector<int32_t> &b, const std::vector<int64_t> &eb,
+                 const std::vector<int32_t> &c, Bits &out)
+{
+    std::vector<int64_t> ec;
+    for (int32_t m : c) ec.push_back(find(a, m) >= 0 ? ea[find(a, m)] : eb[find(b, m)]);
+    return address_bits(c, ec, out);
+}
+
+} // namespace
+
 bool plan_stream_shortk(const std::vector<int32_t> &a, const std::vector<int64_t> &ea,
                         const std::vector<int32_t> &b, const std::vector<int64_t> &eb,
                         const std::vector<int32_t> &c, StreamShortK &p)
 {
-    // One entry per address bit of A, B and C: the (mode, bit) it holds,
-    // lowest bit first.
-    typedef std::vector<std::pair<int32_t, int>> Bits;
-    auto bits_of = [](const std::vector<int32_t> &m, const std::vector<int64_t> &e, Bits &out) {
-        for (size_t i = m.size(); i-- > 0;) {
-            if (e[i] < 1 || (e[i] & (e[i] - 1))) return false;
-            for (int t = 0; (int64_t(1) << t) < e[i]; t++) out.push_back({m[i], t});
-        }
-        return out.size() <= 31;
-    };
     Bits ba, bb, bc;
-    if (!bits_of(a, ea, ba) || !bits_of(b, eb, bb)) return false;
-    std::vector<int64_t> ec;
-    for (int32_t m : c) ec.push_back(find(a, m) >= 0 ? ea[find(a, m)] : eb[find(b, m)]);
-    if (!bits_of(c, ec, bc)) return false;
+    if (!address_bits(a, ea, ba) || !address_bits(b, eb, bb) ||
+        !result_bits(a, ea, b, eb, c, bc))
+        return false;
     p = StreamShortK{};
     p.swap = bb.size() > ba.size() ? 1 : 0;
     const Bits &x = p.swap ? bb : ba, &y = p.swap ? ba : bb;
-    auto at = [](const Bits &v, const std::pair<int32_t, int> &q) {
-        return int(std::find(v.begin(), v.end(), q) - v.begin());
-    };
-    auto in = [&](const Bits &v, const std::pair<int32_t, int> &q) {
-        return at(v, q) < (int)v.size();
-    };
     for (int i = 0; i < (int)x.size(); i++) {
-        const int yi = at(y, x[i]), ci = at(bc, x[i]);
-        if (!in(bc, x[i])) {
+        const int yi = bit_at(y, x[i]), ci = bit_at(bc, x[i]);
+        if (ci < 0) {
             if (p.lk == kStreamMaxLog2K) return false;
             p.xk[p.lk] = int8_t(i);
             p.yk[p.lk++] = int8_t(yi);
         }
-        else if (in(y, x[i])) {
+        else if (yi >= 0) {
             if (p.lb == kStreamMaxBatch || i < 4 || ci < 4) return false;
             p.xb[p.lb] = int8_t(i);
             p.yb[p.lb] = int8_t(yi);
@@ -239,12 +254,126 @@ bool plan_stream_shortk(const std::vector<int32_t> &a, const std::vector<int64_t
         }
     }
     for (int i = 0; i < (int)bc.size(); i++)
-        if (!in(x, bc[i])) {
+        if (bit_at(x, bc[i]) < 0) {
             if (p.ln == kStreamMaxLog2N) return false;
-            p.yn[p.ln] = int8_t(at(y, bc[i]));
+            p.yn[p.ln] = int8_t(bit_at(y, bc[i]));
             p.cn[p.ln++] = int8_t(i);
         }
     return p.lr >= 1;
+}
+
+bool plan_stream_dot(int elem_bytes, const std::vector<int32_t> &a, const std::vector<int64_t> &ea,
+                     const std::vector<int32_t> &b, const std::vector<int64_t> &eb,
+                     const std::vector<int32_t> &c, StreamDot &p)
+{
+    Bits ba, bb, bc;
+    if (!address_bits(a, ea, ba) || !address_bits(b, eb, bb) ||
+        !result_bits(a, ea, b, eb, c, bc))
+        return false;
+    p = StreamDot{};
+    p.swap = bb.size() > ba.size() ? 1 : 0; // they share their k and batch bits
+    if (p.swap) std::swap(ba, bb);
+    // Kinds of A's and B's bits: k (in both, summed), batch (in all), own.
+    std::vector<char> in_tile_a(ba.size(), 0), in_tile_b(bb.size(), 0);
+    for (size_t i = 0; i < ba.size(); i++) {
+        const int j = bit_at(bb, ba[i]), ci = bit_at(bc, ba[i]);
+        if (j < 0) {
+            if (p.lm == kDotMaxLog2MN) return false;
+            p.lm++;
+            in_tile_a[i] = 1;
+        }
+        else if (ci < 0)
+            p.lk++;
+        else
+            p.lb++;
+    }
+    for (size_t i = 0; i < bb.size(); i++)
+        if (bit_at(ba, bb[i]) < 0) {
+            if (p.ln == kDotMaxLog2MN) return false;
+            p.ln++;
+            in_tile_b[i] = 1;
+        }
+    p.xm = std::max(0, p.lm + p.ln - kDotMaxLog2Sums);
+    if (p.xm > 2 || p.lb + p.lm + p.ln > 16 || p.lk < 12) return false;
+    // The tile: lowest bits of A and B in turn while both parts fit.
+    const int cap = elem_bytes == 8 ? kDotMaxLog2Tile : kDotMaxLog2Tile - 1;
+    size_t ia = 0, ib = 0; // bits below are in the tile
+    int lt = 0, tb = 0;
+    auto take = [&](const Bits &own, const Bits &other, std::vector<char> &mine,
+                    std::vector<char> &theirs, size_t &i) {
+        if (i == own.size()) return false;
+        if (!mine[i]) {
+            const bool k = bit_at(bc, own[i]) < 0;
+            if (lt + tb + 1 + std::max(p.lm, p.ln) > cap) return false;
+            if (!k && (tb == kDotMaxTileBatch || tb + p.xm == 6 ||
+                       tb + p.lm + p.ln == kDotMaxLog2Lanes))
+                return false;
+            mine[i] = 1;
+            theirs[bit_at(other, own[i])] = 1;
+            (k ? lt : tb)++;
+        }
+        i++;
+        return true;
+    };
+    for (bool more = true; more;) {
+        const bool x = take(ba, bb, in_tile_a, in_tile_b, ia);
+        const bool y = take(bb, ba, in_tile_b, in_tile_a, ib);
+        more = x || y;
+    }
+    // Runs of at least 128 bytes (64 of an operand a quarter as large), and
+    // work for every thread (m bits go across threads where the tile has few k).
+    const size_t run_a = elem_bytes == 8 ? 4 : 3, run_b = run_a - (p.lm >= p.ln + 2 ? 1 : 0);
+    p.xm = std::max(p.xm, 8 - lt - tb);
+    if (ia < run_a || ib < run_b || p.xm > p.lm || tb + p.xm > 6 || p.lb - tb > 15 ||
+        p.lk - lt > 24)
+        return false;
+    p.lt = lt;
+    p.tb = tb;
+    // Tile bits, and where each k, m, n and batch bit lies.
+    int na = 0, nb = 0;
+    std::vector<int> tile_a(ba.size(), -1), tile_b(bb.size(), -1);
+    for (size_t i = 0; i < ba.size(); i++)
+        if (in_tile_a[i]) {
+            p.a_pos[na] = int8_t(i);
+            tile_a[i] = na++;
+        }
+    for (size_t i = 0; i < bb.size(); i++)
+        if (in_tile_b[i]) {
+            p.b_pos[nb] = int8_t(i);
+            tile_b[i] = nb++;
+        }
+    int k = 0, m = 0, n = 0, t = 0, ok = 0, ob = 0;
+    for (size_t i = 0; i < ba.size(); i++) {
+        const int j = bit_at(bb, ba[i]), ci = bit_at(bc, ba[i]);
+        if (j < 0) {
+            p.am[m] = int8_t(tile_a[i]);
+            p.cm[m++] = int8_t(ci);
+        }
+        else if (ci < 0 && in_tile_a[i]) {
+            p.ak[k] = int8_t(tile_a[i]);
+            p.bk[k++] = int8_t(tile_b[j]);
+        }
+        else if (ci < 0) {
+            p.oak[ok] = int8_t(i);
+            p.obk[ok++] = int8_t(j);
+        }
+        else if (in_tile_a[i]) {
+            p.ab[t] = int8_t(tile_a[i]);
+            p.bb[t] = int8_t(tile_b[j]);
+            p.ctb[t++] = int8_t(ci);
+        }
+        else {
+            p.oab[ob] = int8_t(i);
+            p.obb[ob] = int8_t(j);
+            p.cob[ob++] = int8_t(ci);
+        }
+    }
+    for (size_t i = 0; i < bb.size(); i++)
+        if (bit_at(ba, bb[i]) < 0) {
+            p.bn[n] = int8_t(tile_b[i]);
+            p.cn[n++] = int8_t(bit_at(bc, bb[i]));
+        }
+    return true;
 }
 
 int gemm_variants(int kernel)
@@ -505,6 +634,20 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
         return d;
     }
 
+    // Few outputs and many k: one pass over both operands in place (also
+    // where neither needs a permutation: the split-K kernel reads a row once
+    // per output it takes part in; only single products are its own: 2^22 k
+    // 16 us against 23).
+    if (d.chunks == 1 && (d.need_a || d.need_b || d.M * d.N > 1) && std::max(d.size_a, d.size_b) >= (int64_t(1) << 16) &&
+        plan_stream_dot(elem_bytes, A, EA, B, EB, C, d.dot)) {
+        d.stream_dot = true;
+        d.gemm_kernel = kGemmSplitK;
+        d.gemm_variant = 0;
+        d.fuse_a = d.fuse_b = false;
+        layout_workspace(d);
+        return d;
+    }
+
     // Small steps on the one-thread-per-output or the one-block-per-output
     // VALU kernel that would need a permuted operand or result: one fused
     // pass of the same form, no copies.
@@ -527,6 +670,11 @@ void layout_workspace(ContractionDesc &d)
     const size_t eb = (size_t)d.elem_bytes;
     if (d.fused_small || d.stream_shortk) { // reads and writes the tensors in place
         d.workspace = 0;
+        return;
+    }
+    if (d.stream_dot) {
+        d.off_partials = 0;
+        d.workspace = align256(16 * (size_t)d.dot.outputs() * (size_t)d.dot.chunks());
         return;
     }
     if (d.need_a && !d.fuse_a) {

@@ -43,6 +43,9 @@ struct ContractionDesc {
     // a few k and columns of a large operand: read in place (StreamShortK)
     bool stream_shortk = false;
     StreamShortK sk;
+    // few outputs and many k of two large operands: read in place (StreamDot)
+    bool stream_dot = false;
+    StreamDot dot;
     int gemm_kernel = kGemmSmall;
     int gemm_variant = 0; // tile variant of gemm_kernel (GemmChoice)
     // K split into `chunks` pieces that run as a batch of the MFMA GEMM

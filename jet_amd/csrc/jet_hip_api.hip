@@ -152,6 +152,10 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
         launch_stream_shortk(d.sk, eb, a, b, c, s);
         return;
     }
+    if (d.stream_dot) {
+        launch_stream_dot(d.dot, eb, a, b, c, ws + d.off_partials, s);
+        return;
+    }
     const void *At = a;
     const void *Bt = b;
     if (d.need_a && !d.fuse_a) {

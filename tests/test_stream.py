@@ -1,11 +1,13 @@
-"""In-place contractions of a small tensor with a large one: the plan's offset
+"""In-place contractions of a small tensor with a large one, and of two large
+tensors with few outputs: the plans' offset
 arithmetic on the CPU (tests/native/stream_check.cpp) against numpy's einsum
 over random mode orders, batch modes and permuted results, which forms are
 refused, and the kernels on the GPU against numpy in 64 bits.
 
 GPU tolerance: K <= 16 products summed one after the other, each rounded
 twice: 2 K units of 2^-24 (2^-53) of the sum of magnitudes, normwise under
-2^-24 * 8 (2^-53 * 8) for random operands.
+2^-24 * 8 (2^-53 * 8) for random operands.  The few-output form sums in FP64: 2^-23
+for complex64 (the result's rounding), 2^-53 sqrt(K) for complex128.
 """
 import ctypes
 import os
@@ -128,3 +130,75 @@ def test_gpu(dtype, u, seed):
     if dtype == np.complex128:
         want = _want(a, b, c, ext, x.astype(np.clongdouble), y.astype(np.clongdouble))
     assert np.linalg.norm(got - want) < 8 * u * np.linalg.norm(want)
+
+
+def _dot_case(rng, k, m, n, batch, spread):
+    """Modes of extent 2; batch modes leading, or anywhere (spread)."""
+    ids = list(range(k + m + n + batch))
+    kk, mm = ids[:k], ids[k:k + m]
+    nn, bb = ids[k + m:k + m + n], ids[k + m + n:]
+    head = [] if spread else bb
+    tail = bb if spread else []
+    a = head + [int(x) for x in rng.permutation(kk + mm + tail)]
+    b = head + [int(x) for x in rng.permutation(kk + nn + tail)]
+    c = [int(x) for x in rng.permutation(bb + mm + nn)]
+    return a, b, c, {i: 2 for i in ids}
+
+
+@pytest.mark.parametrize("elem", [8, 16])
+@pytest.mark.parametrize("seed", range(30))
+def test_few_outputs_match_einsum(lib, elem, seed):
+    rng = np.random.default_rng(seed)
+    m, n, batch = (int(x) for x in rng.integers(0, [5, 5, 4]))
+    a, b, c, ext = _dot_case(rng, int(rng.integers(12, 14)), m, n, batch, bool(seed % 2))
+    size = lambda ms: int(np.prod([ext[x] for x in ms])) if ms else 1
+    x = rng.standard_normal(size(a)) + 1j * rng.standard_normal(size(a))
+    y = rng.standard_normal(size(b)) + 1j * rng.standard_normal(size(b))
+    got = np.zeros(size(c), np.complex128)
+    p = lambda v: v.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    rc = lib.stream_dot_emulate(elem, *_args(a, b, c, ext), p(x), p(y), ctypes.c_int64(size(c)),
+                                p(got))
+    if rc == 1:   # refused: too many outputs, or low bits that do not fit a tile
+        assert m + n > 4 or batch > 0
+        return
+    assert rc == 0
+    np.testing.assert_allclose(got, _want(a, b, c, ext, x, y), rtol=1e-10, atol=1e-9)
+
+
+def test_few_outputs_routes(lib):
+    def route(k, m, n, batch, spread=False, ext=None):
+        a, b, c, e = _dot_case(np.random.default_rng(1), k, m, n, batch, spread)
+        ws = ctypes.c_size_t()
+        return lib.stream_route(*_args(a, b, c, {**e, **(ext or {})}), ctypes.byref(ws)), ws.value
+    assert route(18, 2, 1, 0)[0] == 2
+    assert 0 < route(18, 2, 1, 4)[1] <= 4 << 20
+    assert route(18, 3, 3, 0)[0] == 2
+    assert route(18, 5, 0, 0)[0] == 0            # 32 rows
+    assert route(18, 4, 4, 0)[0] == 0            # 256 outputs
+    assert route(18, 2, 1, 0, ext={0: 3})[0] == 0
+    assert route(11, 2, 1, 6)[0] == 0            # 2^11 k
+    # one product of operands in the same order: split-K reads each once as it is
+    one = {i: 2 for i in range(18)}
+    ws = ctypes.c_size_t()
+    assert lib.stream_route(*_args(list(range(18)), list(range(18)), [], one),
+                            ctypes.byref(ws)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("k,m,n,batch,spread", [
+    (16, 0, 0, 0, False), (16, 2, 1, 0, False), (17, 0, 3, 0, False), (17, 3, 3, 0, False),
+    (16, 4, 2, 0, False), (16, 2, 4, 0, False), (16, 1, 0, 5, False), (14, 1, 1, 6, False),
+    (16, 1, 1, 2, True), (16, 0, 0, 4, True), (15, 2, 2, 3, True), (20, 1, 2, 0, False),
+    (12, 4, 0, 8, False), (12, 0, 4, 10, False)])
+def test_gpu_few_outputs(dtype, k, m, n, batch, spread):
+    rng = np.random.default_rng(k + 7 * m + 11 * n)
+    a, b, c, ext = _dot_case(rng, k, m, n, batch, spread)
+    size = lambda ms: int(np.prod([ext[v] for v in ms])) if ms else 1
+    x, y = rand_c(rng, size(a), dtype), rand_c(rng, size(b), dtype)
+    say(f"few outputs: K 2^{k}, M 2^{m}, N 2^{n}, batch 2^{batch}, {np.dtype(dtype).name}")
+    got, _ = contract(nat.default_context(), x, a, [ext[v] for v in a], y, b,
+                      [ext[v] for v in b], c, workspace=True)
+    want = _want(a, b, c, ext, x.astype(np.complex128), y.astype(np.complex128))
+    tol = 2.0 ** -23 if dtype == np.complex64 else 2.0 ** -53 * np.sqrt(2.0 ** k)
+    assert np.linalg.norm(got - want) < tol * np.linalg.norm(want)
