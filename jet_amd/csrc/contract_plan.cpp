@@ -180,7 +180,40 @@ bool plan_fused_small(const std::vector<int32_t> &a, const std::vector<int64_t> 
     f.lm = f.a_m.n;
     f.ln = f.b_n.n;
     f.lk = f.a_k.n;
-    return f.lk <= kFusedMaxLog2K;
+    return f.lk <= kFusedMaxLog2K && f.lb + f.lm + f.ln <= kSmallMaxLog2Outputs;
+}
+
+GroupBlock group_record(const FusedSmall &f)
+{
+    GroupBlock g;
+    g.lo = f.lb + f.lm + f.ln;
+    g.lk = f.lk;
+    auto put = [](uint32_t *words, int i, int pos) {
+        words[i / 6] |= uint32_t(pos) << (5 * (i % 6));
+    };
+    for (int i = 0; i < f.ln; i++) {
+        g.mask_b |= 1u << i;
+        put(g.ob, i, f.b_n.pos[i]);
+        put(g.oc, i, f.c_n.pos[i]);
+    }
+    for (int i = 0; i < f.lm; i++) {
+        g.mask_a |= 1u << (f.ln + i);
+        put(g.oa, f.ln + i, f.a_m.pos[i]);
+        put(g.oc, f.ln + i, f.c_m.pos[i]);
+    }
+    for (int i = 0; i < f.lb; i++) {
+        const int j = f.ln + f.lm + i;
+        g.mask_a |= 1u << j;
+        g.mask_b |= 1u << j;
+        put(g.oa, j, f.a_b.pos[i]);
+        put(g.ob, j, f.b_b.pos[i]);
+        put(g.oc, j, f.c_b.pos[i]);
+    }
+    for (int i = 0; i < f.lk; i++) {
+        put(g.ka, i, f.a_k.pos[i]);
+        put(g.kb, i, f.b_k.pos[i]);
+    }
+    return g;
 }
 
 namespace {
@@ -612,6 +645,22 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
             }
         }
     }
+    // Both sides at least 32 and a long k on a VALU reduction, whose table
+    // entry stems from one walk of k per matrix-core tile: the matrix cores with
+    // slices of k where they are faster.  The reduction reads its operands once per
+    // output (64x64x1024 7.0 us: 9.6 TB/s out of L2).
+    if (d.chunks == 1 && mode != 2 && d.M >= 32 && d.N >= 32 && d.K >= 2048 &&
+        f32x6_shape(d.M, d.N, d.K) && d.batch <= 65535 &&
+        (d.gemm_kernel == kGemmSmallRed || d.gemm_kernel == kGemmSplitK)) {
+        double us = 0;
+        (void)f32x6_slices(d.M, d.N, d.K, d.batch, &us);
+        const double red = double(d.batch) * double(d.M) * double(d.N) * double(d.K) * 16.0 / 9.6e6;
+        const double copies = (d.need_a ? 4.0 : 0.0) + (d.need_b ? 4.0 : 0.0);
+        if (us + copies < red) {
+            d.gemm_kernel = kGemmF32Mfma;
+            d.gemm_variant = 0;
+        }
+    }
     if (d.gemm_kernel == kGemmF16x4m) {
         // fold a permutation into the split pass when the rows need no
         // padding (the split rows are then the permuted rows)
@@ -657,7 +706,6 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
     if ((small || red) && (d.need_a || d.need_b || d.need_c)) {
         const auto &common = best_opt == 0 ? common_a : common_b;
         d.fused_small = plan_fused_small(A, EA, B, EB, C, batch, left, right, common, d.fs);
-        d.fs.red = red ? 1 : 0;
     }
 
     layout_workspace(d);
@@ -720,14 +768,16 @@ void layout_workspace(ContractionDesc &d)
         off = align256(off + eb * (size_t)d.batch * (size_t)d.M * (size_t)d.N);
     }
     d.slices = 1;
-    if ((d.gemm_kernel == kGemmBf16x4m || d.gemm_kernel == kGemmF16x4m) && d.chunks == 1) {
-        const int64_t n = x4m_slices(d.M, d.N, d.K, d.batch, d.gemm_variant);
-        const size_t bytes = align256(eb * (size_t)n * (size_t)d.size_c);
+    int64_t slices = 1;
+    if (d.chunks == 1 && (d.gemm_kernel == kGemmBf16x4m || d.gemm_kernel == kGemmF16x4m))
+        slices = x4m_slices(d.M, d.N, d.K, d.batch, d.gemm_variant);
+    else if (d.chunks == 1 && d.gemm_kernel == kGemmF32Mfma && f32x6_shape(d.M, d.N, d.K))
+        slices = f32x6_slices(d.M, d.N, d.K, d.batch, nullptr);
+    if (slices > 1) {
+        const size_t bytes = align256(eb * (size_t)slices * (size_t)d.size_c);
         // a plan that fits the no-allocation scratch array keeps doing so
-        const bool fits = off > JET_HIP_NOALLOC_SCRATCH_BYTES ||
-                          off + bytes <= JET_HIP_NOALLOC_SCRATCH_BYTES;
-        if (n > 1 && fits) {
-            d.slices = n;
+        if (off > JET_HIP_NOALLOC_SCRATCH_BYTES || off + bytes <= JET_HIP_NOALLOC_SCRATCH_BYTES) {
+            d.slices = slices;
             d.off_slices = off;
             off += bytes;
         }

@@ -219,117 +219,16 @@ __global__ __launch_bounds__(256) void cgemm_small_kernel(GemmArgs g)
     }
 }
 
-// Fused small contraction (FusedSmall): one thread per output element
-// (batch b, row m, column n), the element offsets of A, B and C assembled
-// from their group bits; the k offsets of A and B come from LDS tables that
-// each work-group fills once.  Same summation order and FMA sequence as
-// cgemm_small_kernel.
-__device__ __forceinline__ int64_t fused_offset(const FusedBits &f, int64_t x)
-{
-    int64_t o = 0;
-    for (int i = 0; i < f.n; i++) o |= ((x >> i) & 1) << f.pos[i];
-    return o;
-}
-
-template <class R>
-__global__ __launch_bounds__(256) void fused_small_kernel(const void *Av, const void *Bv,
-                                                          void *Cv, FusedSmall f)
-{
-    using C2 = typename Vec<R>::c;
-    extern __shared__ int32_t koff[]; // [K] offsets in A, then [K] in B
-    const int64_t K = int64_t(1) << f.lk;
-    int32_t *ka = koff, *kb = koff + K;
-    for (int64_t k = threadIdx.x; k < K; k += blockDim.x) {
-        ka[k] = int32_t(fused_offset(f.a_k, k));
-        kb[k] = int32_t(fused_offset(f.b_k, k));
-    }
-    __syncthreads();
-    const C2 *__restrict__ A = static_cast<const C2 *>(Av);
-    const C2 *__restrict__ B = static_cast<const C2 *>(Bv);
-    C2 *__restrict__ C = static_cast<C2 *>(Cv);
-    const int64_t total = int64_t(1) << (f.lb + f.lm + f.ln);
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-    for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < total;
-         idx += stride) {
-        const int64_t n = idx & ((int64_t(1) << f.ln) - 1);
-        const int64_t m = (idx >> f.ln) & ((int64_t(1) << f.lm) - 1);
-        const int64_t b = idx >> (f.ln + f.lm);
-        const C2 *a = A + (fused_offset(f.a_b, b) | fused_offset(f.a_m, m));
-        const C2 *bb = B + (fused_offset(f.b_b, b) | fused_offset(f.b_n, n));
-        R sr = 0, si = 0;
-        for (int64_t k = 0; k < K; k++) {
-            const C2 x = a[ka[k]], y = bb[kb[k]];
-            sr = fma(x.x, y.x, sr);
-            sr = fma(-x.y, y.y, sr);
-            si = fma(x.x, y.y, si);
-            si = fma(x.y, y.x, si);
-        }
-        C[fused_offset(f.c_b, b) | fused_offset(f.c_m, m) | fused_offset(f.c_n, n)] =
-            C2{sr, si};
-    }
-}
-
-// The one-work-group-per-output form of the fused pass (few outputs, long
-// K): threads take k = t, t + 256, ..., the partial sums are reduced across
-// the wave with shuffles and across the four waves in LDS.
-template <class R>
-__global__ __launch_bounds__(256) void fused_small_red_kernel(const void *Av, const void *Bv,
-                                                              void *Cv, FusedSmall f)
-{
-    using C2 = typename Vec<R>::c;
-    extern __shared__ int32_t koff[]; // [K] offsets in A, then [K] in B
-    __shared__ R red_s[2][4];
-    const int64_t K = int64_t(1) << f.lk;
-    int32_t *ka = koff, *kb = koff + K;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int64_t k = tid; k < K; k += blockDim.x) {
-        ka[k] = int32_t(fused_offset(f.a_k, k));
-        kb[k] = int32_t(fused_offset(f.b_k, k));
-    }
-    __syncthreads();
-    const C2 *__restrict__ A = static_cast<const C2 *>(Av);
-    const C2 *__restrict__ B = static_cast<const C2 *>(Bv);
-    C2 *__restrict__ C = static_cast<C2 *>(Cv);
-    const int64_t total = int64_t(1) << (f.lb + f.lm + f.ln);
-    for (int64_t idx = blockIdx.x; idx < total; idx += gridDim.x) {
-        const int64_t n = idx & ((int64_t(1) << f.ln) - 1);
-        const int64_t m = (idx >> f.ln) & ((int64_t(1) << f.lm) - 1);
-        const int64_t b = idx >> (f.ln + f.lm);
-        const C2 *a = A + (fused_offset(f.a_b, b) | fused_offset(f.a_m, m));
-        const C2 *bb = B + (fused_offset(f.b_b, b) | fused_offset(f.b_n, n));
-        R sr = 0, si = 0;
-        for (int64_t k = tid; k < K; k += blockDim.x) {
-            const C2 x = a[ka[k]], y = bb[kb[k]];
-            sr = fma(x.x, y.x, sr);
-            sr = fma(-x.y, y.y, sr);
-            si = fma(x.x, y.y, si);
-            si = fma(x.y, y.x, si);
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            sr += __shfl_xor(sr, off);
-            si += __shfl_xor(si, off);
-        }
-        if (lane == 0) {
-            red_s[0][wave] = sr;
-            red_s[1][wave] = si;
-        }
-        __syncthreads();
-        if (tid == 0)
-            C[fused_offset(f.c_b, b) | fused_offset(f.c_m, m) | fused_offset(f.c_n, n)] =
-                C2{(red_s[0][0] + red_s[0][1]) + (red_s[0][2] + red_s[0][3]),
-                   (red_s[1][0] + red_s[1][1]) + (red_s[1][2] + red_s[1][3])};
-        __syncthreads();
-    }
-}
-
-// Independent small contractions of one dependency level in one launch: a
+// Small contractions read and written in the operands' own mode orders
+// (FusedSmall, GroupBlock): one alone (fused_small_kernel) or the independent
+// ones of one dependency level in one launch (grouped_small_kernel): a
 // circuit's network has hundreds of steps of a few dozen values, and each as
 // a launch of its own costs 3-4 us of launch and memory latency, one after
-// the other.  The kernel is a chain of latencies, so the record comes in one
+// the other.  Both are chains of latencies, so the record comes in one
 // scalar load, its bit positions packed in words (a loop over byte positions
 // waits for a load per bit), k offsets are made from them on the scalar unit
-// for the k bits that all lanes share, and there is no barrier.
+// for the k bits that all lanes share, four k at a time, and there is no
+// barrier unless an output has more lanes than a wave.
 __device__ __forceinline__ uint32_t group_word(const uint32_t *w, int i)
 {
     return (w[i / 6] >> (5 * (i % 6))) & 31u;
@@ -343,23 +242,21 @@ template <int BITS> __device__ __forceinline__ uint32_t group_offset(const uint3
     return o;
 }
 
-template <class R>
-__global__ __launch_bounds__(256) void grouped_small_kernel(const GroupBlock *__restrict__ blocks,
-                                                            const void *const *__restrict__ ptrs)
+// Output `first` + thread / 2^lanes of the work-group; OB, KB: bits of the
+// output index and of k; LANES: most lanes per output (log2).
+template <class R, int OB, int KB, int LANES>
+__device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t first,
+                                                  const void *Av, const void *Bv, void *Cv)
 {
     // global-memory pointers (generic ones would make flat loads)
     typedef R R2 __attribute__((ext_vector_type(2)));
     typedef __attribute__((address_space(1))) const R2 *In;
     typedef __attribute__((address_space(1))) R2 *Out;
-    const GroupBlock g = blocks[blockIdx.x];
     const uint32_t tid = threadIdx.x, G = 1u << g.lanes;
-    const uint32_t idx = g.first + (tid >> g.lanes), k0 = tid & (G - 1);
+    const uint32_t idx = first + (tid >> g.lanes), k0 = tid & (G - 1);
     const bool live = idx < 1u << g.lo;
-    constexpr int OB = kGroupMaxLog2Outputs, KB = kGroupMaxLog2K;
-    const In x = In(ptrs[g.a]) +
-                 (group_offset<OB>(g.oa, idx & g.mask_a) | group_offset<6>(g.ka, k0));
-    const In y = In(ptrs[g.b]) +
-                 (group_offset<OB>(g.ob, idx & g.mask_b) | group_offset<6>(g.kb, k0));
+    const In x = In(Av) + (group_offset<OB>(g.oa, idx & g.mask_a) | group_offset<LANES>(g.ka, k0));
+    const In y = In(Bv) + (group_offset<OB>(g.ob, idx & g.mask_b) | group_offset<LANES>(g.kb, k0));
     R sr = 0, si = 0;
     auto mac = [&](R2 u, R2 v) {
         sr = fma(u.x, v.x, sr);
@@ -385,12 +282,46 @@ __global__ __launch_bounds__(256) void grouped_small_kernel(const GroupBlock *__
             for (uint32_t k = 0; k < K; k += G)
                 mac(x[group_offset<KB>(g.ka, k)], y[group_offset<KB>(g.kb, k)]);
     }
-    for (uint32_t off = G >> 1; off > 0; off >>= 1) {
+    for (uint32_t off = min(G, 64u) >> 1; off > 0; off >>= 1) {
         sr += __shfl_xor(sr, off);
         si += __shfl_xor(si, off);
     }
-    const Out z = Out(const_cast<void *>(ptrs[g.c]));
+    if constexpr (LANES > 6) {
+        __shared__ R sums[2][4];
+        if (g.lanes > 6) { // 128 or 256 lanes: two outputs or one
+            if ((tid & 63) == 0) {
+                sums[0][tid >> 6] = sr;
+                sums[1][tid >> 6] = si;
+            }
+            __syncthreads();
+            const int w = tid >> 6;
+            sr = sums[0][w];
+            si = sums[1][w];
+            for (uint32_t i = 1; i < G >> 6; i++) {
+                sr += sums[0][(w + i) & 3];
+                si += sums[1][(w + i) & 3];
+            }
+        }
+    }
+    const Out z = Out(Cv);
     if (live && k0 == 0) z[group_offset<OB>(g.oc, idx)] = R2{sr, si};
+}
+
+template <class R>
+__global__ __launch_bounds__(256) void grouped_small_kernel(const GroupBlock *__restrict__ blocks,
+                                                            const void *const *__restrict__ ptrs)
+{
+    const GroupBlock g = blocks[blockIdx.x];
+    small_contraction<R, kGroupMaxLog2Outputs, kGroupMaxLog2K, 6>(
+        g, g.first, ptrs[g.a], ptrs[g.b], const_cast<void *>(ptrs[g.c]));
+}
+
+template <class R>
+__global__ __launch_bounds__(256) void fused_small_kernel(const void *A, const void *B, void *C,
+                                                          GroupBlock g)
+{
+    small_contraction<R, kSmallMaxLog2Outputs, kFusedMaxLog2K, 8>(
+        g, blockIdx.x * (256u >> g.lanes), A, B, C);
 }
 
 constexpr int kPointersPerLaunch = 448; // 3.5 KiB of kernel arguments
@@ -878,11 +809,18 @@ __global__ __launch_bounds__(256) void split_f16_gather_kernel(
     // no barrier between the maxima and the split)
     const bool wave_rows = kq_bits <= 6;
     const int nrows = 1 << g.xr;
-    // v-bit -> u-bit
-    int v2u[16];
+    // v-bit -> u-bit.  Here and below loops run over the fixed arrays (bits
+    // that are not there are zero): a loop to the plan's count would load
+    // each position of the kernel arguments as it comes to it.
+    constexpr int TB = kGatherTileBits;
+    int v2u[TB];
 #pragma unroll
-    for (int j = 0; j < 16; j++) v2u[j] = 0;
-    for (int j = 0; j < g.tb; j++) v2u[g.u2v[j]] = j;
+    for (int v = 0; v < TB; v++) {
+        v2u[v] = 0;
+#pragma unroll
+        for (int j = 0; j < TB; j++)
+            if (j < g.tb && g.u2v[j] == v) v2u[v] = j;
+    }
     // loads: pairs (u, u + 1), u even
     int64_t soff[kGatherPairs];
     int ls0[kGatherPairs], ls1[kGatherPairs];
@@ -890,8 +828,8 @@ __global__ __launch_bounds__(256) void split_f16_gather_kernel(
     for (int e = 0; e < kGatherPairs; e++) {
         const int u = 2 * (tid + e * 256);
         int64_t o = 0;
-        for (int j = 1; j < g.tb; j++)
-            if ((u >> j) & 1) o += int64_t(1) << g.su[j];
+#pragma unroll
+        for (int j = 1; j < TB; j++) o |= int64_t((u >> j) & 1) << g.su[j];
         soff[e] = o;
         ls0[e] = gather_lds_index(u);
         ls1[e] = gather_lds_index(u + 1);
@@ -912,24 +850,26 @@ __global__ __launch_bounds__(256) void split_f16_gather_kernel(
         const int q = tid + c * 256;
         const int v = q * 8;
         int u = 0;
-        for (int j = 3; j < g.tb; j++)
-            if ((v >> j) & 1) u |= 1 << v2u[j];
+#pragma unroll
+        for (int j = 3; j < TB; j++) u |= ((v >> j) & 1) << v2u[j];
         cbase[c] = u;
         crow[c] = q >> kq_bits;
         ckq[c] = q & ((1 << kq_bits) - 1);
         int64_t ro = 0;
-        for (int i = 0; i < g.xr; i++)
-            if ((crow[c] >> i) & 1) ro += int64_t(1) << g.vrow[i];
+#pragma unroll
+        for (int i = 0; i < 7; i++) ro |= int64_t((crow[c] >> i) & 1) << g.vrow[i];
         croff[c] = ro;
     }
     const int64_t ntiles = int64_t(1) << g.nw;
     const int kt = 1 << (g.log2k - 5); // 32-wide k tiles per row
     _Float16 *base = static_cast<_Float16 *>(dst.base);
     // the next tile's loads are issued before the current tile is split
-    auto tile_src = [&](int64_t w) {
+    constexpr int FAST = 24; // tile number bits without a loop
+    auto tile_src = [&](int64_t w) __attribute__((always_inline)) {
         int64_t sb = 0;
-        for (int j = 0; j < g.nw; j++)
-            if ((w >> j) & 1) sb += int64_t(1) << g.wsrc[j];
+#pragma unroll
+        for (int j = 0; j < FAST; j++) sb |= ((w >> j) & 1) << g.wsrc[j];
+        for (int j = FAST; j < g.nw; j++) sb |= ((w >> j) & 1) << g.wsrc[j];
         return sb;
     };
     float4 nx[kGatherPairs];
@@ -951,8 +891,9 @@ __global__ __launch_bounds__(256) void split_f16_gather_kernel(
     if (int64_t(blockIdx.x) < ntiles) fetch(blockIdx.x);
     for (int64_t w = blockIdx.x; w < ntiles; w += gridDim.x) {
         int64_t rbase = 0;
-        for (int j = 0; j < g.nw; j++)
-            if ((w >> j) & 1) rbase += int64_t(1) << g.wrow[j];
+#pragma unroll
+        for (int j = 0; j < FAST; j++) rbase |= ((w >> j) & 1) << g.wrow[j];
+        for (int j = FAST; j < g.nw; j++) rbase |= ((w >> j) & 1) << g.wrow[j];
         if (!wave_rows && tid < nrows) rowmax[tid] = 0u;
 #pragma unroll
         for (int e = 0; e < kGatherPairs; e++)
@@ -1952,7 +1893,7 @@ void launch_gemm(int kernel, int elem_bytes, const GemmArgs &g,
         JH_REQUIRE(ceil_div(g.M, BM) * ceil_div(g.N, BN) <= 0x7fffffff, "Too many tiles.");
         dim3 grid((unsigned)(ceil_div(g.M, BM) * ceil_div(g.N, BN)), 1, (unsigned)g.batch);
         prof::Scope ps(prof::kGemmF32, stream, gemm_flops(g), gemm_bytes(g, 8));
-        if (f32x6_applies(g)) {
+        if (f32x6_shape(g.M, g.N, g.K)) {
             launch_f32x6(g, stream);
             return;
         }
@@ -2169,34 +2110,18 @@ void launch_gemm_bf16x4m(const SplitOperand &a, const SplitOperand &b, int64_t K
 void launch_fused_small(const FusedSmall &f, int elem_bytes, const void *a, const void *b,
                         void *c, hipStream_t stream)
 {
-    JH_REQUIRE(f.lk <= kFusedMaxLog2K && f.lb + f.lm + f.ln <= 31, "Fused step out of range.");
-    const int64_t total = int64_t(1) << (f.lb + f.lm + f.ln);
-    const double K = double(int64_t(1) << f.lk);
-    prof::Scope ps(prof::kGemmSmall, stream, 8.0 * double(total) * K,
+    JH_REQUIRE(f.lk <= kFusedMaxLog2K && f.lb + f.lm + f.ln <= kSmallMaxLog2Outputs,
+               "Fused step out of range.");
+    GroupBlock g = group_record(f);
+    g.lanes = group_lanes(g, 8, 18);
+    const int64_t total = int64_t(1) << g.lo;
+    prof::Scope ps(prof::kGemmSmall, stream, 8.0 * double(total) * double(int64_t(1) << f.lk),
                    double(elem_bytes) * double(total));
-    const size_t lds = size_t(2) * sizeof(int32_t) << f.lk;
-    if (f.red) {
-        // Eight work-groups per CU at most: each builds its k offset tables
-        // once and walks many outputs (one work-group per output rebuilt the
-        // tables for every output, about half of the time of a many-output
-        // step).
-        const unsigned grid = (unsigned)std::min<int64_t>(total, 2048);
-        if (elem_bytes == 8)
-            hipLaunchKernelGGL(fused_small_red_kernel<float>, dim3(grid), dim3(256), lds, stream,
-                               a, b, c, f);
-        else
-            hipLaunchKernelGGL(fused_small_red_kernel<double>, dim3(grid), dim3(256), lds,
-                               stream, a, b, c, f);
-        JH_HIP(hipGetLastError());
-        return;
-    }
-    const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(total, int64_t(256)), 4096);
+    const dim3 grid((unsigned)ceil_div(total << g.lanes, int64_t(256)));
     if (elem_bytes == 8)
-        hipLaunchKernelGGL(fused_small_kernel<float>, dim3(grid), dim3(256), lds, stream, a, b,
-                           c, f);
+        hipLaunchKernelGGL(fused_small_kernel<float>, grid, dim3(256), 0, stream, a, b, c, g);
     else
-        hipLaunchKernelGGL(fused_small_kernel<double>, dim3(grid), dim3(256), lds, stream, a,
-                           b, c, f);
+        hipLaunchKernelGGL(fused_small_kernel<double>, grid, dim3(256), 0, stream, a, b, c, g);
     JH_HIP(hipGetLastError());
 }
 

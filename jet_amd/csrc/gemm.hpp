@@ -22,6 +22,10 @@ struct GemmArgs {
     int64_t lda, ldb, ldc; // row strides in elements
     int64_t sA, sB, sC;    // batch strides in elements (0 = broadcast)
     int variant = 0;       // tile / thread-mapping variant (GemmChoice)
+    // FP32 products on the BF16 matrix cores: slices of slice_k k each write a
+    // result of their own, slice_stride elements apart (f32x6_slices).
+    int slices = 1;
+    int64_t slice_k = 0, slice_stride = 0;
 };
 
 // Kernel families (also reported by jet_hip_plan_info).
@@ -77,6 +81,14 @@ inline int64_t splitk_partials(int64_t outputs, int64_t K)
     return outputs * ceil_div(K, splitk_chunk(K));
 }
 
+// Whether the FP32 products run on the BF16 matrix cores: the lane offsets are
+// 32 bits (rows to 2^21 k); 32x32 blocks of which less than half would be
+// outputs, and less than one k step, are left to the FP32 MFMA kernel.
+inline bool f32x6_shape(int64_t M, int64_t N, int64_t K)
+{
+    return K >= 16 && K <= (int64_t(1) << 21) && M >= 16 && N >= 16;
+}
+
 // 4M split products with few 128x128 tiles: slices of k (at least 256 each)
 // that fill the 256 CUs, each slice a result of its own, summed afterwards in
 // FP64 (launch_sum_chunks).  One slice where half the CUs have a tile
@@ -88,6 +100,64 @@ inline int64_t x4m_slices(int64_t M, int64_t N, int64_t K, int64_t batch, int va
     if (variant > 1 || tiles > 128 || kt < 16) return 1;
     const int64_t want = 256 / tiles < kt / 8 ? 256 / tiles : kt / 8;
     return ceil_div(kt, ceil_div(kt, want)); // no slice empty
+}
+
+// The tile form of an FP32 product on the BF16 matrix cores, and its time in
+// us.  A CU that gets `per_cu` tiles (the fullest) runs them `occ` at a time;
+// a stage of `kt` k takes `alone` us while they wait on latency and `full` us
+// of matrix-core time per tile, and a tile costs `out` us beside its stages
+// (prologue and stores).  Measured on shapes with one tile per CU and with
+// many (predicted / measured us: 1024^3 62, 53, 56 / 65, 54, 55 for the 64x64,
+// 64x32 and 32x32 tiles; 2048^3 337, 353 / 336, 369 for 128x128 and 64x64;
+// 256x65536x256 175, 192 / 178, 193 for 256x128 and 128x128); the choices it
+// makes are within 6% of the best of eleven forms timed on 19 shapes from 64^3 to
+// 4096x4096x1024.
+struct TileForm {
+    int bm, bn, kt, occ;
+    float alone, full, out;
+};
+constexpr TileForm kF32x6Forms[] = {{256, 128, 16, 1, 3.9f, 4.85f, 10.f},
+                                    {128, 128, 16, 1, 2.4f, 2.63f, 6.f},
+                                    {64, 64, 16, 3, 0.92f, 0.69f, 1.f},
+                                    {64, 32, 32, 2, 1.05f, 0.77f, 0.6f},
+                                    {32, 32, 64, 2, 1.1f, 0.8f, 0.4f}};
+inline double f32x6_time(int64_t M, int64_t N, int64_t K, int64_t batch, int *form)
+{
+    constexpr int64_t kCus = 256;
+    double best = -1.0;
+    for (int i = 0; i < int(sizeof(kF32x6Forms) / sizeof(kF32x6Forms[0])); i++) {
+        const TileForm &f = kF32x6Forms[i];
+        const int64_t per_cu = ceil_div(ceil_div(M, f.bm) * ceil_div(N, f.bn) * batch, kCus);
+        const double wait = f.alone * double(ceil_div(per_cu, f.occ)), work = f.full * double(per_cu);
+        const double us = double(ceil_div(K, f.kt)) * (wait > work ? wait : work) +
+                          f.out * double(per_cu);
+        if (best < 0.0 || us < best) {
+            best = us;
+            if (form) *form = i;
+        }
+    }
+    return best;
+}
+
+// Its slices of k (multiples of 64) where a few tiles would walk a long k
+// alone; their results are summed in FP64 (launch_sum_chunks: a launch, and the
+// results read back at 3 TB/s).  time: with the sum.
+inline int f32x6_slices(int64_t M, int64_t N, int64_t K, int64_t batch, double *time)
+{
+    int best = 1;
+    double best_us = f32x6_time(M, N, K, batch, nullptr);
+    for (int s = 2; s <= 64 && K / s >= 128; s *= 2) {
+        const int64_t k = ceil_div(ceil_div(K, s), 64) * 64;
+        if (ceil_div(K, k) != s) continue;
+        const double us = f32x6_time(M, N, k, batch * s, nullptr) + 4.0 +
+                          double(s) * double(batch) * double(M) * double(N) * 8.0 / 3e6;
+        if (us < 0.9 * best_us) {
+            best_us = us;
+            best = s;
+        }
+    }
+    if (time) *time = best_us;
+    return best;
 }
 
 // Rows and k of the split-BF16 operand planes are padded to these multiples.
@@ -121,14 +191,13 @@ struct SplitGather {
 // sits at bit pos[i] of the element offset in the operand (row-major, every
 // extent a power of two, so the modes' digits occupy disjoint bit ranges).
 constexpr int kFusedMaxBits = 24;  // bits per group
-constexpr int kFusedMaxLog2K = 12; // k offset tables in LDS (2 x 4 KiB entries)
+constexpr int kFusedMaxLog2K = 12; // two words of fields (GroupBlock)
 struct FusedBits {
     int n = 0;
     int8_t pos[kFusedMaxBits] = {};
 };
 struct FusedSmall {
     int lb = 0, lm = 0, ln = 0, lk = 0; // log2 of batch, M, N, K
-    int red = 0; // 1: one work-group per output, k split over its threads
     FusedBits a_b, a_m, a_k, b_b, b_n, b_k, c_b, c_m, c_n;
 };
 
@@ -142,14 +211,26 @@ struct FusedSmall {
 constexpr int kGroupMaxLog2K = 10;
 constexpr int kGroupMaxLog2Outputs = 14; // results kept apart from the arena's reuse
 constexpr int kGroupMaxLog2Work = 20;    // outputs * K
+constexpr int kSmallMaxLog2Outputs = 24; // four words of fields
 struct GroupBlock {
     int32_t a = 0, b = 0, c = 0;
     int32_t first = 0, lanes = 0;
     int32_t lo = 0, lk = 0; // log2 of outputs and K
     uint32_t mask_a = 0, mask_b = 0;
-    uint32_t oa[3] = {}, ob[3] = {}, oc[3] = {};
+    uint32_t oa[4] = {}, ob[4] = {}, oc[4] = {};
     uint32_t ka[2] = {}, kb[2] = {};
 };
+// The record of a fused small contraction (lb + lm + ln <=
+// kSmallMaxLog2Outputs); lanes, first and the slots are the caller's.
+GroupBlock group_record(const FusedSmall &f);
+// Lanes per output, at most `most` (log2): while each keeps four k and the
+// contraction stays within 2^log2_threads threads.
+inline int group_lanes(const GroupBlock &g, int most, int log2_threads)
+{
+    int lanes = 0;
+    while (lanes < most && g.lk - lanes > 2 && g.lo + lanes < log2_threads) lanes++;
+    return lanes;
+}
 
 // Split-BF16 operand: planes re hi/lo, im hi/lo[, re+im hi/lo].
 //  * planar (3M kernel, six planes): plane p is [batch][rows_p][k_p] bf16 at
@@ -191,9 +272,7 @@ int choose_gemm_kernel(int mode, int64_t M, int64_t N, int64_t K,
 // kGemmSplitK.
 void launch_gemm(int kernel, int elem_bytes, const GemmArgs &g,
                  hipStream_t stream, void *partials = nullptr);
-// The FP32 products on the BF16 matrix cores (gemm_f32x6.hip), where they
-// apply to the operands.
-bool f32x6_applies(const GemmArgs &g);
+// The FP32 products on the BF16 matrix cores (gemm_f32x6.hip).
 void launch_f32x6(const GemmArgs &g, hipStream_t stream);
 // src: complex64 [batch][rows][k] with row stride ld and batch stride s.
 void launch_split_bf16(const void *src, int64_t rows, int64_t k, int64_t ld,
@@ -226,7 +305,7 @@ void launch_gemm_bf16x3(const SplitOperand &a, const SplitOperand &b, int64_t K_
                         void *C, int64_t M, int64_t N, int64_t ldc,
                         int64_t sC, int64_t batch, bool a_bcast, bool b_bcast,
                         hipStream_t stream);
-// C = contract(A, B) through FusedSmall offsets, one thread per output.
+// C = contract(A, B) through FusedSmall offsets.
 void launch_fused_small(const FusedSmall &f, int elem_bytes, const void *a, const void *b,
                         void *c, hipStream_t stream);
 #endif

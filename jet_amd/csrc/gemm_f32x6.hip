@@ -110,9 +110,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
     int64_t tm, tn;
     tile_coords(blockIdx.x, (g.M + BM - 1) / BM, (g.N + BN - 1) / BN, tm, tn);
     const int64_t m0 = tm * BM, n0 = tn * BN;
-    const int K = int(g.K);
-    const char *At = static_cast<const char *>(g.A) + (bz * g.sA + m0 * g.lda) * 8;
-    const char *Bt = static_cast<const char *>(g.B) + (bz * g.sB + n0 * g.ldb) * 8;
+    const int64_t k_first = int64_t(blockIdx.y) * g.slice_k; // of this slice
+    const int K = int(g.slices > 1 ? min(g.K - k_first, g.slice_k) : g.K);
+    const char *At = static_cast<const char *>(g.A) + (bz * g.sA + m0 * g.lda + k_first) * 8;
+    const char *Bt = static_cast<const char *>(g.B) + (bz * g.sB + n0 * g.ldb + k_first) * 8;
 
     // One load instruction fills 64 consecutive chunks (or dwords) of a
     // stage; a stage is [k sixteenth][row of A, then of B][8 chunks], the
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
                     }
     }
 
-    float2 *C = static_cast<float2 *>(g.C) + bz * g.sC;
+    float2 *C = static_cast<float2 *>(g.C) + bz * g.sC + int64_t(blockIdx.y) * g.slice_stride;
     bool bad = false;
 #pragma unroll
     for (int fm = 0; fm < FM; fm++)
@@ -352,8 +353,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
         if (row >= g.M || col >= g.N) continue;
         const float2 v = C[row * g.ldc + col];
         if (__builtin_isfinite(v.x) && __builtin_isfinite(v.y)) continue;
-        const float2 *a = static_cast<const float2 *>(g.A) + bz * g.sA + row * g.lda;
-        const float2 *b = static_cast<const float2 *>(g.B) + bz * g.sB + col * g.ldb;
+        const float2 *a = static_cast<const float2 *>(g.A) + bz * g.sA + row * g.lda + k_first;
+        const float2 *b = static_cast<const float2 *>(g.B) + bz * g.sB + col * g.ldb + k_first;
         float sr = 0.f, si = 0.f;
         for (int k = 0; k < K; k++) {
             const float2 x = a[k], y = b[k];
@@ -366,50 +367,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
     }
 }
 
-// The tile form of a product.  A CU that gets `per_cu` tiles (the fullest)
-// runs them `occ` at a time; a stage of `kt` k takes `alone` us while they
-// wait on latency and `full` us of matrix-core time per tile, and a tile costs
-// `out` us beside its stages (prologue and stores).  Measured on shapes with one tile
-// per CU and with many (predicted / measured us: 1024^3 62, 53, 56 / 65, 54,
-// 55 for the 64x64, 64x32 and 32x32 tiles; 2048^3 337, 353 / 336, 369 for
-// 128x128 and 64x64; 256x65536x256 175, 192 / 178, 193 for 256x128 and
-// 128x128); the choices it makes are within 6% of the best of eleven forms
-// timed on 19 shapes from 64^3 to 4096x4096x1024.
-struct TileForm {
-    int bm, bn, kt, occ;
-    float alone, full, out;
-};
-constexpr TileForm kForms[] = {{256, 128, 16, 1, 3.9f, 4.85f, 10.f},
-                               {128, 128, 16, 1, 2.4f, 2.63f, 6.f},
-                               {64, 64, 16, 3, 0.92f, 0.69f, 1.f},
-                               {64, 32, 32, 2, 1.05f, 0.77f, 0.6f},
-                               {32, 32, 64, 2, 1.1f, 0.8f, 0.4f}};
-constexpr int kCus = 256;
-
-int choose_form(const GemmArgs &g)
-{
-    int best = 0;
-    double best_us = -1.0;
-    for (int i = 0; i < int(sizeof(kForms) / sizeof(kForms[0])); i++) {
-        const TileForm &f = kForms[i];
-        const double per_cu = double(
-            ceil_div(ceil_div(g.M, f.bm) * ceil_div(g.N, f.bn) * g.batch, int64_t(kCus)));
-        const double rounds = double(ceil_div(int64_t(per_cu), f.occ));
-        const double us = double(ceil_div(g.K, f.kt)) *
-                              std::max(f.alone * rounds, f.full * per_cu) + f.out * per_cu;
-        if (best_us < 0.0 || us < best_us) {
-            best_us = us;
-            best = i;
-        }
-    }
-    return best;
-}
-
 template <int BM, int BN, int WM, int WN, int WK, int NS, bool DUAL, int DW = 4>
 void launch_tile(const GemmArgs &g, hipStream_t stream)
 {
     JH_REQUIRE(ceil_div(g.M, BM) * ceil_div(g.N, BN) <= 0x7fffffff, "Too many tiles.");
-    dim3 grid((unsigned)(ceil_div(g.M, BM) * ceil_div(g.N, BN)), 1, (unsigned)g.batch);
+    dim3 grid((unsigned)(ceil_div(g.M, BM) * ceil_div(g.N, BN)), (unsigned)g.slices,
+              (unsigned)g.batch);
     hipLaunchKernelGGL((cgemm_f32x6_kernel<BM, BN, WM, WN, WK, NS, DUAL, DW>), grid,
                        dim3(64 * WM * WN * WK), 0, stream, g);
     JH_HIP(hipGetLastError());
@@ -417,21 +380,14 @@ void launch_tile(const GemmArgs &g, hipStream_t stream)
 
 } // namespace
 
-// The lane offsets are 32 bits (row strides to 2^21); 32x32 blocks of which
-// less than half would be outputs, and one or no k step, are left to the FP32 MFMA kernel.
-bool f32x6_applies(const GemmArgs &g)
-{
-    return g.lda <= (int64_t(1) << 21) && g.ldb <= (int64_t(1) << 21) && g.K >= 16 &&
-           g.M >= 16 && g.N >= 16;
-}
-
 void launch_f32x6(const GemmArgs &g, hipStream_t stream)
 {
     const bool aligned = reinterpret_cast<uintptr_t>(g.A) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(g.B) % 16 == 0 && g.K % 2 == 0 &&
                          g.lda % 2 == 0 && g.ldb % 2 == 0 &&
                          (g.batch == 1 || (g.sA % 2 == 0 && g.sB % 2 == 0));
-    const int form = choose_form(g);
+    int form = 0;
+    (void)f32x6_time(g.M, g.N, g.slices > 1 ? g.slice_k : g.K, g.batch * g.slices, &form);
     if (!aligned) { // four times the load instructions: the smaller tiles hide them
         if (form <= 2)
             launch_tile<64, 64, 2, 2, 1, 3, true, 1>(g, stream);

@@ -224,6 +224,11 @@ void run_contraction(const ContractionDesc &d, const void *a, const void *b, voi
         g.sB = d.N * d.K;
         g.sC = d.M * d.N;
         g.variant = d.gemm_variant;
+        if (d.slices > 1) {
+            g.slices = int(d.slices);
+            g.slice_k = ceil_div(ceil_div(d.K, d.slices), int64_t(64)) * 64;
+            g.slice_stride = d.batch * d.M * d.N;
+        }
         launch_gemm(d.gemm_kernel, eb, g, s, ws + d.off_partials);
     }
     if (d.chunks > 1 || d.slices > 1)

@@ -121,40 +121,6 @@ void choose_grouped(NetworkPlan &np, const std::vector<std::vector<int32_t>> &mo
         for (NetworkStep &st : np.steps) st.grouped = false;
 }
 
-// The offsets of a step's record.
-GroupBlock group_record(const FusedSmall &f)
-{
-    GroupBlock g;
-    g.lo = f.lb + f.lm + f.ln;
-    g.lk = f.lk;
-    auto put = [](uint32_t *words, int i, int pos) {
-        words[i / 6] |= uint32_t(pos) << (5 * (i % 6));
-    };
-    for (int i = 0; i < f.ln; i++) {
-        g.mask_b |= 1u << i;
-        put(g.ob, i, f.b_n.pos[i]);
-        put(g.oc, i, f.c_n.pos[i]);
-    }
-    for (int i = 0; i < f.lm; i++) {
-        g.mask_a |= 1u << (f.ln + i);
-        put(g.oa, f.ln + i, f.a_m.pos[i]);
-        put(g.oc, f.ln + i, f.c_m.pos[i]);
-    }
-    for (int i = 0; i < f.lb; i++) {
-        const int j = f.ln + f.lm + i;
-        g.mask_a |= 1u << j;
-        g.mask_b |= 1u << j;
-        put(g.oa, j, f.a_b.pos[i]);
-        put(g.ob, j, f.b_b.pos[i]);
-        put(g.oc, j, f.c_b.pos[i]);
-    }
-    for (int i = 0; i < f.lk; i++) {
-        put(g.ka, i, f.a_k.pos[i]);
-        put(g.kb, i, f.b_k.pos[i]);
-    }
-    return g;
-}
-
 // The launches: the steps that run alone in their order, and before each (and
 // after the last) the small steps that follow from what has run so far, by
 // level.  With `delay` (contraction DAGs, whose recomputed values would
@@ -234,9 +200,7 @@ std::vector<int> plan_launches(NetworkPlan &np, bool delay)
                 g.a = np.slot(st.a);
                 g.b = np.slot(st.b);
                 g.c = st.is_root ? np.n_leaves : np.slot(np.n_leaves + s);
-                // Lanes per output while each keeps four k and the step stays
-                // within 256 blocks.
-                while (g.lanes < 6 && g.lk - g.lanes > 2 && g.lo + g.lanes < 16) g.lanes++;
+                g.lanes = group_lanes(g, 6, 16); // shuffles within a wave; 256 work-groups
                 for (g.first = 0; g.first < 1 << g.lo; g.first += 256 >> g.lanes)
                     np.blocks.push_back(g);
                 l.flops += st.desc.flops;

@@ -51,7 +51,9 @@ def _run(ctx, a, b, B, M, N, K):
     (129, 33, 62, 1), (500, 1030, 94, 1), (65, 63, 256, 40), (700, 900, 30, 1),
     (1100, 1030, 78, 1), (1030, 2050, 34, 1), (2040, 2040, 1022, 1), (4080, 4090, 130, 1),
     (60, 70, 33, 1), (33, 31, 17, 5), (400, 900, 255, 1),
-    (1030, 2050, 51, 1), (15, 70, 64, 1)])
+    (1030, 2050, 51, 1), (15, 70, 64, 1),
+    # slices of k: even, a short last one, odd k, a batch
+    (64, 64, 4096, 1), (40, 70, 4000, 1), (33, 65, 5001, 1), (64, 96, 3000, 3)])
 def test_against_64_bits(ctx, table, M, N, K, B):
     rng = np.random.default_rng(M * N + K)
     a, b = rand_c(rng, B * M * K, np.complex64), rand_c(rng, B * N * K, np.complex64)
