@@ -25,6 +25,7 @@ SOURCES = [
     "permute.hip",
     "gemm.hip",
     "gemm_f32x6.hip",
+    "gemm_f64.hip",
     "misc.hip",
     "stream.hip",
     "profiler.hip",

@@ -3,13 +3,14 @@
 // Three arithmetic modes, all computing C[b][m][n] = sum_k A[b][m][k] B[b][n][k]
 // (no conjugation, alpha = 1, beta = 0):
 //
-//  * FP32 / FP64 "4M" (cgemm_embed_kernel): the complex product is the real
+//  * FP32 "4M" (cgemm_embed_kernel; products too short or narrow for
+//    gemm_f32x6.hip): the complex product is the real
 //    product of A viewed as an M x 2K real matrix (re/im interleaved along k)
 //    and the 2K x 2N real matrix B' with B'[2k][2n]=br, B'[2k][2n+1]=bi,
 //    B'[2k+1][2n]=-bi, B'[2k+1][2n+1]=br.  Its output is C with re/im
 //    interleaved, so A and C are used in their native layout and B' is formed
-//    in registers.  v_mfma_{f32,f64}_16x16x4 each cover 16 rows x 8 complex
-//    columns x 2 complex k.
+//    in registers.  v_mfma_f32_16x16x4 covers 16 rows x 8 complex columns x 2
+//    complex k.
 //
 //  * split-BF16 "3M" (cgemm_bf16x3_kernel): T1 = Ar.Br, T2 = Ai.Bi,
 //    T3 = (Ar+Ai).(Br+Bi), Cr = T1 - T2, Ci = T3 - T1 - T2, where every real
@@ -31,15 +32,13 @@ namespace jet_hip {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 template <class R> struct Vec;
 // Output row of accumulator item r held by lane group q (= lane / 16) in a
-// 16x16x4 MFMA block: v_mfma_f32_16x16x4_f32 returns D[4q + r][lane % 16],
-// v_mfma_f64_16x16x4_f64 returns D[q + 4r][lane % 16] (both measured on
-// gfx950).
+// 16x16x4 MFMA block: v_mfma_f32_16x16x4_f32 returns D[4q + r][lane % 16]
+// (measured on gfx950).
 template <> struct Vec<float> {
     using c = float2;
     using acc = f32x4;
@@ -47,21 +46,15 @@ template <> struct Vec<float> {
 };
 template <> struct Vec<double> {
     using c = double2;
-    using acc = f64x4;
-    static __device__ __forceinline__ int row(int q, int r) { return q + 4 * r; }
 };
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f64x4 mfma4(double a, double b, f64x4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
 
 // ---------------------------------------------------------------------------
-// 4M complex GEMM on FP32 / FP64 MFMA.
+// 4M complex GEMM on FP32 MFMA.
 // Block tile BM x BN complex outputs, BK complex k per LDS stage, 4 waves in
 // a WM x WN grid, double-buffered LDS with register prefetch.
 // Lane l of a 16x16x4 MFMA holds A[l%16][l/16] and B[l/16][l%16] and gets
@@ -1909,12 +1902,9 @@ void launch_gemm(int kernel, int elem_bytes, const GemmArgs &g,
     }
     else if (kernel == kGemmF64Mfma) {
         JH_REQUIRE(elem_bytes == 16, "FP64 MFMA kernel needs complex128 data.");
-        constexpr int BM = 128, BN = 64;
-        JH_REQUIRE(ceil_div(g.M, BM) * ceil_div(g.N, BN) <= 0x7fffffff, "Too many tiles.");
-        dim3 grid((unsigned)(ceil_div(g.M, BM) * ceil_div(g.N, BN)), 1, (unsigned)g.batch);
         prof::Scope ps(prof::kGemmF64, stream, gemm_flops(g), gemm_bytes(g, 16));
-        hipLaunchKernelGGL((cgemm_embed_kernel<double, BM, BN, 8, 2, 2>), grid, dim3(256), 0,
-                           stream, g);
+        launch_f64(g, stream);
+        return;
     }
     else {
         JH_FAIL(JET_HIP_ERROR_INTERNAL, "launch_gemm: unknown kernel.");

@@ -22,8 +22,8 @@ struct GemmArgs {
     int64_t lda, ldb, ldc; // row strides in elements
     int64_t sA, sB, sC;    // batch strides in elements (0 = broadcast)
     int variant = 0;       // tile / thread-mapping variant (GemmChoice)
-    // FP32 products on the BF16 matrix cores: slices of slice_k k each write a
-    // result of their own, slice_stride elements apart (f32x6_slices).
+    // FP32 and FP64 matrix-core products: slices of slice_k k each write a
+    // result of their own, slice_stride elements apart (tile_slices).
     int slices = 1;
     int64_t slice_k = 0, slice_stride = 0;
 };
@@ -36,7 +36,7 @@ enum GemmKernel {
                         // each value and six products (gemm_f32x6.hip), or 4M
                         // complex on v_mfma_f32_16x16x4_f32 where that does
                         // not apply (k, M or N < 16)
-    kGemmF64Mfma = 3,   // 4M complex on v_mfma_f64_16x16x4_f64
+    kGemmF64Mfma = 3,   // 4M complex on v_mfma_f64_16x16x4_f64 (gemm_f64.hip)
     kGemmBf16x3 = 4,    // 3M complex, split-BF16, v_mfma_f32_16x16x32_bf16
     kGemmBf16x4m = 5,   // 4M complex, split-BF16, v_mfma_f32_16x16x32_bf16
     kGemmSplitK = 6,    // VALU, few outputs and long k: k split over blocks,
@@ -49,7 +49,7 @@ enum GemmKernel {
 // lets the launcher pick by shape; the others force one form:
 //   kGemmF32Mfma              1: 128x128  2: 64x128  3: 128x64 block tiles of
 //                             the FP32 MFMA kernel
-//   kGemmF64Mfma              1: 128x64 block tiles
+//   kGemmF64Mfma              1: its tile forms by shape
 //   kGemmBf16x4m, kGemmF16x4m 1: 128x128  2: 128x192 block tiles
 //                             3: 128x128 persistent (one work-group per
 //                             CU walking the tiles)
@@ -102,16 +102,18 @@ inline int64_t x4m_slices(int64_t M, int64_t N, int64_t K, int64_t batch, int va
     return ceil_div(kt, ceil_div(kt, want)); // no slice empty
 }
 
-// The tile form of an FP32 product on the BF16 matrix cores, and its time in
-// us.  A CU that gets `per_cu` tiles (the fullest) runs them `occ` at a time;
-// a stage of `kt` k takes `alone` us while they wait on latency and `full` us
-// of matrix-core time per tile, and a tile costs `out` us beside its stages
-// (prologue and stores).  Measured on shapes with one tile per CU and with
-// many (predicted / measured us: 1024^3 62, 53, 56 / 65, 54, 55 for the 64x64,
-// 64x32 and 32x32 tiles; 2048^3 337, 353 / 336, 369 for 128x128 and 64x64;
-// 256x65536x256 175, 192 / 178, 193 for 256x128 and 128x128); the choices it
-// makes are within 6% of the best of eleven forms timed on 19 shapes from 64^3 to
-// 4096x4096x1024.
+// A tile form of the FP32 (gemm_f32x6.hip) or FP64 (gemm_f64.hip) matrix-core
+// products, and the time in us that a product takes with it.  A CU that gets
+// `per_cu` tiles (the fullest) runs them `occ` at a time; a stage of `kt` k
+// takes `alone` us while they wait on latency and `full` us of matrix-core
+// time per tile, and a tile costs `out` us beside its stages (prologue and
+// stores).  Measured on shapes with one tile per CU and with many; FP32,
+// predicted / measured us: 1024^3 62, 53, 56 / 65, 54, 55 for the 64x64, 64x32
+// and 32x32 tiles, 2048^3 337, 353 / 336, 369 for 128x128 and 64x64,
+// 256x65536x256 175, 192 / 178, 193 for 256x128 and 128x128; FP64: 1024^3 137,
+// 137 / 144, 148 for 32x32 with and without slices in the tile, 1536x1536x512
+// 158, 252 / 160, 256 for 32x32 and 128x128.  The FP32 choices are within 6% of
+// the best of eleven forms timed on 19 shapes from 64^3 to 4096x4096x1024.
 struct TileForm {
     int bm, bn, kt, occ;
     float alone, full, out;
@@ -121,12 +123,17 @@ constexpr TileForm kF32x6Forms[] = {{256, 128, 16, 1, 3.9f, 4.85f, 10.f},
                                     {64, 64, 16, 3, 0.92f, 0.69f, 1.f},
                                     {64, 32, 32, 2, 1.05f, 0.77f, 0.6f},
                                     {32, 32, 64, 2, 1.1f, 0.8f, 0.4f}};
-inline double f32x6_time(int64_t M, int64_t N, int64_t K, int64_t batch, int *form)
+constexpr TileForm kF64Forms[] = {{128, 128, 8, 1, 3.8f, 3.92f, 9.f},
+                                  {32, 32, 16, 3, 0.70f, 0.523f, 0.83f},
+                                  {32, 32, 8, 6, 0.445f, 0.264f, 0.39f}};
+template <int COUNT>
+inline double tile_time(const TileForm (&forms)[COUNT], int64_t M, int64_t N, int64_t K,
+                        int64_t batch, int *form)
 {
     constexpr int64_t kCus = 256;
     double best = -1.0;
-    for (int i = 0; i < int(sizeof(kF32x6Forms) / sizeof(kF32x6Forms[0])); i++) {
-        const TileForm &f = kF32x6Forms[i];
+    for (int i = 0; i < COUNT; i++) {
+        const TileForm &f = forms[i];
         const int64_t per_cu = ceil_div(ceil_div(M, f.bm) * ceil_div(N, f.bn) * batch, kCus);
         const double wait = f.alone * double(ceil_div(per_cu, f.occ)), work = f.full * double(per_cu);
         const double us = double(ceil_div(K, f.kt)) * (wait > work ? wait : work) +
@@ -139,18 +146,20 @@ inline double f32x6_time(int64_t M, int64_t N, int64_t K, int64_t batch, int *fo
     return best;
 }
 
-// Its slices of k (multiples of 64) where a few tiles would walk a long k
-// alone; their results are summed in FP64 (launch_sum_chunks: a launch, and the
+// Slices of k (multiples of 64) where a few tiles would walk a long k alone;
+// their results are summed in FP64 (launch_sum_chunks: a launch, and the
 // results read back at 3 TB/s).  time: with the sum.
-inline int f32x6_slices(int64_t M, int64_t N, int64_t K, int64_t batch, double *time)
+template <int COUNT>
+inline int tile_slices(const TileForm (&forms)[COUNT], int elem_bytes, int64_t M, int64_t N,
+                       int64_t K, int64_t batch, double *time)
 {
     int best = 1;
-    double best_us = f32x6_time(M, N, K, batch, nullptr);
+    double best_us = tile_time(forms, M, N, K, batch, nullptr);
     for (int s = 2; s <= 64 && K / s >= 128; s *= 2) {
         const int64_t k = ceil_div(ceil_div(K, s), 64) * 64;
         if (ceil_div(K, k) != s) continue;
-        const double us = f32x6_time(M, N, k, batch * s, nullptr) + 4.0 +
-                          double(s) * double(batch) * double(M) * double(N) * 8.0 / 3e6;
+        const double us = tile_time(forms, M, N, k, batch * s, nullptr) + 4.0 +
+                          double(s) * double(batch) * double(M) * double(N) * elem_bytes / 3e6;
         if (us < 0.9 * best_us) {
             best_us = us;
             best = s;
@@ -274,6 +283,8 @@ void launch_gemm(int kernel, int elem_bytes, const GemmArgs &g,
                  hipStream_t stream, void *partials = nullptr);
 // The FP32 products on the BF16 matrix cores (gemm_f32x6.hip).
 void launch_f32x6(const GemmArgs &g, hipStream_t stream);
+// complex128 products (gemm_f64.hip).
+void launch_f64(const GemmArgs &g, hipStream_t stream);
 // src: complex64 [batch][rows][k] with row stride ld and batch stride s.
 void launch_split_bf16(const void *src, int64_t rows, int64_t k, int64_t ld,
                        int64_t s, int64_t batch, const SplitOperand &dst,

@@ -387,7 +387,8 @@ void launch_f32x6(const GemmArgs &g, hipStream_t stream)
                          g.lda % 2 == 0 && g.ldb % 2 == 0 &&
                          (g.batch == 1 || (g.sA % 2 == 0 && g.sB % 2 == 0));
     int form = 0;
-    (void)f32x6_time(g.M, g.N, g.slices > 1 ? g.slice_k : g.K, g.batch * g.slices, &form);
+    (void)tile_time(kF32x6Forms, g.M, g.N, g.slices > 1 ? g.slice_k : g.K, g.batch * g.slices,
+                    &form);
     if (!aligned) { // four times the load instructions: the smaller tiles hide them
         if (form <= 2)
             launch_tile<64, 64, 2, 2, 1, 3, true, 1>(g, stream);
