@@ -6,7 +6,8 @@
 // permutation is a permutation of the bits of the linear index, and the
 // LDS-tiled bit kernel moves tiles made of the lowest input bits and the
 // lowest output bits, so that both the reads and the writes are contiguous
-// runs.  Other shapes use a gather kernel (coalesced writes).
+// runs.  Other shapes go by tiles of whole axes where such tiles have runs on
+// both sides, or use a gather kernel (coalesced writes).
 //
 // Pure C++: the index helpers below are shared by the kernels and by the CPU
 // emulation that checks plans and bounds before anything runs on a GPU.
@@ -40,11 +41,35 @@ struct GenericPermParams {
     int64_t in_stride[kMaxRank]; // input stride of output axis i
 };
 
+// A generic permutation by tiles: a tile is every value of a few axes, the
+// trailing ones of the input and of the output (axes longer than 64 are split
+// at a divisor first), so that reads and writes are runs; LDS turns one order
+// into the other.
+constexpr int kTileAxes = 8, kOuterAxes = 12;
+constexpr int kTileBytes = 32768;
+// Beyond these a permutation runs out of HBM (last-level cache 256 MiB).
+constexpr int kPermCacheBits = 25;
+constexpr int64_t kPermCacheBytes = int64_t(1) << 28;
+struct TilePermParams {
+    int elems = 0; // of a tile; 0: no tiling
+    int cap = 0;   // 1024, 2048 or 4096: the smallest with runs on both sides
+    uint32_t tiles = 0;
+    // Tile axes from the fastest, in input order and in output order: extent,
+    // reciprocal (2^20 / extent, rounded up: exact below 2^12 for extents to
+    // 128), offset per step in the input or output, and for the output order
+    // the step in the input-order tile.  Unused axes have extent 1.
+    uint32_t in_ext[kTileAxes], in_rec[kTileAxes], in_step[kTileAxes];
+    uint32_t out_ext[kTileAxes], out_rec[kTileAxes], out_step[kTileAxes], out_u[kTileAxes];
+    int n_outer = 0; // other axes, fastest (of the output) first
+    uint32_t outer_ext[kOuterAxes], outer_in[kOuterAxes], outer_out[kOuterAxes];
+};
+
 struct PermutePlan {
     enum Kind { kCopy, kBits, kGeneric } kind = kCopy;
     int64_t numel = 0;
     BitPermParams bits{};
     GenericPermParams gen{};
+    TilePermParams tiles8, tiles16; // kGeneric, for 8- and 16-byte elements
 };
 
 // Build a plan; extents are the input's (row-major), perm[i] = input axis of
@@ -106,6 +131,48 @@ JH_HD int bits_lds_index(int u, int elem_bytes)
     const int s = elem_bytes == 8 ? 5 : 4;
     return u ^ ((u >> s) & ((1 << s) - 1));
 }
+
+// Offset of element u of a tile (axes from the fastest; `other`: a second sum
+// of steps).
+JH_HD uint32_t tile_axes_offset(const uint32_t (&ext)[kTileAxes], const uint32_t (&rec)[kTileAxes],
+                                const uint32_t (&step)[kTileAxes],
+                                const uint32_t (&other)[kTileAxes], uint32_t u, uint32_t *second)
+{
+    uint32_t o = 0, s = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+    for (int i = 0; i < kTileAxes; i++) {
+        const uint32_t q = (u * rec[i]) >> 20, c = u - q * ext[i];
+        o += c * step[i];
+        s += c * other[i];
+        u = q;
+    }
+    *second = s;
+    return o;
+}
+
+// Input and output offsets of tile w.
+JH_HD void tile_axes_base(const TilePermParams &p, uint32_t w, uint32_t *in, uint32_t *out)
+{
+    uint32_t a = 0, b = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+    for (int i = 0; i < kOuterAxes; i++) {
+        if (i < p.n_outer) {
+            const uint32_t q = w / p.outer_ext[i], c = w - q * p.outer_ext[i];
+            a += c * p.outer_in[i];
+            b += c * p.outer_out[i];
+            w = q;
+        }
+    }
+    *in = a;
+    *out = b;
+}
+
+// LDS slot of tile element u: one slot of padding per 32.
+JH_HD uint32_t tile_axes_slot(uint32_t u) { return u + (u >> 5); }
 
 // Input offset of output element o for the gather kernel.
 JH_HD int64_t generic_in_offset(const GenericPermParams &p, int64_t o)
