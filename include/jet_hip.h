@@ -105,6 +105,11 @@ int jet_hip_ctx_stream(jet_hip_ctx_t ctx, void **stream);
  * buffer must be synchronized first. */
 int jet_hip_malloc(jet_hip_ctx_t ctx, size_t bytes, void **ptr);
 int jet_hip_free(jet_hip_ctx_t ctx, void *ptr);
+/* The same for work on the context stream alone: small buffers come without a
+ * synchronization, from blocks of the context whose earlier use that stream
+ * may not have finished (other streams wait for it first).  Freed with the same
+ * context. */
+int jet_hip_malloc_ordered(jet_hip_ctx_t ctx, size_t bytes, void **ptr);
 /* kind: 0 host->device, 1 device->host, 2 device->device.  Synchronous when
  * stream is NULL and async == 0. */
 int jet_hip_memcpy(jet_hip_ctx_t ctx, void *dst, const void *src, size_t bytes,

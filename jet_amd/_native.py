@@ -32,7 +32,8 @@ GEMM_KERNEL_NAMES = {0: "valu", 1: "valu_reduce", 2: "fp32_mfma", 3: "fp64_mfma"
 # Exported symbols (must match include/jet_hip.h).
 EXPORTS = [
     "jet_hip_get_version", "jet_hip_last_error", "jet_hip_ctx_create", "jet_hip_ctx_destroy",
-    "jet_hip_ctx_device", "jet_hip_ctx_stream", "jet_hip_malloc", "jet_hip_free",
+    "jet_hip_ctx_device", "jet_hip_ctx_stream", "jet_hip_malloc", "jet_hip_malloc_ordered",
+    "jet_hip_free",
     "jet_hip_memcpy", "jet_hip_memset", "jet_hip_stream_synchronize",
     "jet_hip_device_synchronize", "jet_hip_permute", "jet_hip_contraction_plan_create",
     "jet_hip_plan_workspace_size", "jet_hip_plan_info", "jet_hip_plan_destroy",
@@ -75,6 +76,7 @@ def _declare(L):
         "jet_hip_ctx_device": [_vp, ctypes.POINTER(ctypes.c_int)],
         "jet_hip_ctx_stream": [_vp, ctypes.POINTER(_vp)],
         "jet_hip_malloc": [_vp, ctypes.c_size_t, ctypes.POINTER(_vp)],
+        "jet_hip_malloc_ordered": [_vp, ctypes.c_size_t, ctypes.POINTER(_vp)],
         "jet_hip_free": [_vp, _vp],
         "jet_hip_memcpy": [_vp, _vp, _vp, ctypes.c_size_t, ctypes.c_int, _vp, ctypes.c_int],
         "jet_hip_memset": [_vp, _vp, ctypes.c_int, ctypes.c_size_t, _vp],
@@ -226,13 +228,15 @@ def default_context() -> Context:
 
 
 class DeviceBuffer:
-    """Owning device allocation."""
+    """Owning device allocation.  ``ordered``: for work on the context's
+    stream alone (no wait; other streams wait for that one first)."""
 
-    def __init__(self, nbytes: int, ctx: Optional[Context] = None):
+    def __init__(self, nbytes: int, ctx: Optional[Context] = None, ordered: bool = False):
         self.ctx = ctx or default_context()
         self.nbytes = int(nbytes)
         p = _vp()
-        check(lib().jet_hip_malloc(self.ctx.handle, self.nbytes, ctypes.byref(p)))
+        alloc = lib().jet_hip_malloc_ordered if ordered else lib().jet_hip_malloc
+        check(alloc(self.ctx.handle, self.nbytes, ctypes.byref(p)))
         self.ptr = p.value
 
     def upload(self, host, stream=None) -> None:

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <new>
 #include <string>
@@ -20,9 +21,74 @@
 
 using namespace jet_hip;
 
+// Small device buffers of one stream, cut from slabs of equal blocks: a block
+// given back is handed out again at once, as both uses are ordered by the
+// stream.  At most kSlabs MiB stay here; slabs without a block in use go
+// back when memory runs out and with the context.  Measured on an
+// amplitude of 207 small contractions: 5.5 ms with a pool allocation and a wait
+// for each, 10.9 in a loop of them without the wait (the pool reuses a block only
+// once the stream has passed its release), 3.3 with these blocks.
+class SmallBuffers {
+public:
+    static constexpr size_t kSlabBytes = size_t(1) << 20, kMaxBlock = size_t(1) << 16;
+    static constexpr size_t kSlabs = 32;
+
+    // A block of `bytes` or more; `slab()` gets a new slab where no block is left.
+    template <class NewSlab> void *take(size_t bytes, const NewSlab &slab)
+    {
+        size_t block = 256;
+        while (block < bytes) block *= 2;
+        std::lock_guard<std::recursive_mutex> lock(mutex_);
+        auto it = slabs_.begin();
+        while (it != slabs_.end() && (it->second.block != block || it->second.unused.empty())) ++it;
+        if (it == slabs_.end()) {
+            if (slabs_.size() == kSlabs) return nullptr;
+            char *base = static_cast<char *>(slab());
+            it = slabs_.emplace(base, Slab{block, {}}).first;
+            it->second.unused.reserve(kSlabBytes / block);
+            for (size_t o = kSlabBytes; o > 0; o -= block)
+                it->second.unused.push_back(base + o - block);
+        }
+        void *p = it->second.unused.back();
+        it->second.unused.pop_back();
+        return p;
+    }
+    // Takes a block back; false for other memory.
+    bool give(void *ptr)
+    {
+        char *p = static_cast<char *>(ptr);
+        std::lock_guard<std::recursive_mutex> lock(mutex_);
+        auto it = slabs_.upper_bound(p);
+        if (it == slabs_.begin() || p >= (--it)->first + kSlabBytes) return false;
+        it->second.unused.push_back(p);
+        return true;
+    }
+    template <class Free> void trim(const Free &free)
+    {
+        std::lock_guard<std::recursive_mutex> lock(mutex_);
+        for (auto it = slabs_.begin(); it != slabs_.end();) {
+            if (it->second.unused.size() == kSlabBytes / it->second.block) {
+                free(it->first);
+                it = slabs_.erase(it);
+            }
+            else
+                ++it;
+        }
+    }
+
+private:
+    struct Slab {
+        size_t block;
+        std::vector<char *> unused;
+    };
+    std::recursive_mutex mutex_; // a new slab may trim the others
+    std::map<char *, Slab> slabs_;
+};
+
 struct jet_hip_ctx_s {
     int device = 0;
     hipStream_t stream = nullptr;
+    SmallBuffers small;
 };
 
 struct jet_hip_plan_s {
@@ -287,6 +353,29 @@ void *device_alloc(size_t bytes, int device)
     return p;
 }
 
+// Stream-ordered pool allocation on the context stream, made visible to every
+// stream before returning.  The pool keeps freed blocks cached; when a
+// request does not fit, the cache is released to the device and the request
+// made once more.
+void *pool_alloc(jet_hip_ctx_s *ctx, size_t bytes)
+{
+    void *p = nullptr;
+    hipError_t e = hipMallocAsync(&p, bytes, ctx->stream);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        JH_HIP(hipDeviceSynchronize());
+        ctx->small.trim([&](void *slab) { (void)hipFreeAsync(slab, ctx->stream); });
+        JH_HIP(hipDeviceSynchronize());
+        hipMemPool_t pool;
+        JH_HIP(hipDeviceGetDefaultMemPool(&pool, ctx->device));
+        JH_HIP(hipMemPoolTrimTo(pool, 0));
+        e = hipMallocAsync(&p, bytes, ctx->stream);
+    }
+    JH_HIP(e);
+    JH_HIP(hipStreamSynchronize(ctx->stream));
+    return p;
+}
+
 void free_memory(jet_hip_network_s *net)
 {
     if (net->arena) (void)hipFree(net->arena);
@@ -410,6 +499,7 @@ int jet_hip_ctx_destroy(jet_hip_ctx_t ctx)
     return guarded([&] {
         if (!ctx) return;
         set_device(ctx);
+        ctx->small.trim([&](void *slab) { (void)hipFreeAsync(slab, ctx->stream); });
         JH_HIP(hipStreamSynchronize(ctx->stream));
         JH_HIP(hipStreamDestroy(ctx->stream));
         delete ctx;
@@ -438,22 +528,22 @@ int jet_hip_malloc(jet_hip_ctx_t ctx, size_t bytes, void **ptr)
         set_device(ctx);
         JH_REQUIRE(ptr != nullptr, "Null output pointer.");
         *ptr = nullptr;
-        if (bytes == 0) bytes = 1;
-        // Stream-ordered pool allocation on the context stream, made visible
-        // to every stream before returning.  The pool keeps freed blocks
-        // cached; when a request does not fit, the cache is released to the
-        // device and the request made once more.
-        hipError_t e = hipMallocAsync(ptr, bytes, ctx->stream);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            JH_HIP(hipDeviceSynchronize());
-            hipMemPool_t pool;
-            JH_HIP(hipDeviceGetDefaultMemPool(&pool, ctx->device));
-            JH_HIP(hipMemPoolTrimTo(pool, 0));
-            e = hipMallocAsync(ptr, bytes, ctx->stream);
-        }
-        JH_HIP(e);
-        JH_HIP(hipStreamSynchronize(ctx->stream));
+        *ptr = pool_alloc(ctx, std::max<size_t>(bytes, 1));
+    });
+}
+
+int jet_hip_malloc_ordered(jet_hip_ctx_t ctx, size_t bytes, void **ptr)
+{
+    return guarded([&] {
+        set_device(ctx);
+        JH_REQUIRE(ptr != nullptr, "Null output pointer.");
+        *ptr = nullptr;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (bytes <= SmallBuffers::kMaxBlock) JH_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+        if (bytes <= SmallBuffers::kMaxBlock && capture == hipStreamCaptureStatusNone)
+            *ptr = ctx->small.take(bytes,
+                                   [&] { return pool_alloc(ctx, SmallBuffers::kSlabBytes); });
+        if (!*ptr) *ptr = pool_alloc(ctx, std::max<size_t>(bytes, 1));
     });
 }
 
@@ -463,7 +553,7 @@ int jet_hip_free(jet_hip_ctx_t ctx, void *ptr)
         set_device(ctx);
         // Ordered after all work queued on the context stream; callers that
         // used other streams synchronize them first.
-        if (ptr) JH_HIP(hipFreeAsync(ptr, ctx->stream));
+        if (ptr && !ctx->small.give(ptr)) JH_HIP(hipFreeAsync(ptr, ctx->stream));
     });
 }
 

@@ -272,19 +272,30 @@ class AdjointProgram:
         self.dtype = self.dag.dtype
         self._one = nat.DeviceBuffer(16, self.ctx)
         self._one.upload(np.ones(1, self.dtype))
+        # Where the kept region holds the root value and, in each leaf's label
+        # order, the environments.
+        self._root_at = self._region_index(self.root_node, []).item()
+        self._env_at = {w: self._region_index(self.env_node[w], self.leaf_labels[w])
+                        for w in self.wanted}
 
-    def run(self, leaf_ptrs: Sequence[int]):
-        """(root value, {leaf: environment in the leaf's label order})."""
+    def _region_index(self, node: int, order: Sequence[str]) -> np.ndarray:
+        ptr, labels, shape = self.dag.values[node]
+        at = np.arange(max(1, int(np.prod(shape)))).reshape(shape)
+        at = at.transpose([labels.index(l) for l in order]) if order else at
+        return at + (ptr - self.dag._region[0]) // self.dtype.itemsize
+
+    def run_region(self, leaf_ptrs: Sequence[int]) -> np.ndarray:
+        """The kept region after one execution."""
         if len(leaf_ptrs) != self.n:
             raise JetError("Wrong number of leaf tensors.")
         self.dag.launch(list(leaf_ptrs) + [self._one.ptr])
-        vals = self.dag.kept_values()
-        root = complex(vals[self.root_node][1].reshape(-1)[0])
-        envs = {}
-        for w in self.wanted:
-            labels, data = vals[self.env_node[w]]
-            want = self.leaf_labels[w]
-            envs[w] = np.transpose(data, [labels.index(l) for l in want]) if want else data
+        return self.dag.kept_region()
+
+    def run(self, leaf_ptrs: Sequence[int]):
+        """(root value, {leaf: environment in the leaf's label order})."""
+        region = self.run_region(leaf_ptrs)
+        root = complex(region[self._root_at])
+        envs = {w: region[at] for w, at in self._env_at.items()}
         return root, envs
 
 
@@ -325,7 +336,7 @@ class ParameterizedAmplitude:
                 self.theta[g.param_index:g.param_index + 2] = g.params
         self.amplitude: Optional[complex] = None
         self._fp64 = None
-        self._envs: Optional[Dict[int, np.ndarray]] = None
+        self._envs: Optional[np.ndarray] = None  # one row of 16 per fSim gate
         if method == "eager":
             self.leaves = [Tensor(ix, sh, d.astype(self.dtype), dtype=self.dtype, ctx=self.ctx)
                            for ix, sh, d in zip(net.indices, net.shapes, net.data)]
@@ -342,6 +353,8 @@ class ParameterizedAmplitude:
         self._bufs = []
         self._leaf_ptrs = []
         self._param_buf = nat.DeviceBuffer(len(self.param_leaf) * 16 * item, self.ctx)
+        self._env_at = np.stack([self.program._env_at[leaf].reshape(-1)
+                                 for leaf in self.param_leaf])
         pos = {leaf: j for j, leaf in enumerate(self.param_leaf)}
         for i, d in enumerate(net.data):
             if i in is_param:
@@ -354,9 +367,14 @@ class ParameterizedAmplitude:
         self._upload_params()
 
     def _upload_params(self) -> None:
-        gates = np.stack([fsim(self.theta[slot], self.theta[slot + 1]).reshape(-1)
-                          for slot in self.param_slot]).astype(self.dtype)
-        self._param_buf.upload(np.ascontiguousarray(gates.reshape(-1)))
+        slots = np.asarray(self.param_slot)
+        th, ph = self.theta[slots], self.theta[slots + 1]
+        gates = np.zeros((len(slots), 16), np.complex128)  # rows as of fsim()
+        gates[:, 0] = 1
+        gates[:, 5] = gates[:, 10] = np.cos(th)
+        gates[:, 6] = gates[:, 9] = -1j * np.sin(th)
+        gates[:, 15] = np.exp(-1j * ph)
+        self._param_buf.upload(gates.astype(self.dtype).reshape(-1))
 
     def set_angles(self, theta: Sequence[float]) -> None:
         theta = np.asarray(theta, dtype=np.float64).reshape(-1)
@@ -377,7 +395,9 @@ class ParameterizedAmplitude:
         if theta is not None:
             self.set_angles(theta)
         if self.method == "graph":
-            self.amplitude, self._envs = self.program.run(self._leaf_ptrs)
+            region = self.program.run_region(self._leaf_ptrs)
+            self.amplitude = complex(region[self.program._root_at])
+            self._envs = region[self._env_at]
             return self.amplitude
         root = self.adjoint.forward(self.leaves)
         self.amplitude = complex(root.get_data().reshape(-1)[0])
@@ -390,8 +410,7 @@ class ParameterizedAmplitude:
         if self.method == "graph":
             if self._envs is None:
                 raise JetError("Run forward() before amplitude_gradient().")
-            E = np.stack([self._envs[leaf].reshape(-1) for leaf in self.param_leaf]
-                         ).astype(np.complex128)
+            E = self._envs.astype(np.complex128)
         else:
             envs = self.adjoint.environments()
             buf = nat.DeviceBuffer(k * 16 * self.dtype.itemsize, self.ctx)
@@ -404,17 +423,16 @@ class ParameterizedAmplitude:
             host = np.empty(k * 16, self.dtype)
             buf.download(host)
             E = host.astype(np.complex128).reshape(k, 16)
+        slots = np.asarray(self.param_slot)
+        th, ph = self.theta[slots], self.theta[slots + 1]
+        d_th = np.zeros((k, 16), np.complex128)
+        d_th[:, 5] = d_th[:, 10] = -np.sin(th)
+        d_th[:, 6] = d_th[:, 9] = -1j * np.cos(th)
+        d_ph = np.zeros((k, 16), np.complex128)
+        d_ph[:, 15] = -1j * np.exp(-1j * ph)
         grad = np.zeros(self.n_params, dtype=np.complex128)
-        for j, slot in enumerate(self.param_slot):
-            th, ph = self.theta[slot], self.theta[slot + 1]
-            c, s = np.cos(th), np.sin(th)
-            d_th = np.zeros((4, 4), np.complex128)
-            d_th[1, 1] = d_th[2, 2] = -s
-            d_th[1, 2] = d_th[2, 1] = -1j * c
-            d_ph = np.zeros((4, 4), np.complex128)
-            d_ph[3, 3] = -1j * np.exp(-1j * ph)
-            grad[slot] = np.sum(E[j] * d_th.reshape(-1))
-            grad[slot + 1] = np.sum(E[j] * d_ph.reshape(-1))
+        grad[slots] = np.sum(E * d_th, axis=1)
+        grad[slots + 1] = np.sum(E * d_ph, axis=1)
         return grad
 
     def loss_and_gradient(self, theta: Optional[Sequence[float]] = None):

@@ -210,18 +210,21 @@ class DeviceDag:
             self._graph_key = key
         nat.check(nat.lib().jet_hip_network_launch(self.handle, stream))
 
-    def kept_values(self) -> Dict[int, Tuple[List[str], np.ndarray]]:
-        """{node: (labels, row-major data)} of the kept results, read back in
-        one copy of their region."""
+    def kept_region(self) -> np.ndarray:
+        """The region of the kept results, read back in one copy."""
         first, size = self._region
         raw = np.empty(size // self.dtype.itemsize, self.dtype)
         nat.check(nat.lib().jet_hip_memcpy(self.ctx.handle, raw.ctypes.data, first, size, 1,
                                            None, 0))
+        return raw
+
+    def kept_values(self) -> Dict[int, Tuple[List[str], np.ndarray]]:
+        """{node: (labels, row-major data)} of the kept results."""
+        raw = self.kept_region()
+        first = self._region[0]
         out = {}
         for k, (ptr, labels, shape) in self.values.items():
-            o = (ptr - first) // self.dtype.itemsize
-            n = max(1, int(np.prod(shape)))
-            out[k] = (labels, raw[o:o + n].reshape(shape) if shape else raw[o:o + 1].reshape(()))
+            out[k] = (labels, np.ndarray(shape, self.dtype, raw, ptr - first))
         return out
 
     def close(self) -> None:

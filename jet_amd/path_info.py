@@ -11,6 +11,7 @@ indices without an edge (extent 1, or sliced away) count as 1.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -99,10 +100,8 @@ class PathInfo:
     GetIndexSizes = lambda self: dict(self._sizes)  # noqa: E731
 
     def _size(self, labels: Sequence[str]) -> float:
-        out = 1.0
-        for l in labels:
-            out *= self._sizes.get(l, 1)
-        return out
+        size = self._sizes.get
+        return math.prod([size(l, 1) for l in labels], start=1.0)
 
     def GetPathStepFlops(self, step_id: int) -> float:
         """PathInfo.hpp:157-183."""

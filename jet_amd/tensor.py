@@ -42,26 +42,32 @@ def _dtype_code(dtype) -> int:
 
 class _PlanCache:
     """Contraction plans keyed by the relabelled problem (so contractions of
-    the same shapes with different label names share one plan)."""
+    the same shapes with different label names share one plan), each with the
+    context whose stream it runs on."""
 
     def __init__(self):
-        self._plans: Dict[tuple, ctypes.c_void_p] = {}
+        self._plans: Dict[tuple, tuple] = {}
 
     def get(self, ctx, dtype_code, prec, a_modes, a_ext, b_modes, b_ext, c_modes):
         key = (ctx.device, dtype_code, prec, tuple(a_modes), tuple(a_ext), tuple(b_modes),
                tuple(b_ext), tuple(c_modes))
-        p = self._plans.get(key)
-        if p is None:
+        known = self._plans.get(key)
+        if known is None:
             p = ctypes.c_void_p()
             nat.check(nat.lib().jet_hip_contraction_plan_create(
                 ctx.handle, dtype_code, prec, nat.ROW_MAJOR, len(a_modes), nat.i32(a_modes),
                 nat.i64(a_ext), len(b_modes), nat.i32(b_modes), nat.i64(b_ext), len(c_modes),
                 nat.i32(c_modes), ctypes.byref(p)))
-            self._plans[key] = p
-        return p
+            known = self._plans[key] = (p, ctx)
+        return known
 
 
 _plan_cache = _PlanCache()
+
+# ContractTensors by its operands' labels, extents and type: the result's labels,
+# extents and size, and its plan.  Emptied when full.
+_contractions: Dict[tuple, tuple] = {}
+_MAX_CONTRACTIONS = 16384
 
 
 def _relabel(*label_lists):
@@ -115,9 +121,11 @@ class Tensor:
         self._shape = [int(s) for s in shape]
         self._index_to_dimension = {i: s for i, s in zip(self._indices, self._shape)}
 
-    def _alloc(self, n: int):
+    def _alloc(self, n: int, ordered: bool = True):
+        """``ordered``: what fills the tensor runs on its context's stream."""
         self._size = int(n)
-        self._buf = nat.DeviceBuffer(max(1, self._size) * self.dtype.itemsize, self._ctx)
+        self._buf = nat.DeviceBuffer(max(1, self._size) * self.dtype.itemsize, self._ctx,
+                                     ordered)
 
     def _zero(self):
         nat.check(nat.lib().jet_hip_memset(self._ctx.handle, self._buf.ptr, 0,
@@ -356,15 +364,30 @@ class Tensor:
         indices; the result's indices are (A \\ B) ++ (B \\ A)."""
         if A.dtype != B.dtype:
             raise JetError("Tensor data types do not match.")
-        left = vector_subtraction(A._indices, B._indices)
-        right = vector_subtraction(B._indices, A._indices)
-        c_indices = vector_union(left, right)
-        c_shape = [A._index_to_dimension[i] for i in left] + \
-                  [B._index_to_dimension[i] for i in right]
-        C = Tensor._empty(c_indices, c_shape, A.dtype, A._ctx)
-        ma, mb, mc = _relabel(A._indices, B._indices, c_indices)
-        plan = _plan_cache.get(A._ctx, A._code, _PRECISIONS[precision], ma, A._shape, mb,
-                               B._shape, mc)
+        key = (A._ctx.device, A._code, precision, tuple(A._indices), tuple(A._shape),
+               tuple(A._index_to_dimension.items()), tuple(B._indices), tuple(B._shape),
+               tuple(B._index_to_dimension.items()))
+        known = _contractions.get(key)
+        if known is None:
+            left = vector_subtraction(A._indices, B._indices)
+            right = vector_subtraction(B._indices, A._indices)
+            c_indices = vector_union(left, right)
+            c_shape = [A._index_to_dimension[i] for i in left] + \
+                      [B._index_to_dimension[i] for i in right]
+            ma, mb, mc = _relabel(A._indices, B._indices, c_indices)
+            plan, ctx = _plan_cache.get(A._ctx, A._code, _PRECISIONS[precision], ma, A._shape,
+                                        mb, B._shape, mc)
+            if len(_contractions) >= _MAX_CONTRACTIONS:
+                _contractions.clear()
+            known = _contractions[key] = (c_indices, c_shape, shape_to_size(c_shape), plan, ctx)
+        c_indices, c_shape, size, plan, ctx = known
+        C = Tensor.__new__(Tensor)
+        C._ctx = A._ctx
+        C.dtype = A.dtype
+        C._code = A._code
+        C._default = False
+        C._init_indices_and_shape(c_indices, c_shape)
+        C._alloc(size, ordered=ctx is A._ctx)
         nat.check(nat.lib().jet_hip_contract(plan, A._buf.ptr, B._buf.ptr, C._buf.ptr, None, 0,
                                              None))
         return C
