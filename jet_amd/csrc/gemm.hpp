@@ -109,8 +109,8 @@ inline int64_t x4m_slices(int64_t M, int64_t N, int64_t K, int64_t batch, int va
 // time per tile, and a tile costs `out` us beside its stages (prologue and
 // stores).  Measured on shapes with one tile per CU and with many; FP32,
 // predicted / measured us: 1024^3 62, 53, 56 / 65, 54, 55 for the 64x64, 64x32
-// and 32x32 tiles, 2048^3 337, 353 / 336, 369 for 128x128 and 64x64,
-// 256x65536x256 175, 192 / 178, 193 for 256x128 and 128x128; FP64: 1024^3 137,
+// and 32x32 tiles, 2048^3 301, 353 / 308, 369 for 128x128 and 64x64,
+// 256x65536x256 160, 173 / 160, 177 for 256x128 and 128x128; FP64: 1024^3 137,
 // 137 / 144, 148 for 32x32 with and without slices in the tile, 1536x1536x512
 // 158, 252 / 160, 256 for 32x32 and 128x128.  The FP32 choices are within 6% of
 // the best of eleven forms timed on 19 shapes from 64^3 to 4096x4096x1024.
@@ -118,8 +118,8 @@ struct TileForm {
     int bm, bn, kt, occ;
     float alone, full, out;
 };
-constexpr TileForm kF32x6Forms[] = {{256, 128, 16, 1, 3.9f, 4.85f, 10.f},
-                                    {128, 128, 16, 1, 2.4f, 2.63f, 6.f},
+constexpr TileForm kF32x6Forms[] = {{256, 128, 16, 1, 3.33f, 4.27f, 11.5f},
+                                    {128, 128, 16, 1, 1.89f, 2.3f, 6.5f},
                                     {64, 64, 16, 3, 0.92f, 0.69f, 1.f},
                                     {64, 32, 32, 2, 1.05f, 0.77f, 0.6f},
                                     {32, 32, 64, 2, 1.1f, 0.8f, 0.4f}};

@@ -8,8 +8,8 @@
 // normal, an absolute 2^-126).  Four real products make 24 v_mfma_f32_32x32x16_bf16 per 32x32
 // block and 16 k: at BF16's rate (16 times FP32's on the same matrix cores)
 // that is 2.7 times the FP32 MFMA rate.  Measured (TFLOP/s of 8 M N K, FP32
-// MFMA kernel before -> this one): 4096^3 121 -> 227, 4096x4096x1024 119 ->
-// 219, 256x65536x256 113 -> 192, 1024^3 52 -> 158; 512^3 (which the VALU
+// MFMA kernel before -> this one): 4096^3 121 -> 248, 4096x4096x1024 119 ->
+// 238, 256x65536x256 113 -> 216, 1024^3 52 -> 166; 512^3 (which the VALU
 // kernel ran) 368 -> 12 us.  Errors against 64 bits (normwise, random
 // operands): 4096^3 1.6e-6 -> 1.4e-6, 1024^3 8.1e-7 -> 1.9e-7, 512^3 5.7e-7
 // -> 9.8e-8, K = 64 7.4e-8 -> 5.6e-8: the accumulator takes fewer roundings
@@ -20,8 +20,15 @@
 //
 // The operands stay FP32 in memory and in LDS (8 bytes per complex value:
 // three pieces of each part would be 12) and are split in registers after
-// the LDS read, about 5.5 VALU instructions per value, issued beside the
-// other wave's MFMAs; there is no operand pass and no workspace.
+// the LDS read, 5.5 VALU instructions per value; there is no operand pass and
+// no workspace.  A wave issues a VALU instruction every 8 cycles and an MFMA holds
+// the matrix cores for 32, so a split hides behind the products where it is
+// little work and stands beside them: the wide tiles give a wave 128x64 (64x64)
+// outputs and one SIMD, three VALU instructions per MFMA, and read and split the
+// next operands during the products (4096^3, eight waves of 64x64 that split
+// first: 2520 us, matrix cores busy 60% of the cycles; four pipelined waves of 128x64:
+// 2230, 75%, at a clock lowered for power).  Small tiles keep two or three
+// waves per SIMD instead; pipelined they measured the same or less.
 #include "common.hpp"
 #include "gemm.hpp"
 #include "gemm_device.hpp"
@@ -123,13 +130,21 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
 #pragma unroll
     for (int i = 0; i < L; i++) {
         const bool isa = i < A_IN;
-        const int pd = (wave * (isa ? A_IN : B_IN) + (isa ? i : i - A_IN)) * 64 + lane;
-        const int p = pd / PER, sub = (pd % PER) * DW;
-        const int r = (p >> 3) % (isa ? BM : BN), slot = p & 7, kk = (p >> 3) / (isa ? BM : BN);
+        const int load = wave * (isa ? A_IN : B_IN) + (isa ? i : i - A_IN);
         const int64_t rows = isa ? g.M - m0 : g.N - n0;
+        const int R = isa ? BM : BN;
+        int r, kk;
+        if (DW == 4) { // eight rows a load: the lane's k is the same in every load
+            r = load * 8 % R + (lane >> 3), kk = load * 8 / R;
+            ck[i] = 16 * kk + 2 * ((lane & 7) ^ (lane >> 3));
+        }
+        else {
+            const int p = (load * 64 + lane) / PER;
+            r = (p >> 3) % R, kk = (p >> 3) / R;
+            ck[i] = 16 * kk + 2 * ((p & 7) ^ (r & 7)) + (lane % PER) * DW / 2;
+        }
         const int64_t rr = r < rows ? r : rows - 1;
-        ck[i] = 16 * kk + 2 * (slot ^ (r & 7)) + sub / 2;
-        off[i] = uint32_t(rr * (isa ? g.lda : g.ldb) * 8) + (sub & 1) * 4;
+        off[i] = uint32_t(rr * (isa ? g.lda : g.ldb) * 8) + (DW == 4 ? 0 : ((lane % PER) & 1) * 4);
     }
     auto issue = [&](int kt, f32x4 *s) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
@@ -182,108 +197,197 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
             im.h[c] = h, im.m[c] = m, im.l[c] = l;
         }
     };
-    auto compute = [&](const f32x4 *s, bool tail, int kt) __attribute__((always_inline)) {
-        const int kv = K - kt * KT - 16 * wk - 8 * q;
-        Pieces br[FN], bi[FN];
-#pragma unroll
-        for (int fn = 0; fn < FN; fn++) {
-            const int r = wn * WTN + fn * 32 + j;
-            fetch(s + (BM * WK + BN * wk + r) * 8, r & 7, tail, kv, br[fn], bi[fn]);
+    // The products of one block: smallest terms first, the two accumulators by
+    // turns.
+    auto products = [&](int fm, int fn, const Pieces &ar, const Pieces &ai, const Pieces &br,
+                        const Pieces &bi) __attribute__((always_inline)) {
+        Pieces ni;
+        ni.h = ai.h ^ 0x80008000u;
+        ni.m = ai.m ^ 0x80008000u;
+        ni.l = ai.l ^ 0x80008000u;
+        f32x16 x = DUAL ? dr[fm % DM][fn % DN] : cr[fm][fn];
+        f32x16 y = DUAL ? di[fm % DM][fn % DN] : ci[fm][fn];
+        auto term = [&](u32x4 Pieces::*a, u32x4 Pieces::*b) __attribute__((always_inline)) {
+            x = mma(ar.*a, br.*b, x);
+            y = mma(ar.*a, bi.*b, y);
+            x = mma(ni.*a, bi.*b, x);
+            y = mma(ai.*a, br.*b, y);
+        };
+        term(&Pieces::l, &Pieces::h);
+        term(&Pieces::h, &Pieces::l);
+        term(&Pieces::m, &Pieces::m);
+        term(&Pieces::m, &Pieces::h);
+        term(&Pieces::h, &Pieces::m);
+        if (DUAL) {
+            dr[fm % DM][fn % DN] = x;
+            di[fm % DM][fn % DN] = y;
+            x = cr[fm][fn];
+            y = ci[fm][fn];
         }
-#pragma unroll
-        for (int fm = 0; fm < FM; fm++) {
-            const int r = wm * WTM + fm * 32 + j;
-            Pieces ar, ai, ni;
-            fetch(s + (BM * wk + r) * 8, r & 7, tail, kv, ar, ai);
-            ni.h = ai.h ^ 0x80008000u;
-            ni.m = ai.m ^ 0x80008000u;
-            ni.l = ai.l ^ 0x80008000u;
-#pragma unroll
-            for (int fn = 0; fn < FN; fn++) {
-                f32x16 x = DUAL ? dr[fm % DM][fn % DN] : cr[fm][fn];
-                f32x16 y = DUAL ? di[fm % DM][fn % DN] : ci[fm][fn];
-                x = mma(ar.l, br[fn].h, x);
-                y = mma(ar.l, bi[fn].h, y);
-                x = mma(ni.l, bi[fn].h, x);
-                y = mma(ai.l, br[fn].h, y);
-                x = mma(ar.h, br[fn].l, x);
-                y = mma(ar.h, bi[fn].l, y);
-                x = mma(ni.h, bi[fn].l, x);
-                y = mma(ai.h, br[fn].l, y);
-                x = mma(ar.m, br[fn].m, x);
-                y = mma(ar.m, bi[fn].m, y);
-                x = mma(ni.m, bi[fn].m, x);
-                y = mma(ai.m, br[fn].m, y);
-                x = mma(ar.m, br[fn].h, x);
-                y = mma(ar.m, bi[fn].h, y);
-                x = mma(ni.m, bi[fn].h, x);
-                y = mma(ai.m, br[fn].h, y);
-                x = mma(ar.h, br[fn].m, x);
-                y = mma(ar.h, bi[fn].m, y);
-                x = mma(ni.h, bi[fn].m, x);
-                y = mma(ai.h, br[fn].m, y);
-                if (DUAL) {
-                    dr[fm % DM][fn % DN] = x;
-                    di[fm % DM][fn % DN] = y;
-                    x = cr[fm][fn];
-                    y = ci[fm][fn];
-                }
-                x = mma(ar.h, br[fn].h, x);
-                y = mma(ar.h, bi[fn].h, y);
-                x = mma(ni.h, bi[fn].h, x);
-                y = mma(ai.h, br[fn].h, y);
-                cr[fm][fn] = x;
-                ci[fm][fn] = y;
-            }
-        }
+        term(&Pieces::h, &Pieces::h);
+        cr[fm][fn] = x;
+        ci[fm][fn] = y;
+    };
+    auto fetch_a = [&](const f32x4 *s, int fm, bool tail, int kt, Pieces &re,
+                       Pieces &im) __attribute__((always_inline)) {
+        const int r = wm * WTM + fm * 32 + j;
+        fetch(s + (BM * wk + r) * 8, r & 7, tail, K - kt * KT - 16 * wk - 8 * q, re, im);
+    };
+    auto fetch_b = [&](const f32x4 *s, int fn, bool tail, int kt, Pieces &re,
+                       Pieces &im) __attribute__((always_inline)) {
+        const int r = wn * WTN + fn * 32 + j;
+        fetch(s + (BM * WK + BN * wk + r) * 8, r & 7, tail, K - kt * KT - 16 * wk - 8 * q, re,
+              im);
     };
 
-    const int nk = (K + KT - 1) / KT;
-    // vmcnt(L): the loads of the next stage may stay in flight.
-    constexpr int kWaitPrev = 0x0f70 | (L & 15) | ((L >> 4) << 14);
+    const int nk = (K + KT - 1) / KT, nfull = K / KT;
+    // vmcnt(L), vmcnt(2 L): the loads of later stages may stay in flight.
     constexpr int kWaitAll = 0x0f70;
-    issue(0, S0);
-    if (NS == 3 && nk > 1) issue(1, S1);
-    // Stage kt is in LDS for every wave once each has waited for its own
-    // loads; every wave is then also past its reads of stage kt - 1, whose
-    // buffer takes stage kt + NS - 1.
-    auto arrive = [&](int kt, f32x4 *next) __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (NS == 3 && kt + 1 < nk)
-            __builtin_amdgcn_s_waitcnt(kWaitPrev);
-        else
-            __builtin_amdgcn_s_waitcnt(kWaitAll);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        if (kt + NS - 1 < nk) issue(kt + NS - 1, next);
-    };
-    const int nfull = K / KT;
-    int kt = 0;
-    if (NS == 3) {
-        for (; kt + 3 <= nfull; kt += 3) {
-            arrive(kt, S2);
-            compute(S0, false, kt);
-            arrive(kt + 1, S0);
-            compute(S1, false, kt + 1);
-            arrive(kt + 2, S1);
-            compute(S2, false, kt + 2);
+    constexpr int kWaitPrev = kWaitAll | (L & 15) | ((L >> 4) << 14);
+    constexpr int kWaitTwo = kWaitAll | ((2 * L) & 15) | (((2 * L) >> 4) << 14);
+    if constexpr (FM > 1) {
+        // One wave per SIMD: the next operand of its own is read and split
+        // beside each block's products, in the order in which registers get
+        // free: B's second half beside (0, 0), A's row fm + 1 beside (fm, 1), and
+        // beside the last row the next stage's A row 0 and first half of B.
+        // That stage is in LDS for every wave once each has waited for its own
+        // loads; every wave is then past its reads of this stage, whose buffer
+        // takes the stage after the next two.
+        static_assert(NS == 3 && WK == 1 && FN == 2 && DW == 4 && 2 * L < 64, "pipelined form");
+        Pieces ar, ai, br[2], bi[2];
+        // 24 products: six before the values just read are used, then by turns
+        // with the VALU.
+        auto interleave = [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+#pragma unroll
+            for (int i = 6; i < 24; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // Stage kt (in s) into LDS for every wave: own loads, zeros for k past K
+        // (K is even here), own reads of the stage before; then the barrier.
+        auto arrive = [&](int kt, f32x4 *s) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (kt + 1 < nk) {
+                if (kt == 0 && nk > 2)
+                    __builtin_amdgcn_s_waitcnt(kWaitTwo);
+                else
+                    __builtin_amdgcn_s_waitcnt(kWaitPrev);
+            }
+            else {
+                __builtin_amdgcn_s_waitcnt(kWaitAll);
+                if (kt < nk && nk > nfull) {
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int i = 0; i < L; i++)
+                        if (kt * KT + ck[i] >= K)
+                            s[(i < A_IN ? wave * A_IN + i : BM / 8 + wave * B_IN + i - A_IN) * 64 +
+                              lane] = f32x4{};
+                }
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0)
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // After the last stage what is read and split is not used.
+        auto stage = [&](int kt, f32x4 *s, f32x4 *next) __attribute__((always_inline)) {
+            Pieces nr, ni;
+            fetch_b(s, 1, false, kt, br[1], bi[1]);
+            products(0, 0, ar, ai, br[0], bi[0]);
+            interleave();
+#pragma unroll
+            for (int fm = 0; fm + 1 < FM; fm++) {
+                fetch_a(s, fm + 1, false, kt, nr, ni);
+                products(fm, 1, ar, ai, br[1], bi[1]);
+                interleave();
+                ar = nr, ai = ni;
+                if (fm + 2 < FM) {
+                    products(fm + 1, 0, ar, ai, br[0], bi[0]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // split before the branches, beside the products above
+            asm volatile(""
+                         : "+v"(ar.h), "+v"(ar.m), "+v"(ar.l), "+v"(ai.h), "+v"(ai.m), "+v"(ai.l));
+            arrive(kt + 1, next);
+            if (kt + 3 < nk) issue(kt + 3, s);
+            fetch_a(next, 0, false, kt + 1, nr, ni);
+            products(FM - 1, 0, ar, ai, br[0], bi[0]);
+            interleave();
+            fetch_b(next, 0, false, kt + 1, br[0], bi[0]);
+            products(FM - 1, 1, ar, ai, br[1], bi[1]);
+            interleave();
+            ar = nr, ai = ni;
+        };
+        issue(0, S0);
+        if (nk > 1) issue(1, S1);
+        if (nk > 2) issue(2, S2);
+        arrive(0, S0);
+        fetch_b(S0, 0, false, 0, br[0], bi[0]);
+        fetch_a(S0, 0, false, 0, ar, ai);
+        int kt = 0;
+        for (; kt + 3 <= nk; kt += 3) {
+            stage(kt, S0, S1);
+            stage(kt + 1, S1, S2);
+            stage(kt + 2, S2, S0);
         }
-        // At most three stages are left; only the third is still to be issued.
-        for (int b = 0; kt < nk; kt++, b++) {
-            arrive(kt, S2);
-            compute(b == 0 ? S0 : b == 1 ? S1 : S2, true, kt);
-        }
+        for (int b = 0; kt < nk; kt++, b++) stage(kt, b == 0 ? S0 : S1, b == 0 ? S1 : S2);
     }
     else {
-        for (; kt + 2 <= nfull; kt += 2) {
-            arrive(kt, S1);
-            compute(S0, false, kt);
-            arrive(kt + 1, S0);
-            compute(S1, false, kt + 1);
+        auto compute = [&](const f32x4 *s, bool tail, int kt) __attribute__((always_inline)) {
+            static_assert(FN == 1, "one block per wave");
+            Pieces ar, ai, br, bi;
+            fetch_b(s, 0, tail, kt, br, bi);
+            fetch_a(s, 0, tail, kt, ar, ai);
+            products(0, 0, ar, ai, br, bi);
+        };
+        issue(0, S0);
+        if (NS == 3 && nk > 1) issue(1, S1);
+        // Stage kt is in LDS for every wave once each has waited for its own
+        // loads; every wave is then also past its reads of stage kt - 1, whose
+        // buffer takes stage kt + NS - 1.
+        auto arrive = [&](int kt, f32x4 *next) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (NS == 3 && kt + 1 < nk)
+                __builtin_amdgcn_s_waitcnt(kWaitPrev);
+            else
+                __builtin_amdgcn_s_waitcnt(kWaitAll);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            if (kt + NS - 1 < nk) issue(kt + NS - 1, next);
+        };
+        int kt = 0;
+        if (NS == 3) {
+            for (; kt + 3 <= nfull; kt += 3) {
+                arrive(kt, S2);
+                compute(S0, false, kt);
+                arrive(kt + 1, S0);
+                compute(S1, false, kt + 1);
+                arrive(kt + 2, S1);
+                compute(S2, false, kt + 2);
+            }
+            // At most three stages are left; only the third is still to be issued.
+            for (int b = 0; kt < nk; kt++, b++) {
+                arrive(kt, S2);
+                compute(b == 0 ? S0 : b == 1 ? S1 : S2, true, kt);
+            }
         }
-        for (int b = 0; kt < nk; kt++, b++) {
-            arrive(kt, b == 0 ? S1 : S0);
-            compute(b == 0 ? S0 : S1, true, kt);
+        else {
+            for (; kt + 2 <= nfull; kt += 2) {
+                arrive(kt, S1);
+                compute(S0, false, kt);
+                arrive(kt + 1, S0);
+                compute(S1, false, kt + 1);
+            }
+            for (int b = 0; kt < nk; kt++, b++) {
+                arrive(kt, b == 0 ? S1 : S0);
+                compute(b == 0 ? S0 : S1, true, kt);
+            }
         }
     }
 
@@ -329,18 +433,37 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
 
     float2 *C = static_cast<float2 *>(g.C) + bz * g.sC + int64_t(blockIdx.y) * g.slice_stride;
     bool bad = false;
+    const int64_t row0 = m0 + wm * WTM + 4 * q, col0 = n0 + wn * WTN + j;
+    const bool whole = m0 + BM <= g.M && n0 + BN <= g.N;
 #pragma unroll
     for (int fm = 0; fm < FM; fm++)
 #pragma unroll
         for (int fn = 0; fn < FN; fn++) {
-            const int64_t col = n0 + wn * WTN + fn * 32 + j;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int64_t row = m0 + wm * WTM + fm * 32 + 8 * (i / 4) + 4 * q + (i & 3);
-                const float2 v{cr[fm][fn][i], ci[fm][fn][i]};
-                bad |= !(__builtin_isfinite(v.x) && __builtin_isfinite(v.y));
-                if (row < g.M && col < g.N) C[row * g.ldc + col] = v;
+            if constexpr (FM > 1) {
+                // Block by block: all sums at once do not fit beside the matrix
+                // cores' registers, and a spilled value read back between stores
+                // waits for them.
+                asm volatile("" : "+a"(cr[fm][fn]), "+a"(ci[fm][fn]));
+                __builtin_amdgcn_sched_barrier(0);
             }
+            float2 *const p = C + (row0 + fm * 32) * g.ldc + col0 + fn * 32;
+            auto store = [&](bool masked) __attribute__((always_inline)) {
+                float2 *o = p;
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const float2 v{cr[fm][fn][i], ci[fm][fn][i]};
+                    bad |= !(__builtin_isfinite(v.x) && __builtin_isfinite(v.y));
+                    if (!masked || (col0 + fn * 32 < g.N &&
+                                    row0 + fm * 32 + 8 * (i / 4) + (i & 3) < g.M))
+                        *o = v;
+                    // to the next row: 1 further, or past the other half's 4
+                    o += ((i & 3) == 3 ? 5 : 1) * g.ldc;
+                }
+            };
+            if (whole)
+                store(false);
+            else
+                store(true);
         }
     if (!bad) return;
     // An infinite or NaN input (or a result out of range): the pieces of an
@@ -398,7 +521,7 @@ void launch_f32x6(const GemmArgs &g, hipStream_t stream)
     }
     switch (form) {
     case 0:
-        launch_tile<256, 128, 4, 2, 1, 3, false>(g, stream);
+        launch_tile<256, 128, 2, 2, 1, 3, false>(g, stream);
         break;
     case 1:
         launch_tile<128, 128, 2, 2, 1, 3, true>(g, stream);

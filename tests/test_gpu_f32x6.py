@@ -93,3 +93,14 @@ def test_infinities_and_nan_propagate(ctx, table, M, N, K):
         w, g, o = (re + 1j * im)[rows], got[rows], ok[rows]
         err = np.linalg.norm((g[o] - w[o]).astype(np.complex128)) / np.linalg.norm(w[o])
         assert err < 2.0 ** -24 * (math.sqrt(K) + 8), (rows, err)
+
+
+# The wide tiles' stages of 16 k run three at a time, read ahead by one and loaded
+# ahead by three: 3 to 12 stages, whole and partial last ones (256x128, then
+# 128x128 tiles).
+@pytest.mark.parametrize("M,N,K", [
+    (4090, 4094, 34), (4096, 4096, 64), (4090, 4094, 80), (4096, 4096, 112), (4090, 4094, 146),
+    (4096, 4080, 176), (4090, 4094, 178), (2040, 2044, 974), (2048, 2048, 992),
+    (2040, 2044, 1006)])
+def test_wide_tile_stages(ctx, table, M, N, K):
+    test_against_64_bits(ctx, table, M, N, K, 1)
