@@ -221,7 +221,9 @@ __global__ __launch_bounds__(256) void cgemm_small_kernel(GemmArgs g)
 // scalar load, its bit positions packed in words (a loop over byte positions
 // waits for a load per bit), k offsets are made from them on the scalar unit
 // for the k bits that all lanes share, four k at a time, and there is no
-// barrier unless an output has more lanes than a wave.
+// barrier unless an output has more lanes than a wave.  Sums run in FP64, which
+// costs nothing beside the latencies, so that a value passing hundreds of
+// steps is rounded once in each.
 __device__ __forceinline__ uint32_t group_word(const uint32_t *w, int i)
 {
     return (w[i / 6] >> (5 * (i % 6))) & 31u;
@@ -250,12 +252,13 @@ __device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t 
     const bool live = idx < 1u << g.lo;
     const In x = In(Av) + (group_offset<OB>(g.oa, idx & g.mask_a) | group_offset<LANES>(g.ka, k0));
     const In y = In(Bv) + (group_offset<OB>(g.ob, idx & g.mask_b) | group_offset<LANES>(g.kb, k0));
-    R sr = 0, si = 0;
+    double sr = 0, si = 0;
     auto mac = [&](R2 u, R2 v) {
-        sr = fma(u.x, v.x, sr);
-        sr = fma(-u.y, v.y, sr);
-        si = fma(u.x, v.y, si);
-        si = fma(u.y, v.x, si);
+        const double ar = u.x, ai = u.y, br = v.x, bi = v.y;
+        sr = fma(ar, br, sr);
+        sr = fma(-ai, bi, sr);
+        si = fma(ar, bi, si);
+        si = fma(ai, br, si);
     };
     if (live) {
         const uint32_t K = 1u << g.lk;
@@ -280,7 +283,7 @@ __device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t 
         si += __shfl_xor(si, off);
     }
     if constexpr (LANES > 6) {
-        __shared__ R sums[2][4];
+        __shared__ double sums[2][4];
         if (g.lanes > 6) { // 128 or 256 lanes: two outputs or one
             if ((tid & 63) == 0) {
                 sums[0][tid >> 6] = sr;
@@ -297,7 +300,7 @@ __device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t 
         }
     }
     const Out z = Out(Cv);
-    if (live && k0 == 0) z[group_offset<OB>(g.oc, idx)] = R2{sr, si};
+    if (live && k0 == 0) z[group_offset<OB>(g.oc, idx)] = R2{R(sr), R(si)};
 }
 
 template <class R>
