@@ -223,7 +223,9 @@ __global__ __launch_bounds__(256) void cgemm_small_kernel(GemmArgs g)
 // for the k bits that all lanes share, four k at a time, and there is no
 // barrier unless an output has more lanes than a wave.  Sums run in FP64, which
 // costs nothing beside the latencies, so that a value passing hundreds of
-// steps is rounded once in each.
+// steps is rounded once in each.  Measured on loss and gradient of 300 angles (36
+// qubits, about 1400 steps): 8.9 ms with a launch per step, 4.1 grouped, 3.75 with the
+// record in scalar registers, 2.8 with the single steps alike.
 __device__ __forceinline__ uint32_t group_word(const uint32_t *w, int i)
 {
     return (w[i / 6] >> (5 * (i % 6))) & 31u;
@@ -237,23 +239,27 @@ template <int BITS> __device__ __forceinline__ uint32_t group_offset(const uint3
     return o;
 }
 
-// Output `first` + thread / 2^lanes of the work-group; OB, KB: bits of the
-// output index and of k; LANES: most lanes per output (log2).
-template <class R, int OB, int KB, int LANES>
+// Output `first` + thread / 2^lanes of the work-group; A, B and C hold values
+// of RA, RB and RC; OB, KB: bits of the output index and of k; LANES: most lanes
+// per output (log2).
+template <class RA, class RB, class RC, int OB, int KB, int LANES>
 __device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t first,
                                                   const void *Av, const void *Bv, void *Cv)
 {
     // global-memory pointers (generic ones would make flat loads)
-    typedef R R2 __attribute__((ext_vector_type(2)));
-    typedef __attribute__((address_space(1))) const R2 *In;
-    typedef __attribute__((address_space(1))) R2 *Out;
+    typedef RA A2 __attribute__((ext_vector_type(2)));
+    typedef RB B2 __attribute__((ext_vector_type(2)));
+    typedef RC C2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(1))) const A2 *InA;
+    typedef __attribute__((address_space(1))) const B2 *InB;
+    typedef __attribute__((address_space(1))) C2 *Out;
     const uint32_t tid = threadIdx.x, G = 1u << g.lanes;
     const uint32_t idx = first + (tid >> g.lanes), k0 = tid & (G - 1);
     const bool live = idx < 1u << g.lo;
-    const In x = In(Av) + (group_offset<OB>(g.oa, idx & g.mask_a) | group_offset<LANES>(g.ka, k0));
-    const In y = In(Bv) + (group_offset<OB>(g.ob, idx & g.mask_b) | group_offset<LANES>(g.kb, k0));
+    const InA x = InA(Av) + (group_offset<OB>(g.oa, idx & g.mask_a) | group_offset<LANES>(g.ka, k0));
+    const InB y = InB(Bv) + (group_offset<OB>(g.ob, idx & g.mask_b) | group_offset<LANES>(g.kb, k0));
     double sr = 0, si = 0;
-    auto mac = [&](R2 u, R2 v) {
+    auto mac = [&](A2 u, B2 v) {
         const double ar = u.x, ai = u.y, br = v.x, bi = v.y;
         sr = fma(ar, br, sr);
         sr = fma(-ai, bi, sr);
@@ -264,7 +270,8 @@ __device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t 
         const uint32_t K = 1u << g.lk;
         if (K >= 4 * G) {
             for (uint32_t k = 0; k < K; k += 4 * G) {
-                R2 u[4], v[4];
+                A2 u[4];
+                B2 v[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     u[e] = x[group_offset<KB>(g.ka, k + e * G)];
@@ -300,23 +307,46 @@ __device__ __forceinline__ void small_contraction(const GroupBlock &g, uint32_t 
         }
     }
     const Out z = Out(Cv);
-    if (live && k0 == 0) z[group_offset<OB>(g.oc, idx)] = R2{R(sr), R(si)};
+    if (live && k0 == 0) z[group_offset<OB>(g.oc, idx)] = C2{RC(sr), RC(si)};
 }
 
+template <class RA, class RB, class RC>
+__device__ __forceinline__ void grouped_contraction(const GroupBlock &g,
+                                                    const void *const *__restrict__ ptrs)
+{
+    small_contraction<RA, RB, RC, kGroupMaxLog2Outputs, kGroupMaxLog2K, 6>(
+        g, g.first, ptrs[g.a], ptrs[g.b], const_cast<void *>(ptrs[g.c]));
+}
 template <class R>
 __global__ __launch_bounds__(256) void grouped_small_kernel(const GroupBlock *__restrict__ blocks,
                                                             const void *const *__restrict__ ptrs)
 {
     const GroupBlock g = blocks[blockIdx.x];
-    small_contraction<R, kGroupMaxLog2Outputs, kGroupMaxLog2K, 6>(
-        g, g.first, ptrs[g.a], ptrs[g.b], const_cast<void *>(ptrs[g.c]));
+    switch (sizeof(R) == 4 ? g.wide : 0) {
+    case 0:
+        return grouped_contraction<R, R, R>(g, ptrs);
+    case 1:
+        return grouped_contraction<double, R, R>(g, ptrs);
+    case 2:
+        return grouped_contraction<R, double, R>(g, ptrs);
+    case 3:
+        return grouped_contraction<double, double, R>(g, ptrs);
+    case 4:
+        return grouped_contraction<R, R, double>(g, ptrs);
+    case 5:
+        return grouped_contraction<double, R, double>(g, ptrs);
+    case 6:
+        return grouped_contraction<R, double, double>(g, ptrs);
+    default:
+        return grouped_contraction<double, double, double>(g, ptrs);
+    }
 }
 
 template <class R>
 __global__ __launch_bounds__(256) void fused_small_kernel(const void *A, const void *B, void *C,
                                                           GroupBlock g)
 {
-    small_contraction<R, kSmallMaxLog2Outputs, kFusedMaxLog2K, 8>(
+    small_contraction<R, R, R, kSmallMaxLog2Outputs, kFusedMaxLog2K, 8>(
         g, blockIdx.x * (256u >> g.lanes), A, B, C);
 }
 
@@ -779,7 +809,8 @@ __global__ __launch_bounds__(256) void split_f16_block_rows_kernel(
 //   3. the planes and scales are written from registers as
 //      split_f16_rows_kernel writes them.
 // Every per-element offset is computed once per thread, outside the tile
-// loop.
+// loop, and bit positions come from unrolled code: as loops over the kernel's
+// arguments the pass took 11.2 ms of a 32-slice execution instead of 5.7.
 // LDS slot of tile element u: its low five bits (the bank of an 8-byte
 // element in a 256-byte bank row) XORed with bits 5-9 and 10-11, so that the
 // lanes of the row phase, which step through arbitrary u bits, spread over

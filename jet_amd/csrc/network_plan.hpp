@@ -20,7 +20,7 @@
 //     of two) run in groups of one launch each: all whose operands are ready
 //     at the same dependency level.  Their results have memory of their own,
 //     so their order does not matter to the arena; the other steps keep
-//     their order.
+//     their order.  complex64 results that only groups read are FP64.
 //
 // Pure C++ so that plans can be checked on the CPU.
 #pragma once
@@ -40,6 +40,7 @@ struct NetworkStep {
     size_t offset = 0;                // arena offset of the result
     bool is_root = false;
     bool grouped = false;             // runs in a group of small steps
+    bool wide = false;                // its result is FP64 for the groups that read it
     FusedSmall small;                 // its offsets then
 };
 
@@ -68,6 +69,11 @@ struct NetworkPlan {
     // caller's output (n_leaves), then the step results.
     std::vector<GroupBlock> blocks;
     int slot(int node) const { return node < n_leaves ? node : node + 1; }
+    size_t result_bytes(int s) const
+    {
+        return (size_t)elem_bytes * (steps[s].wide ? 2 : 1) * (size_t)steps[s].desc.size_c;
+    }
+    bool wide(int node) const { return node >= n_leaves && steps[node - n_leaves].wide; }
     // Contraction DAGs (plan_dag): no root and no output; `kept` marks the
     // step results that stay in the arena (a contiguous region at its end,
     // in the order they were listed) after an execution.

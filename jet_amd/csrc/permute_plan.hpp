@@ -9,8 +9,9 @@
 // runs.  Other shapes go by tiles of whole axes where such tiles have runs on
 // both sides, or use a gather kernel (coalesced writes).
 //
-// Pure C++: the index helpers below are shared by the kernels and by the CPU
-// emulation that checks plans and bounds before anything runs on a GPU.
+// Pure C++: the index helpers below are those of the CPU emulation that checks
+// plans and bounds before anything runs on a GPU; the kernels share them, or
+// unroll them (bit positions).
 #pragma once
 
 #include "errors.hpp"

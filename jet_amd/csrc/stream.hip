@@ -29,6 +29,13 @@ template <class R> __device__ __forceinline__ void mac(R &re, R &im, R xr, R xi,
     im = fma(xi, yr, im);
 }
 
+// A small tensor on a few modes of a large one (StreamShortK).  Bound by reading
+// the large operand and writing the result once: 16-byte loads along its lowest
+// mode, the small operand in LDS, products on the VALU.  Partial lines stored
+// past the caches cost a read of the line each, so rows that are one piece of
+// the result are gathered in LDS.  Measured: a two-qubit gate on 26 qubits (read
+// and written twice with permuted copies before) 596 -> 188 us, 5.7 TB/s; gates
+// of one to four qubits on 25 qubits 126-619 -> 77-124 us.
 // NPAIR: columns n and n + 1 are neighbours in C.  STAGE: a step's rows and all
 // N columns are one contiguous piece of C: it is gathered in LDS (16-byte
 // chunks, swizzled within a row) and written in order.
@@ -224,6 +231,8 @@ void launch_typed(const StreamShortK &p, const void *x, const void *y, void *c, 
 // is in LDS.  Thread bits, lowest first: the tile's batch bits, m bits beyond
 // what a thread can sum, k.  Sums in FP64, as the split-K kernel's, first per
 // thread, then over the threads, then over the work-groups (final kernel).
+// Measured (permuted copies and the split-K kernel before): 4 x 2 outputs over
+// 2^22 k 263 -> 48 us, 2 x 2 over 2^20 k in 128 batches 3089 -> 759 us (5.7 TB/s).
 template <class R, int LM, int LN>
 __global__ __launch_bounds__(256) void stream_dot_kernel(
     const typename Pair<R>::c *__restrict__ A, const typename Pair<R>::c *__restrict__ B,

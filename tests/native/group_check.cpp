@@ -30,6 +30,7 @@ static int check(const NetworkPlan &np, int elem_bytes, int *n_launches, int *n_
             if (s < 0 || !np.steps[s].grouped) return 2;
             const NetworkStep &st = np.steps[s];
             if (g.a != np.slot(st.a) || g.b != np.slot(st.b)) return 3;
+            if (g.wide != (np.wide(st.a) | np.wide(st.b) << 1 | st.wide << 2)) return 10;
             if (at[s] >= 0 && at[s] != l) return 4;
             const int64_t lo = st.small.lb + st.small.lm + st.small.ln;
             if (int64_t(1) << lo != st.desc.size_c || g.first >= 1 << lo || g.lanes > 6) return 5;
@@ -42,6 +43,13 @@ static int check(const NetworkPlan &np, int elem_bytes, int *n_launches, int *n_
         for (int x : {np.steps[s].a, np.steps[s].b})
             if (x >= np.n_leaves && at[x - np.n_leaves] >= at[s]) return 7;
     }
+    // FP64 results: of networks, read by groups alone, not the root
+    for (int s = 0; s < ns; s++) {
+        const NetworkStep &st = np.steps[s];
+        if (st.wide && (elem_bytes != 8 || !st.grouped || st.is_root || np.dag))
+            return 11;
+        if (!st.grouped && (np.wide(st.a) || np.wide(st.b))) return 12;
+    }
     // life in launches; kept results to the end
     std::vector<int> end(at);
     for (int s = 0; s < ns; s++)
@@ -50,11 +58,11 @@ static int check(const NetworkPlan &np, int elem_bytes, int *n_launches, int *n_
     for (int s = 0; s < ns; s++) {
         if (np.dag && np.kept[s]) end[s] = (int)np.launches.size();
         if (np.steps[s].is_root) continue;
-        const size_t len = (size_t)elem_bytes * (size_t)np.steps[s].desc.size_c;
+        const size_t len = np.result_bytes(s);
         if (np.steps[s].offset + len > np.arena_bytes) return 8;
         for (int t = 0; t < s; t++) {
             if (np.steps[t].is_root || end[t] < at[s] || end[s] < at[t]) continue;
-            const size_t lt = (size_t)elem_bytes * (size_t)np.steps[t].desc.size_c;
+            const size_t lt = np.result_bytes(t);
             if (np.steps[s].offset < np.steps[t].offset + lt &&
                 np.steps[t].offset < np.steps[s].offset + len)
                 return 9;
