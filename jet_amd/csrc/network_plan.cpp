@@ -120,14 +120,21 @@ void choose_grouped(NetworkPlan &np, const std::vector<std::vector<int32_t>> &mo
     }
     if (n < kMinGrouped)
         for (NetworkStep &st : np.steps) st.grouped = false;
-    // complex64 results of a network that only groups read stay in FP64, as they
-    // are summed: rounded at the few steps that other kernels read, at no cost
-    // (the loads wait on latency).  24 amplitudes of 42 qubits, largest relative
-    // error 1.3e-5 -> 7.2e-6, root mean square 3.3e-6 -> 2.7e-6.  Not in DAGs,
-    // where it gains nothing: a loss and its gradients are as far off as their
-    // rounded gates (2.0e-6, and 1.2e-6 with FP32 results).
-    for (NetworkStep &st : np.steps)
-        st.wide = np.elem_bytes == 8 && !np.dag && st.grouped && !st.is_root;
+    // complex64 results that only groups read stay in FP64, as they are summed:
+    // rounded at the few steps that other kernels read, at no cost (the loads wait on
+    // latency).  24 amplitudes of 42 qubits (split FP16), largest relative error
+    // 1.2e-5 -> 7.8e-6.  In DAGs, products of two leaves are rounded all the same:
+    // the leaves of circuits are rounded roots of 1/2, whose products round back to
+    // what they were (root mean square error of twelve losses 1.2e-6 with FP32
+    // results, 2.0e-6 with FP64 ones, 0.9e-6 so; their gradients 1.5e-6, 2.1e-6,
+    // 1.0e-6; the amplitudes' largest error would be 1.3e-5).
+    std::vector<int> depth(np.n_leaves, 0);
+    for (size_t s = 0; s < np.steps.size(); s++) {
+        NetworkStep &st = np.steps[s];
+        depth.push_back(std::max(depth[st.a], depth[st.b]) + 1);
+        st.wide = np.elem_bytes == 8 && st.grouped && !st.is_root && !(np.dag && np.kept[s]) &&
+                  depth.back() > (np.dag ? 1 : 0);
+    }
     for (const NetworkStep &st : np.steps)
         if (!st.grouped)
             for (int x : {st.a, st.b})

@@ -43,10 +43,10 @@ static int check(const NetworkPlan &np, int elem_bytes, int *n_launches, int *n_
         for (int x : {np.steps[s].a, np.steps[s].b})
             if (x >= np.n_leaves && at[x - np.n_leaves] >= at[s]) return 7;
     }
-    // FP64 results: of networks, read by groups alone, not the root
+    // FP64 results: read by groups alone, neither kept nor the root
     for (int s = 0; s < ns; s++) {
         const NetworkStep &st = np.steps[s];
-        if (st.wide && (elem_bytes != 8 || !st.grouped || st.is_root || np.dag))
+        if (st.wide && (elem_bytes != 8 || !st.grouped || st.is_root || (np.dag && np.kept[s])))
             return 11;
         if (!st.grouped && (np.wide(st.a) || np.wide(st.b))) return 12;
     }
