@@ -122,18 +122,18 @@ void choose_grouped(NetworkPlan &np, const std::vector<std::vector<int32_t>> &mo
         for (NetworkStep &st : np.steps) st.grouped = false;
     // complex64 results that only groups read stay in FP64, as they are summed:
     // rounded at the few steps that other kernels read, at no cost (the loads wait on
-    // latency).  24 amplitudes of 42 qubits (split FP16), largest relative error
-    // 1.2e-5 -> 7.8e-6.  In DAGs, products of two leaves are rounded all the same:
-    // the leaves of circuits are rounded roots of 1/2, whose products round back to
-    // what they were (root mean square error of twelve losses 1.2e-6 with FP32
-    // results, 2.0e-6 with FP64 ones, 0.9e-6 so; their gradients 1.5e-6, 2.1e-6,
-    // 1.0e-6; the amplitudes' largest error would be 1.3e-5).
+    // latency).  Products with a leaf (in DAGs, of two leaves) are rounded all the
+    // same: the leaves of circuits are rounded roots of 1/2, whose products
+    // round back to what they were.  24 amplitudes of 42 qubits (split FP16), norm
+    // and largest error: 1.5e-6, 1.2e-5 with FP32 results, 2.1e-6, 7.8e-6 with FP64
+    // ones, 1.5e-6, 8.2e-6 so; root mean square of twelve losses 1.2e-6, 2.0e-6 and
+    // 0.9e-6, of their gradients 1.5e-6, 2.1e-6 and 1.0e-6.
     std::vector<int> depth(np.n_leaves, 0);
     for (size_t s = 0; s < np.steps.size(); s++) {
         NetworkStep &st = np.steps[s];
         depth.push_back(std::max(depth[st.a], depth[st.b]) + 1);
         st.wide = np.elem_bytes == 8 && st.grouped && !st.is_root && !(np.dag && np.kept[s]) &&
-                  depth.back() > (np.dag ? 1 : 0);
+                  (np.dag ? depth.back() > 1 : st.a >= np.n_leaves && st.b >= np.n_leaves);
     }
     for (const NetworkStep &st : np.steps)
         if (!st.grouped)
