@@ -1,11 +1,16 @@
 // gemm_f32x6.hip -- complex64 GEMM at FP32 accuracy on the BF16 matrix cores
 // (gfx950): the FP32 products of every precision mode.
 //
-// Each FP32 value is the sum of three BF16 pieces, x = h + m + l (rounded to
-// nearest: 3 x 8 significant bits, so the sum is exact), and a real product
-// keeps the six terms hh, hm, mh, hl, lh, mm; the dropped ones are below
-// 2^-24 of it (values under 2^-110 lose their low piece to BF16's smallest
-// normal, an absolute 2^-126).  Four real products make 24 v_mfma_f32_32x32x16_bf16 per 32x32
+// Each FP32 value is the sum of three BF16 pieces, 2^24 x = h + m + l (rounded
+// to nearest: 3 x 8 significant bits, so the sum is exact; unscaled, the pieces
+// of values under 2^-110 would fall below BF16's smallest normal), and a real
+// product keeps the six terms hh, hm, mh, hl, lh, mm; the dropped ones are below
+// 2^-24 of it.  Values from 2^103 on and sums from 2^79 on leave the scaled
+// range, and with infinities and NaN their outputs are computed again with the
+// FP32 instruction.  The scaling is one VALU instruction per value (4096^3 2380 ->
+// 2420 us, 64x32 tiles 3% more).
+//
+// Four real products make 24 v_mfma_f32_32x32x16_bf16 per 32x32
 // block and 16 k: at BF16's rate (16 times FP32's on the same matrix cores)
 // that is 2.7 times the FP32 MFMA rate.  Measured (TFLOP/s of 8 M N K, FP32
 // MFMA kernel before -> this one): 4096^3 121 -> 248, 4096x4096x1024 119 ->
@@ -20,11 +25,11 @@
 //
 // The operands stay FP32 in memory and in LDS (8 bytes per complex value:
 // three pieces of each part would be 12) and are split in registers after
-// the LDS read, 5.5 VALU instructions per value; there is no operand pass and
+// the LDS read, 6.5 VALU instructions per value; there is no operand pass and
 // no workspace.  A wave issues a VALU instruction every 8 cycles and an MFMA holds
 // the matrix cores for 32, so a split hides behind the products where it is
 // little work and stands beside them: the wide tiles give a wave 128x64 (64x64)
-// outputs and one SIMD, three VALU instructions per MFMA, and read and split the
+// outputs and one SIMD, 3.5 VALU instructions per MFMA, and read and split the
 // next operands during the products (4096^3, eight waves of 64x64 that split
 // first: 2520 us, matrix cores busy 60% of the cycles; four pipelined waves of 128x64:
 // 2230, 75%, at a clock lowered for power).  Small tiles keep two or three
@@ -62,12 +67,14 @@ __device__ __forceinline__ float high_bf16(uint32_t p)
     return __uint_as_float(p & 0xffff0000u);
 }
 
-// x = h + m + l, each rounded to nearest: 24 significant bits, so the sum is
-// exact unless l falls below BF16's smallest normal.
+// 2^24 x = h + m + l, each rounded to nearest: 24 significant bits, so the sum is
+// exact, and no piece of any FP32 number is below BF16's smallest normal.
+// Sums of products carry 2^48 until they are stored.
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l)
 {
-    h = pack_bf16(a, b);
-    const float ra = a - low_bf16(h), rb = b - high_bf16(h);
+    h = pack_bf16(a * kScale, b * kScale);
+    const float ra = fmaf(a, kScale, -low_bf16(h)), rb = fmaf(b, kScale, -high_bf16(h));
     m = pack_bf16(ra, rb);
     l = pack_bf16(ra - low_bf16(m), rb - high_bf16(m));
 }
@@ -451,7 +458,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
                 float2 *o = p;
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const float2 v{cr[fm][fn][i], ci[fm][fn][i]};
+                    const float2 v{cr[fm][fn][i] * kUnscale, ci[fm][fn][i] * kUnscale};
                     bad |= !(__builtin_isfinite(v.x) && __builtin_isfinite(v.y));
                     if (!masked || (col0 + fn * 32 < g.N &&
                                     row0 + fm * 32 + 8 * (i / 4) + (i & 3) < g.M))
@@ -465,28 +472,45 @@ __global__ __launch_bounds__(64 * WM * WN * WK,
             else
                 store(true);
         }
-    if (!bad) return;
-    // An infinite or NaN input (or a result out of range): the pieces of an
-    // infinity do not multiply as the infinity does, so those outputs are
-    // computed again from the operands.
-    for (int e = 0; e < FM * FN * 16; e++) {
-        const int i = e & 15, fn = (e >> 4) % FN, fm = (e >> 4) / FN;
-        const int64_t col = n0 + wn * WTN + fn * 32 + j;
-        const int64_t row = m0 + wm * WTM + fm * 32 + 8 * (i / 4) + 4 * q + (i & 3);
-        if (row >= g.M || col >= g.N) continue;
-        const float2 v = C[row * g.ldc + col];
-        if (__builtin_isfinite(v.x) && __builtin_isfinite(v.y)) continue;
-        const float2 *a = static_cast<const float2 *>(g.A) + bz * g.sA + row * g.lda + k_first;
-        const float2 *b = static_cast<const float2 *>(g.B) + bz * g.sB + col * g.ldb + k_first;
-        float sr = 0.f, si = 0.f;
-        for (int k = 0; k < K; k++) {
-            const float2 x = a[k], y = b[k];
-            sr = fmaf(x.x, y.x, sr);
-            sr = fmaf(-x.y, y.y, sr);
-            si = fmaf(x.x, y.y, si);
-            si = fmaf(x.y, y.x, si);
+    if (!__any(bad)) return;
+    // An infinite or NaN input, or values too large for the scaled sums: 32x32
+    // blocks with such an output run again with the FP32 instruction, straight
+    // from the operands, and give those outputs.  Lane l holds row (column) l % 32
+    // at k = l / 32; results lie as above.
+#pragma unroll 1
+    for (int e = 0; e < FM * FN; e++) {
+        const int64_t r0 = m0 + wm * WTM + (e / FN) * 32, col = n0 + wn * WTN + (e % FN) * 32 + j;
+        const int rows = int(min(g.M - r0 - 4 * q, int64_t(32))); // of this lane
+        float2 *const c = C + (r0 + 4 * q) * g.ldc + col;
+        uint32_t again = 0; // bit 8 (i / 4) + i % 4 for the lane's result i
+#pragma unroll 1
+        for (int r = 0; r < 32; r++)
+            if (!(r & 4) && r < rows && col < g.N) {
+                const float2 v = c[r * g.ldc];
+                if (!(__builtin_isfinite(v.x) && __builtin_isfinite(v.y))) again |= 1u << r;
+            }
+        if (!__any(again != 0)) continue;
+        const float2 *a = static_cast<const float2 *>(g.A) + bz * g.sA +
+                          min(r0 + j, g.M - 1) * g.lda + k_first;
+        const float2 *b = static_cast<const float2 *>(g.B) + bz * g.sB +
+                          min(col, g.N - 1) * g.ldb + k_first;
+        f32x16 re{}, im{};
+#pragma unroll 4
+        for (int k = 0; k < K; k += 2) {
+            const int kk = min(k + q, K - 1);
+            float2 x = a[kk], y = b[kk];
+            if (k + q >= K) x = y = float2{0.f, 0.f};
+            re = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, re, 0, 0, 0);
+            im = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.y, im, 0, 0, 0);
+            re = __builtin_amdgcn_mfma_f32_32x32x2f32(-x.y, y.y, re, 0, 0, 0);
+            im = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.x, im, 0, 0, 0);
         }
-        C[row * g.ldc + col] = float2{sr, si};
+        float2 *o = c;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            if (again >> (8 * (i / 4) + (i & 3)) & 1) *o = float2{re[i], im[i]};
+            o += ((i & 3) == 3 ? 5 : 1) * g.ldc;
+        }
     }
 }
 
