@@ -648,15 +648,17 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
     // Both sides at least 32 and a long k on a VALU reduction, whose table
     // entry stems from one walk of k per matrix-core tile: the matrix cores with
     // slices of k where they are faster.  The reduction reads its operands once per
-    // output (64x64x1024 7.0 us: 9.6 TB/s out of L2; complex128 18 TB/s).
+    // output (64x64x1024 7.0 us: 9.6 TB/s out of L2; complex128 18 TB/s).  The
+    // complex64 split-K form sums in FP64 and keeps its shapes (32x32x65536 error
+    // 2.6e-8, on the matrix cores 1.4e-7).
     if (d.chunks == 1 && d.M >= 32 && d.N >= 32 && d.K >= 2048 && d.batch <= 65535 &&
         (mode == 2 || f32x6_shape(d.M, d.N, d.K)) &&
-        (d.gemm_kernel == kGemmSmallRed || d.gemm_kernel == kGemmSplitK)) {
+        (d.gemm_kernel == kGemmSmallRed || (mode == 2 && d.gemm_kernel == kGemmSplitK))) {
         double us = 0;
         if (mode == 2)
             (void)tile_slices(kF64Forms, 16, d.M, d.N, d.K, d.batch, &us);
         else
-            (void)tile_slices(kF32x6Forms, 8, d.M, d.N, d.K, d.batch, &us);
+            (void)f32x6_slices(d.M, d.N, d.K, d.batch, &us);
         const double red = d.flops / 8.0 * (mode == 2 ? 32.0 / 18e6 : 16.0 / 9.6e6);
         const double copies = (d.need_a ? 4.0 : 0.0) + (d.need_b ? 4.0 : 0.0);
         if (us + copies < red) {
@@ -776,7 +778,7 @@ void layout_workspace(ContractionDesc &d)
     if (d.chunks == 1 && (d.gemm_kernel == kGemmBf16x4m || d.gemm_kernel == kGemmF16x4m))
         slices = x4m_slices(d.M, d.N, d.K, d.batch, d.gemm_variant);
     else if (d.chunks == 1 && d.gemm_kernel == kGemmF32Mfma && f32x6_shape(d.M, d.N, d.K))
-        slices = tile_slices(kF32x6Forms, 8, d.M, d.N, d.K, d.batch, nullptr);
+        slices = f32x6_slices(d.M, d.N, d.K, d.batch, nullptr);
     else if (d.chunks == 1 && d.gemm_kernel == kGemmF64Mfma)
         slices = tile_slices(kF64Forms, 16, d.M, d.N, d.K, d.batch, nullptr);
     if (slices > 1) {

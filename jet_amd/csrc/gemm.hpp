@@ -170,6 +170,25 @@ inline int tile_slices(const TileForm (&forms)[COUNT], int elem_bytes, int64_t M
     return best;
 }
 
+// The FP32 products' slices.  Up to 2^17 outputs with a side of at most 128 and a
+// long k were sums over the 256 threads of a work-group (kGemmSmallRed), whose
+// error grows more slowly with k than a chain's: slices of at most 256 k, from 8192
+// k on 512, keep the error below theirs on all tiles but the widest, which have
+// one sum per output (4096x32x16384 2.2e-7 as a reduction, 2.8e-7 in four slices,
+// 1.3e-7 in 32, 120 -> 161 us; 32x4096x1024 9.4e-8, in two slices 1.0e-7, in four
+// 7.9e-8).
+inline int f32x6_slices(int64_t M, int64_t N, int64_t K, int64_t batch, double *time)
+{
+    const int s = tile_slices(kF32x6Forms, 8, M, N, K, batch, time);
+    if (K < 1024 || (M > 128 && N > 128) || batch * M * N > (int64_t(1) << 17)) return s;
+    const int64_t parts = ceil_div(K, int64_t(K < 8192 ? 256 : 512)), least = parts < 64 ? parts : 64;
+    const int64_t k = ceil_div(ceil_div(K, least), 64) * 64;
+    if (least <= s || ceil_div(K, k) != least) return s; // none empty
+    int form = 0;
+    (void)tile_time(kF32x6Forms, M, N, k, batch * least, &form);
+    return form == 0 ? s : int(least);
+}
+
 // Rows and k of the split-BF16 operand planes are padded to these multiples.
 constexpr int kSplitRowPad = 16;
 constexpr int kSplitKPad = 32;
