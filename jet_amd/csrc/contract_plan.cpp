@@ -703,15 +703,25 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
         return d;
     }
 
-    // Small steps on the one-thread-per-output or the one-block-per-output
-    // VALU kernel that would need a permuted operand or result: one fused
-    // pass of the same form, no copies.
+    // Small steps that would need a permuted operand or result: one fused
+    // pass in place, no copies.  The table knows products without their copies;
+    // with them, up to 2^22 multiply-adds, one launch beats three or four whatever
+    // the kernel (complex64 scrambled: 64x64x64 3.7 us against 10.5, 2^20 5.6
+    // and 13, 2^22 10-13 and 16-18, but 2^23 17-22 and 14-18; complex128 8x8x8 3.7 and
+    // 6.3, 2^20 5.5 and 13-16, 2^23 17-21 and 16-18).  Long sums of few outputs
+    // that the table leaves to the VALU stay here up to 2^26.
     const double work = double(d.batch) * double(d.M) * double(d.N) * double(d.K);
-    const bool small = d.gemm_kernel == kGemmSmall && d.gemm_variant <= 1 && work <= double(1 << 22);
+    const bool copies = d.need_a || d.need_b || d.need_c;
+    const bool split = d.gemm_kernel == kGemmBf16x3 || d.gemm_kernel == kGemmBf16x4m ||
+                       d.gemm_kernel == kGemmF16x4m;
     const bool red = d.gemm_kernel == kGemmSmallRed && work <= double(1 << 26);
-    if ((small || red) && (d.need_a || d.need_b || d.need_c)) {
+    if (copies && d.chunks == 1 && (red || (!split && work <= double(1 << 22)))) {
         const auto &common = best_opt == 0 ? common_a : common_b;
         d.fused_small = plan_fused_small(A, EA, B, EB, C, batch, left, right, common, d.fs);
+        if (d.fused_small && d.gemm_kernel != kGemmSmallRed) {
+            d.gemm_kernel = kGemmSmall;
+            d.gemm_variant = 0;
+        }
     }
 
     layout_workspace(d);

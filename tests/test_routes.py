@@ -1,0 +1,77 @@
+"""Which form the planner gives a contraction (host only,
+tests/native/route_check.cpp).
+
+* Small contractions in scrambled orders run as one launch without workspace, in
+  every precision mode, whatever kernel the table names for their shape.
+"""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+from jet_amd import _native as nat
+from jet_amd import build as jb
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PRODUCT, FUSED, SHORT_K, FEW_OUTPUTS = 0, 1, 2, 3
+SPLIT_KERNELS = (4, 5, 7)
+
+
+@pytest.fixture(scope="module")
+def lib():
+    jb.write_tuning_table()
+    out = os.path.join(ROOT, "tests", "native", "_build", f"libroute_check.{os.getpid()}.so")
+    os.makedirs(os.path.dirname(out), exist_ok=True)
+    csrc = os.path.join(ROOT, "jet_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + jb.BUILD, "-o", out,
+                    os.path.join(ROOT, "tests", "native", "route_check.cpp")] +
+                   [os.path.join(csrc, f) for f in ("contract_plan.cpp", "permute_plan.cpp",
+                                                    "tuning.cpp")], check=True)
+    L = ctypes.CDLL(out)
+    os.remove(out)
+    return L
+
+
+def route(lib, mode, a, b, c, ext=2):
+    """Every mode of extent `ext`."""
+    e = lambda ms: nat.i64([ext] * len(ms))
+    out = (ctypes.c_int64 * 5)()
+    assert lib.contraction_route(mode, len(a), nat.i32(a), e(a), len(b), nat.i32(b), e(b), len(c),
+                                 nat.i32(c), out) == 0
+    return dict(zip(("form", "kernel", "launches", "slices", "workspace"), out))
+
+
+def modes(batch, m, n, k, rng=None):
+    """Modes of A, B and C, in the order of a batched product or (rng) scrambled."""
+    bb, mm = list(range(batch)), list(range(100, 100 + m))
+    nn, kk = list(range(200, 200 + n)), list(range(300, 300 + k))
+    a, b = bb + mm + kk, bb + nn + kk
+    if rng is None:
+        return a, b, bb + mm + nn
+    rng.shuffle(a)
+    rng.shuffle(b)
+    c = [x for x in a if x < 200] + [x for x in b if 200 <= x < 300]
+    return a, b, c
+
+
+@pytest.mark.parametrize("mode", [0, 2, 3, 4])
+def test_small_scrambled_contractions_are_one_launch(lib, mode):
+    rng = random.Random(mode)
+    named = [(0, 0, 0, 3), (0, 3, 3, 3), (0, 2, 6, 3), (0, 6, 6, 6), (0, 4, 4, 8), (0, 8, 8, 6)]
+    drawn = [(rng.choice([0, 0, 2, 4]), rng.randint(0, 9), rng.randint(0, 9), rng.randint(0, 11))
+             for _ in range(400)]
+    for batch, m, n, k in named + [d for d in drawn if sum(d) <= 22]:
+        r = route(lib, mode, *modes(batch, m, n, k, rng))
+        if r["kernel"] not in SPLIT_KERNELS:
+            assert r["launches"] == 1 and r["workspace"] == 0, ((batch, m, n, k), r)
+
+
+def test_larger_scrambled_contractions_are_products(lib):
+    """From 2^23 multiply-adds the matrix cores earn their copies."""
+    rng = random.Random(1)
+    for mode in (0, 2):
+        for shape in ((0, 9, 9, 5), (0, 8, 8, 8), (0, 8, 9, 8), (2, 8, 7, 8)):
+            assert route(lib, mode, *modes(*shape, rng))["form"] == PRODUCT, (mode, shape)
