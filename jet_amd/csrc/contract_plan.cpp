@@ -478,6 +478,37 @@ int choose_gemm_kernel(int mode, int64_t M, int64_t N, int64_t K,
     return kGemmSmall;
 }
 
+namespace {
+
+// Whether the in-place short-k form (d.sk) is the fastest for this problem.
+// Each batch has work-groups of its own, which put the small operand into LDS:
+// with fewer rows than one step of a work-group that pays where they have enough
+// multiply-adds left (2^15 batches of 8 rows, 2 k and 2 columns: 18 us, table kernel
+// 4; 2^12 batches of 4 rows, 16 and 16: 6.9, table 12; complex128, whose rows are
+// not staged then, 2^12 of 8, 16 and 8: 16 against 12, 2^12 of 8, 16 and 16: 14
+// against 21).  A thread's chain of k and columns shows in small problems: in place
+// by the fused pass instead (2^12 rows, 16 and 16: 7.0 us, fused 5.4; complex128 8.6 and
+// 6.3; 2^18 rows, 2 and 2: 4.0 and 6.8), and in the operands' own order by the
+// table's kernel (complex128 2^12 rows, 16 and 16: 9.3 us, table 3.6), but for its
+// reductions (2^2 batches of 2^9 rows, 16 and 8: 5.0, table 15).
+// There the matrix cores stay ahead with 16 k and 16 columns (complex128 2^15 rows:
+// 9.8 and 6.8 us, 2^17: 14 and 18; complex64 2^15: 7.2 and 6.0, 2^17: 9.3 and 18.5).
+bool stream_shortk_pays(const ContractionDesc &d, bool copies, double work)
+{
+    const StreamShortK &p = d.sk;
+    const bool c128 = d.elem_bytes == 16;
+    const int per_group = p.lr + p.lk + p.ln;
+    if (p.lb > 0 && p.lr < 9 && (!copies || work <= double(1 << 22)) &&
+        (c128 ? p.lk < 3 || per_group < 11 : p.lk < 1 || per_group < 10))
+        return false;
+    if (copies) return work > double(1 << 20) || p.lk + p.ln <= 5;
+    if (work <= double(1 << 20)) return d.gemm_kernel == kGemmSmallRed;
+    const bool matrix = d.gemm_kernel == kGemmF32Mfma || d.gemm_kernel == kGemmF64Mfma;
+    return !(matrix && p.lk + p.ln == 8 && work <= double(c128 ? 1 << 24 : 1 << 23));
+}
+
+} // namespace
+
 ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
                                  int ra, const int32_t *modes_a,
                                  const int64_t *ext_a, int rb,
@@ -675,12 +706,15 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
             d.fuse_b = plan_split_gather(B, EB, cat(gemm_batch, right, gemm_common), d.K, d.gb);
     }
 
+    const double work = double(d.batch) * double(d.M) * double(d.N) * double(d.K);
+    const bool copies = d.need_a || d.need_b || d.need_c;
+
     // A small tensor on a few modes of a large one: one pass over the large
     // one in place.  Up to 16 k and 16 columns the VALU keeps up with memory (2^25
     // values, 16 x 16: 124 us, 619 with permuted copies); below 2^14 elements the
     // fused small step is a launch as short.
     if (d.chunks == 1 && std::max(d.size_a, d.size_b) >= (int64_t(1) << 14) &&
-        plan_stream_shortk(A, EA, B, EB, C, d.sk)) {
+        plan_stream_shortk(A, EA, B, EB, C, d.sk) && stream_shortk_pays(d, copies, work)) {
         d.stream_shortk = true;
         d.gemm_kernel = kGemmSmall;
         d.gemm_variant = 0;
@@ -710,8 +744,6 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
     // and 13, 2^22 10-13 and 16-18, but 2^23 17-22 and 14-18; complex128 8x8x8 3.7 and
     // 6.3, 2^20 5.5 and 13-16, 2^23 17-21 and 16-18).  Long sums of few outputs
     // that the table leaves to the VALU stay here up to 2^26.
-    const double work = double(d.batch) * double(d.M) * double(d.N) * double(d.K);
-    const bool copies = d.need_a || d.need_b || d.need_c;
     const bool split = d.gemm_kernel == kGemmBf16x3 || d.gemm_kernel == kGemmBf16x4m ||
                        d.gemm_kernel == kGemmF16x4m;
     const bool red = d.gemm_kernel == kGemmSmallRed && work <= double(1 << 26);

@@ -3,6 +3,8 @@ tests/native/route_check.cpp).
 
 * Small contractions in scrambled orders run as one launch without workspace, in
   every precision mode, whatever kernel the table names for their shape.
+* The in-place form for a few k and columns is for problems with enough rows or
+  work per batch value, and large enough to hide its chain of sums.
 """
 import ctypes
 import os
@@ -75,3 +77,35 @@ def test_larger_scrambled_contractions_are_products(lib):
     for mode in (0, 2):
         for shape in ((0, 9, 9, 5), (0, 8, 8, 8), (0, 8, 9, 8), (2, 8, 7, 8)):
             assert route(lib, mode, *modes(*shape, rng))["form"] == PRODUCT, (mode, shape)
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+@pytest.mark.parametrize("shape", [
+    (15, 1, 4, 2), (15, 3, 1, 1), (15, 3, 2, 2), (8, 2, 3, 4), (14, 2, 2, 2), (15, 4, 0, 2),
+    (12, 2, 2, 2)])
+def test_few_rows_a_batch(lib, mode, shape):
+    """Many batches of few rows and little work each: the table's kernel, which
+    fills whole work-groups across batches."""
+    r = route(lib, mode, *modes(*shape))
+    assert r["form"] == PRODUCT and r["launches"] == 1, r
+    # the same with the larger operand second
+    a, b, c = modes(shape[0], shape[2], shape[1], shape[3])
+    assert route(lib, mode, a, b, c)["form"] == PRODUCT
+
+
+def test_short_k_where_it_pays(lib):
+    rng = random.Random(2)
+    for mode in (0, 2):
+        # gates on states, and batches of enough rows
+        for shape in ((0, 14, 2, 2), (0, 20, 1, 1), (0, 24, 2, 2), (0, 20, 4, 4)):
+            assert route(lib, mode, *modes(*shape))["form"] == \
+                (SHORT_K if sum(shape) > 20 else PRODUCT), (mode, shape)
+        assert route(lib, mode, *modes(6, 12, 2, 2))["form"] == SHORT_K
+        # small scrambled ones with many k and columns go to the fused pass
+        a, b, c = modes(0, 12, 4, 4)
+        assert route(lib, mode, a[::-1], b, c)["form"] == FUSED
+        # table kernels in the operands' own order
+        assert route(lib, mode, *modes(0, 12, 4, 4))["form"] == PRODUCT
+    assert route(lib, 0, *modes(15, 4, 3, 4))["form"] == SHORT_K   # 2^15 of 16 x 8 x 16
+    assert route(lib, 2, *modes(0, 15, 4, 4))["form"] == PRODUCT   # matrix cores
+    assert route(lib, 2, *modes(0, 18, 4, 4))["form"] == SHORT_K
