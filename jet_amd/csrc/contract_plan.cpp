@@ -723,11 +723,24 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
         return d;
     }
 
-    // Few outputs and many k: one pass over both operands in place (also
-    // where neither needs a permutation: the split-K kernel reads a row once
-    // per output it takes part in; only single products are its own: 2^22 k
-    // 16 us against 23).
-    if (d.chunks == 1 && (d.need_a || d.need_b || d.M * d.N > 1) && std::max(d.size_a, d.size_b) >= (int64_t(1) << 16) &&
+    // Few outputs and many k: one pass over both operands in place, in two
+    // launches.  With copies to spare it is the fastest but for what the fused
+    // pass does in one launch (4x2 outputs over 2^12 k 14 us, fused 5.5; batches of
+    // 2^20 multiply-adds 13 and 6, of 2^22 14 and 13-19).  In the operands' own order
+    // the table's kernels read a row once per output it takes part in, out of the
+    // caches, and are faster up to 2^24 multiply-adds, 2^23 in complex128 (16x4
+    // outputs over 2^12 k 12 us, table 4.6; 8x2 over 2^18 32 and 17, 2^20 42 and 34,
+    // 2^21 and more 0.5-0.9 of theirs), for 2x2 outputs up to a quarter of that (2^21
+    // k 21-33 us, table 25-42); but not where they too take two launches for almost
+    // no outputs (2x1 over 2^15 7.3 us, table 9.3).  Single products of unpermuted
+    // operands stay there (2^22 k 16 us against 23).
+    const int few = d.M == 2 && d.N == 2 ? 2 : 0;
+    const bool dot_pays =
+        copies ? d.K > (int64_t(1) << kFusedMaxLog2K) || work > double(1 << 20)
+               : work > double(1 << ((elem_bytes == 8 ? 24 : 23) - few)) ||
+                     (d.M * d.N <= 4 && d.K >= (1 << 14) && work <= double(1 << 18));
+    if (d.chunks == 1 && dot_pays && (d.need_a || d.need_b || d.M * d.N > 1) &&
+        std::max(d.size_a, d.size_b) >= (int64_t(1) << 16) &&
         plan_stream_dot(elem_bytes, A, EA, B, EB, C, d.dot)) {
         d.stream_dot = true;
         d.gemm_kernel = kGemmSplitK;

@@ -439,11 +439,14 @@ __global__ __launch_bounds__(256) void cgemm_shortk_rows_kernel(GemmArgs g, int6
     }
 }
 
+// One work-group per output, its threads k apart.  Bound by L2: each output reads
+// its operands' rows (64x64x1024 7 us).  Sums in FP64, as in the other forms for
+// few outputs and many k, which cost nothing beside the reads.
 template <class R>
 __global__ __launch_bounds__(256) void cgemm_smallred_kernel(GemmArgs g)
 {
     using C2 = typename Vec<R>::c;
-    __shared__ R red[2][256];
+    __shared__ double red[2][256];
     const int64_t o = blockIdx.x;
     const int64_t n = o % g.N;
     const int64_t rest = o / g.N;
@@ -451,13 +454,14 @@ __global__ __launch_bounds__(256) void cgemm_smallred_kernel(GemmArgs g)
     const int64_t b = rest / g.M;
     const C2 *a = static_cast<const C2 *>(g.A) + b * g.sA + m * g.lda;
     const C2 *bb = static_cast<const C2 *>(g.B) + b * g.sB + n * g.ldb;
-    R sr = 0, si = 0;
+    double sr = 0, si = 0;
     for (int64_t k = threadIdx.x; k < g.K; k += 256) {
         const C2 x = a[k], y = bb[k];
-        sr = fma(x.x, y.x, sr);
-        sr = fma(-x.y, y.y, sr);
-        si = fma(x.x, y.y, si);
-        si = fma(x.y, y.x, si);
+        const double xr = x.x, xi = x.y, yr = y.x, yi = y.y;
+        sr = fma(xr, yr, sr);
+        sr = fma(-xi, yi, sr);
+        si = fma(xr, yi, si);
+        si = fma(xi, yr, si);
     }
     red[0][threadIdx.x] = sr;
     red[1][threadIdx.x] = si;
@@ -470,7 +474,7 @@ __global__ __launch_bounds__(256) void cgemm_smallred_kernel(GemmArgs g)
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        static_cast<C2 *>(g.C)[b * g.sC + m * g.ldc + n] = C2{red[0][0], red[1][0]};
+        static_cast<C2 *>(g.C)[b * g.sC + m * g.ldc + n] = C2{R(red[0][0]), R(red[1][0])};
 }
 
 // ---------------------------------------------------------------------------

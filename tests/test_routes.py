@@ -5,12 +5,16 @@ tests/native/route_check.cpp).
   every precision mode, whatever kernel the table names for their shape.
 * The in-place form for a few k and columns is for problems with enough rows or
   work per batch value, and large enough to hide its chain of sums.
+* The two-launch form for few outputs leaves small problems to the fused pass,
+  and in the operands' own order to the table; all of them sum in FP64.
 """
 import ctypes
+import math
 import os
 import random
 import subprocess
 
+import numpy as np
 import pytest
 
 from jet_amd import _native as nat
@@ -109,3 +113,41 @@ def test_short_k_where_it_pays(lib):
     assert route(lib, 0, *modes(15, 4, 3, 4))["form"] == SHORT_K   # 2^15 of 16 x 8 x 16
     assert route(lib, 2, *modes(0, 15, 4, 4))["form"] == PRODUCT   # matrix cores
     assert route(lib, 2, *modes(0, 18, 4, 4))["form"] == SHORT_K
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+def test_few_outputs(lib, mode):
+    rng = random.Random(3)
+    for shape in ((0, 4, 2, 12), (1, 3, 1, 12), (4, 2, 2, 12), (6, 1, 1, 12)):
+        assert route(lib, mode, *modes(*shape, rng))["form"] == FUSED, shape
+    for shape in ((0, 4, 2, 14), (0, 1, 1, 20), (0, 2, 1, 22), (6, 3, 3, 12)):
+        assert route(lib, mode, *modes(*shape, rng))["form"] == FEW_OUTPUTS, shape
+    for shape in ((0, 4, 2, 12), (2, 2, 2, 13), (0, 4, 2, 16), (0, 3, 1, 18), (4, 3, 1, 12)):
+        r = route(lib, mode, *modes(*shape))
+        assert r["form"] == PRODUCT and r["kernel"] in (1, 6), (shape, r)
+    for shape in ((0, 2, 1, 22), (0, 4, 2, 20), (4, 3, 3, 15)):
+        assert route(lib, mode, *modes(*shape))["form"] == FEW_OUTPUTS, shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,batch", [
+    (16, 4, 4096, 1), (4, 4, 8192, 4), (2, 2, 4096, 16), (7, 5, 1000, 3), (1, 1, 300, 1),
+    (3, 2, 257, 2)])
+def test_reductions_sum_in_fp64(m, n, k, batch):
+    """In the operands' own order: one rounding to complex64 for each output."""
+    from hiputil import contract, rand_c, say
+    rng = np.random.default_rng(m * n + k)
+    row = (ctypes.c_int32 * 7)(0, *[round(math.log2(x)) for x in (m, n, k, batch)], 1, 1)
+    a, b = rand_c(rng, batch * m * k, np.complex64), rand_c(rng, batch * n * k, np.complex64)
+    say(f"reduction {m}x{n}x{k} batch {batch}")
+    try:
+        nat.check(nat.lib().jet_hip_tuning_set(1, row))
+        got, info = contract(nat.default_context(), a, [0, 1, 3], [batch, m, k], b, [0, 2, 3],
+                             [batch, n, k], [0, 1, 2])
+    finally:
+        nat.check(nat.lib().jet_hip_tuning_set(-1, None))
+    assert info["kernel"] == "valu_reduce"
+    want = np.einsum("bmk,bnk->bmn", a.reshape(batch, m, k).astype(np.complex128),
+                     b.reshape(batch, n, k).astype(np.complex128)).reshape(-1)
+    err = np.abs(got - want)
+    assert np.all(err <= 2.0 ** -23 * np.maximum(np.abs(want.real), np.abs(want.imag)))
