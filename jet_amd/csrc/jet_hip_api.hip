@@ -812,6 +812,8 @@ int jet_hip_autotune_gemm(jet_hip_ctx_t ctx, jet_hip_dtype_t dtype,
             for (int v = 1; v <= gemm_variants(kern); v++) {
                 const GemmChoice c{kern, v};
                 if (!gemm_choice_valid(mode, m, n, k, batch, c)) continue;
+                // one kernel, whatever the variant (launch_gemm)
+                if (kern == kGemmF32Mfma && v > 1 && f32x6_shape(m, n, k)) continue;
                 const bool valu = kern == kGemmSmall || kern == kGemmSmallRed ||
                                   kern == kGemmSplitK;
                 if ((kern == kGemmSmallRed || kern == kGemmSplitK) && outputs > (1 << 20))
