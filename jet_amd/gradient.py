@@ -272,17 +272,6 @@ class AdjointProgram:
         self.dtype = self.dag.dtype
         self._one = nat.DeviceBuffer(16, self.ctx)
         self._one.upload(np.ones(1, self.dtype))
-        # Where the kept region holds the root value and, in each leaf's label
-        # order, the environments.
-        self._root_at = self._region_index(self.root_node, []).item()
-        self._env_at = {w: self._region_index(self.env_node[w], self.leaf_labels[w])
-                        for w in self.wanted}
-
-    def _region_index(self, node: int, order: Sequence[str]) -> np.ndarray:
-        ptr, labels, shape = self.dag.values[node]
-        at = np.arange(max(1, int(np.prod(shape)))).reshape(shape)
-        at = at.transpose([labels.index(l) for l in order]) if order else at
-        return at + (ptr - self.dag._region[0]) // self.dtype.itemsize
 
     def run_region(self, leaf_ptrs: Sequence[int]) -> np.ndarray:
         """The kept region after one execution."""
@@ -291,12 +280,19 @@ class AdjointProgram:
         self.dag.launch(list(leaf_ptrs) + [self._one.ptr])
         return self.dag.kept_region()
 
+    def value_of(self, region: np.ndarray, node: int, order: Sequence[str] = ()) -> np.ndarray:
+        """A kept node's value in a kept region (of any type), as a view."""
+        ptr, labels, shape = self.dag.values[node]
+        first = (ptr - self.dag._region[0]) // self.dtype.itemsize
+        view = np.ndarray(shape, region.dtype, region, first * region.itemsize)
+        return np.transpose(view, [labels.index(l) for l in order]) if order else view
+
     def run(self, leaf_ptrs: Sequence[int]):
         """(root value, {leaf: environment in the leaf's label order})."""
         region = self.run_region(leaf_ptrs)
-        root = complex(region[self._root_at])
-        envs = {w: region[at] for w, at in self._env_at.items()}
-        return root, envs
+        root = complex(self.value_of(region, self.root_node).reshape(-1)[0])
+        return root, {w: self.value_of(region, self.env_node[w], self.leaf_labels[w])
+                      for w in self.wanted}
 
 
 class ParameterizedAmplitude:
@@ -353,7 +349,12 @@ class ParameterizedAmplitude:
         self._bufs = []
         self._leaf_ptrs = []
         self._param_buf = nat.DeviceBuffer(len(self.param_leaf) * 16 * item, self.ctx)
-        self._env_at = np.stack([self.program._env_at[leaf].reshape(-1)
+        # where the kept region holds the root value and each gate's environment
+        at = np.arange(self.program.dag._region[1] // item)
+        where = lambda node, order: self.program.value_of(at, node, order).reshape(-1)
+        self._root_at = where(self.program.root_node, [])[0]
+        self._env_at = np.stack([where(self.program.env_node[leaf],
+                                       self.program.leaf_labels[leaf])
                                  for leaf in self.param_leaf])
         pos = {leaf: j for j, leaf in enumerate(self.param_leaf)}
         for i, d in enumerate(net.data):
@@ -396,7 +397,7 @@ class ParameterizedAmplitude:
             self.set_angles(theta)
         if self.method == "graph":
             region = self.program.run_region(self._leaf_ptrs)
-            self.amplitude = complex(region[self.program._root_at])
+            self.amplitude = complex(region[self._root_at])
             self._envs = region[self._env_at]
             return self.amplitude
         root = self.adjoint.forward(self.leaves)
