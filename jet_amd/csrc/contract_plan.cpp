@@ -692,7 +692,9 @@ ContractionDesc plan_contraction(int elem_bytes, int mode, int layout,
             (void)f32x6_slices(d.M, d.N, d.K, d.batch, &us);
         const double red = d.flops / 8.0 * (mode == 2 ? 32.0 / 18e6 : 16.0 / 9.6e6);
         const double copies = (d.need_a ? 4.0 : 0.0) + (d.need_b ? 4.0 : 0.0);
-        if (us + copies < red) {
+        // and 2.5 us that few tiles take beyond their times (32x32x4096 9.3 us, reduction
+        // 6.5; 64x64x2048 8.4 and 9.9)
+        if (us + 2.5 + copies < red) {
             d.gemm_kernel = mode == 2 ? kGemmF64Mfma : kGemmF32Mfma;
             d.gemm_variant = 0;
         }

@@ -104,7 +104,9 @@ int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n 
 
 
 // out[i] = sum over c of part[c * n + i] (c ascending, accumulated in FP64):
-// the per-chunk results of a GEMM whose K was split into batched chunks.
+// the per-chunk results of a GEMM whose K was split into batched chunks or slices.
+// Few outputs leave this a chain of loads: eight are in flight at a time (the
+// 64 slices of 64x32x8192, with their product, 26.9 -> 11.5 us).
 template <class C2>
 __global__ __launch_bounds__(256) void sum_chunks_kernel(const C2 *__restrict__ part,
                                                          C2 *__restrict__ out, int64_t n,
@@ -113,7 +115,19 @@ __global__ __launch_bounds__(256) void sum_chunks_kernel(const C2 *__restrict__ 
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
          i += int64_t(gridDim.x) * blockDim.x) {
         double re = 0.0, im = 0.0;
-        for (int64_t c = 0; c < chunks; c++) {
+        int64_t c = 0;
+        constexpr int kAhead = 8;
+        for (; c + kAhead <= chunks; c += kAhead) {
+            C2 v[kAhead];
+#pragma unroll
+            for (int e = 0; e < kAhead; e++) v[e] = part[(c + e) * n + i];
+#pragma unroll
+            for (int e = 0; e < kAhead; e++) {
+                re += double(v[e].x);
+                im += double(v[e].y);
+            }
+        }
+        for (; c < chunks; c++) {
             const C2 v = part[c * n + i];
             re += double(v.x);
             im += double(v.y);

@@ -59,7 +59,7 @@ def test_long_k_error(M, N, K, precision):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(32, 4096, 1024), (4096, 32, 4096), (4096, 32, 16384),
-                                   (4000, 17, 16000)])
+                                   (4000, 17, 16000), (100, 100, 1100), (90, 120, 3000)])
 def test_replaced_reductions_error(M, N, K):
     err, _ = _error(M, N, K, nat.PREC_FP32)
     assert err < 2.0 ** -24 * (1.25 + math.sqrt(K) / 48), err

@@ -151,3 +151,15 @@ def test_reductions_sum_in_fp64(m, n, k, batch):
                      b.reshape(batch, n, k).astype(np.complex128)).reshape(-1)
     err = np.abs(got - want)
     assert np.all(err <= 2.0 ** -23 * np.maximum(np.abs(want.real), np.abs(want.imag)))
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (32, 32, 4096, 1), (32, 64, 2048, 1), (64, 32, 2048, 1),         # reductions
+    (64, 64, 4096, 2), (128, 128, 4096, 2), (48, 48, 8192, 2)])      # slices of products
+def test_long_k_with_few_outputs(lib, m, n, k, kernel):
+    """Matrix-core slices in place of a reduction where they are faster with their sum."""
+    i64 = lambda *v: (ctypes.c_int64 * len(v))(*v)
+    out = (ctypes.c_int64 * 5)()
+    assert lib.contraction_route(0, 2, nat.i32([0, 2]), i64(m, k), 2, nat.i32([1, 2]), i64(n, k),
+                                 2, nat.i32([0, 1]), out) == 0
+    assert out[0] == PRODUCT and out[1] == kernel, list(out)
