@@ -181,8 +181,8 @@ int jet_hip_contract_noalloc(jet_hip_plan_t plan, const void *a,
  *
  * Kernel ids (jet_hip_plan_info's gemm_kernel): 0 VALU per output, 1 VALU
  * block reduction, 2 FP32 products on the matrix cores (six BF16 MFMA
- * products of three-piece operands; FP32 MFMA where k, M or N is
- * below 16), 3 FP64 MFMA, 4 split-BF16 3M, 5 split-BF16
+ * products of three-piece operands; FP32 MFMA where k is below
+ * 16), 3 FP64 MFMA, 4 split-BF16 3M, 5 split-BF16
  * 4M, 6 split-K with FP64 partials, 7 split-FP16 4M.  Variants: kernel 2
  * 1 = 128x128 / 2 = 64x128 / 3 = 128x64 block tiles of its FP32 MFMA form
  * (no effect on its BF16 products, which choose tiles by the shape);

@@ -3,7 +3,7 @@
 // Three arithmetic modes, all computing C[b][m][n] = sum_k A[b][m][k] B[b][n][k]
 // (no conjugation, alpha = 1, beta = 0):
 //
-//  * FP32 "4M" (cgemm_embed_kernel; products too short or narrow for
+//  * FP32 "4M" (cgemm_embed_kernel; products too short for
 //    gemm_f32x6.hip): the complex product is the real
 //    product of A viewed as an M x 2K real matrix (re/im interleaved along k)
 //    and the 2K x 2N real matrix B' with B'[2k][2n]=br, B'[2k][2n+1]=bi,

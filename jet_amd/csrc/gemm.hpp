@@ -35,7 +35,7 @@ enum GemmKernel {
     kGemmF32Mfma = 2,   // FP32 products on the matrix cores: three BF16 pieces of
                         // each value and six products (gemm_f32x6.hip), or 4M
                         // complex on v_mfma_f32_16x16x4_f32 where that does
-                        // not apply (k, M or N < 16)
+                        // not apply (k < 16)
     kGemmF64Mfma = 3,   // 4M complex on v_mfma_f64_16x16x4_f64 (gemm_f64.hip)
     kGemmBf16x3 = 4,    // 3M complex, split-BF16, v_mfma_f32_16x16x32_bf16
     kGemmBf16x4m = 5,   // 4M complex, split-BF16, v_mfma_f32_16x16x32_bf16
@@ -82,11 +82,13 @@ inline int64_t splitk_partials(int64_t outputs, int64_t K)
 }
 
 // Whether the FP32 products run on the BF16 matrix cores: the lane offsets are
-// 32 bits (rows to 2^21 k); 32x32 blocks of which less than half would be
-// outputs, and less than one k step, are left to the FP32 MFMA kernel.
+// 32 bits (rows to 2^21 k), and less than one k step is left to the FP32 MFMA kernel.
+// Narrow products waste most of a 32x32 block here, but more of the FP32 kernel's
+// 128x64 tiles (12x3000x1000 14.0 us and 160, 256x10x87 7.7 and 18.9, batches of 300
+// 5x5x64 6.0 and 22).
 inline bool f32x6_shape(int64_t M, int64_t N, int64_t K)
 {
-    return K >= 16 && K <= (int64_t(1) << 21) && M >= 16 && N >= 16;
+    return M >= 1 && N >= 1 && K >= 16 && K <= (int64_t(1) << 21);
 }
 
 // 4M split products with few 128x128 tiles: slices of k (at least 256 each)

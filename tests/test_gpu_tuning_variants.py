@@ -12,8 +12,8 @@ F32 = 2
 
 
 @pytest.mark.parametrize("m,n,k,variants", [
-    (16, 16, 16, [1]), (64, 100, 300, [1]),                     # BF16 products
-    (15, 64, 64, [1, 2, 3]), (64, 64, 12, [1, 2, 3])])          # FP32 MFMA tiles
+    (16, 16, 16, [1]), (64, 100, 300, [1]), (5, 64, 64, [1]),   # BF16 products
+    (15, 64, 12, [1, 2, 3]), (64, 64, 12, [1, 2, 3])])          # FP32 MFMA tiles
 def test_fp32_variants(m, n, k, variants):
     cap = 32
     ks, vs = (ctypes.c_int32 * cap)(), (ctypes.c_int32 * cap)()
