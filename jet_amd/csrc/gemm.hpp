@@ -126,6 +126,12 @@ constexpr TileForm kF32x6Forms[] = {{256, 128, 16, 1, 3.33f, 4.27f, 11.5f},
                                     {64, 64, 16, 3, 0.92f, 0.69f, 1.f},
                                     {64, 32, 32, 2, 1.05f, 0.77f, 0.6f},
                                     {32, 32, 64, 2, 1.1f, 0.8f, 0.4f}};
+// Rows that are not 16-byte aligned (odd k): four times the load instructions, and
+// registers for one work-group of the 32x32 form on a CU.  Predicted / measured us:
+// 1030x1030x1001 106 / 100, 2050x1030x255 44 / 48 (64x64), 300x513x405 12.5 / 14.5
+// (32x32; chosen by the aligned forms' times before, 1030x1030x17 took 24.8, now 8.3).
+constexpr TileForm kF32x6DwordForms[] = {{64, 64, 16, 2, 1.2f, 0.81f, 1.75f},
+                                         {32, 32, 64, 1, 1.25f, 1.23f, 3.7f}};
 constexpr TileForm kF64Forms[] = {{128, 128, 8, 1, 3.8f, 3.92f, 9.f},
                                   {32, 32, 16, 3, 0.70f, 0.523f, 0.83f},
                                   {32, 32, 8, 6, 0.445f, 0.264f, 0.39f}};

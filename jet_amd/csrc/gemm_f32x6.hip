@@ -533,16 +533,17 @@ void launch_f32x6(const GemmArgs &g, hipStream_t stream)
                          reinterpret_cast<uintptr_t>(g.B) % 16 == 0 && g.K % 2 == 0 &&
                          g.lda % 2 == 0 && g.ldb % 2 == 0 &&
                          (g.batch == 1 || (g.sA % 2 == 0 && g.sB % 2 == 0));
+    const int64_t k = g.slices > 1 ? g.slice_k : g.K, count = g.batch * g.slices;
     int form = 0;
-    (void)tile_time(kF32x6Forms, g.M, g.N, g.slices > 1 ? g.slice_k : g.K, g.batch * g.slices,
-                    &form);
-    if (!aligned) { // four times the load instructions: the smaller tiles hide them
-        if (form <= 2)
+    if (!aligned) {
+        (void)tile_time(kF32x6DwordForms, g.M, g.N, k, count, &form);
+        if (form == 0)
             launch_tile<64, 64, 2, 2, 1, 3, true, 1>(g, stream);
         else
             launch_tile<32, 32, 1, 1, 4, 2, true, 1>(g, stream);
         return;
     }
+    (void)tile_time(kF32x6Forms, g.M, g.N, k, count, &form);
     switch (form) {
     case 0:
         launch_tile<256, 128, 2, 2, 1, 3, false>(g, stream);
