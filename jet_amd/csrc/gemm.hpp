@@ -135,14 +135,19 @@ constexpr TileForm kF32x6DwordForms[] = {{64, 64, 16, 2, 1.2f, 0.81f, 1.75f},
 constexpr TileForm kF64Forms[] = {{128, 128, 8, 1, 3.8f, 3.92f, 9.f},
                                   {32, 32, 16, 3, 0.70f, 0.523f, 0.83f},
                                   {32, 32, 8, 6, 0.445f, 0.264f, 0.39f}};
+// Tiles of a launch: fewer than 2^32 threads at 512 each.  Products with more of
+// every form's take the first form, whose tiles are the largest.
+constexpr int64_t kMaxTiles = (int64_t(1) << 23) - 1;
 template <int COUNT>
 inline double tile_time(const TileForm (&forms)[COUNT], int64_t M, int64_t N, int64_t K,
                         int64_t batch, int *form)
 {
     constexpr int64_t kCus = 256;
     double best = -1.0;
+    if (form) *form = 0;
     for (int i = 0; i < COUNT; i++) {
         const TileForm &f = forms[i];
+        if (i > 0 && ceil_div(M, f.bm) * ceil_div(N, f.bn) > kMaxTiles) continue;
         const int64_t per_cu = ceil_div(ceil_div(M, f.bm) * ceil_div(N, f.bn) * batch, kCus);
         const double wait = f.alone * double(ceil_div(per_cu, f.occ)), work = f.full * double(per_cu);
         const double us = double(ceil_div(K, f.kt)) * (wait > work ? wait : work) +

@@ -24,3 +24,14 @@ extern "C" int contraction_route(int mode, int ra, const int32_t *ma, const int6
     out[4] = (int64_t)d.workspace;
     return 0;
 }
+
+// Tiles of the form that an FP32 (aligned rows or not) or FP64 product takes.
+extern "C" int64_t product_tiles(int fp64, int aligned, int64_t M, int64_t N, int64_t K)
+{
+    int form = 0;
+    const TileForm *f = fp64 ? kF64Forms : aligned ? kF32x6Forms : kF32x6DwordForms;
+    (void)(fp64      ? tile_time(kF64Forms, M, N, K, 1, &form)
+           : aligned ? tile_time(kF32x6Forms, M, N, K, 1, &form)
+                     : tile_time(kF32x6DwordForms, M, N, K, 1, &form));
+    return ceil_div(M, f[form].bm) * ceil_div(N, f[form].bn);
+}

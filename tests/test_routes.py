@@ -163,3 +163,14 @@ def test_long_k_with_few_outputs(lib, m, n, k, kernel):
     assert lib.contraction_route(0, 2, nat.i32([0, 2]), i64(m, k), 2, nat.i32([1, 2]), i64(n, k),
                                  2, nat.i32([0, 1]), out) == 0
     assert out[0] == PRODUCT and out[1] == kernel, list(out)
+
+
+@pytest.mark.parametrize("fp64,aligned,threads", [(0, 1, 256), (0, 0, 256), (1, 1, 512)])
+@pytest.mark.parametrize("m", [1, 16, 32, 40])
+def test_tiles_fit_a_launch(lib, fp64, aligned, threads, m):
+    """Long thin products: 2^32 threads is what a launch takes."""
+    lib.product_tiles.restype = ctypes.c_int64
+    lib.product_tiles.argtypes = [ctypes.c_int] * 2 + [ctypes.c_int64] * 3
+    for log2n in (20, 24, 28, 29):
+        for a, b in ((m, 1 << log2n), (1 << log2n, m)):
+            assert lib.product_tiles(fp64, aligned, a, b, 16) * threads < 2 ** 32, log2n
