@@ -17,7 +17,8 @@ Workloads:
       the split 16-bit MFMA GEMM of --split (default split-FP16: each
       complex64 operand row scaled by a power of two, split into hi + lo
       FP16, three products per real product, FP32 accumulation), then the
-      --compare modes (default split-BF16) and plain FP32 MFMA; one
+      --compare modes (default split-BF16) and plain FP32 (products at FP32
+      accuracy as six BF16 products); one
       execution in complex128 on FP64 MFMA is the FP64 reference of the
       relative errors.  Each execution's per-slice amplitudes are summed by
       the FP64 compensated reduction.
@@ -26,7 +27,7 @@ Workloads:
       positions in both index orders, re/im ~ N(0, 1/2); one
       2^14 x 2^14 x 2^14 complex GEMM behind the index permutations.
       A step is one ContractTensors call with the --split GEMM (the headline
-      value); the plain FP32-MFMA path is timed beside it, and complex128 on
+      value); the plain FP32 path is timed beside it, and complex128 on
       FP64 MFMA gives the FP64 reference the error is measured against.
 
 value (c2) = slices/s, with the operands resident in HBM when the timed region
@@ -59,6 +60,8 @@ def mfma_peak(family: str) -> float:
         return PEAK["fp16"]
     if "fp64" in family:
         return PEAK["fp64"]
+    if "fp32" in family:  # six BF16 products (the FP32 instruction only below 16 k)
+        return PEAK["bf16"] / 6
     return PEAK["fp32"]
 
 # Split 16-bit MFMA modes: precision constant name, network precision string,
@@ -76,9 +79,10 @@ ROCPROF_NAME = {"gemm_bf16x3_4m_mfma": ("cgemm_x4m_kernel bf16", "cgemm_x4m_wide
                                        "cgemm_x4m_wide_kernel f16 192x128",
                                        "cgemm_x4m_persist_kernel f16"),
                 "gemm_bf16x3_mfma": ("cgemm_bf16x3_kernel",),
-                "gemm_fp32_mfma": ("cgemm_embed_kernel f32 128x128", "cgemm_embed_kernel f32 128x64",
-                                   "cgemm_embed_kernel f32 64x128"),
-                "gemm_fp64_mfma": ("cgemm_embed_kernel f64 128x64",),
+                "gemm_fp32_mfma": ("cgemm_f32x6_kernel 256x128", "cgemm_f32x6_kernel 128x128",
+                                   "cgemm_f32x6_kernel 64x64", "cgemm_f32x6_kernel 64x32",
+                                   "cgemm_f32x6_kernel 32x32"),
+                "gemm_fp64_mfma": ("cgemm_f64_kernel 128x128", "cgemm_f64_kernel 32x32"),
                 "permute_bits": ("permute_bits_kernel c64",)}
 
 
@@ -629,7 +633,7 @@ def run_c2(args):
         "unit": "slices/s",
         "ms_per_step": round(ms16 / steps, 3),
         "dtype": f"c64 ({label} MFMA, three terms, fp32 accumulate, on MFMA-bound steps; "
-                 "fp32 MFMA elsewhere)",
+                 "fp32 as six BF16 products elsewhere)",
         "config": {"workload": "c2: one amplitude of a seeded 7x7-qubit grid random circuit, "
                                f"depth 14, complex64, {path_desc} sliced on 12 bond-2 indices "
                                "(4096 slices); a step is one batched execution of "
@@ -928,7 +932,7 @@ def run_c3(args):
     forms, tuning = ub.forms(), ub.tuning
     ub.close()
     del ub
-    # The same batch on FP32 MFMA: the complex64 error floor the split run is
+    # The same batch in plain FP32: the complex64 error floor the split run is
     # judged beside.
     ub32 = UnevenBatch(jobs, dtype=np.complex64, precision="fp32", ctx=ctx)
     ub32.launch()
@@ -956,7 +960,7 @@ def run_c3(args):
     ub64.close()
     errs, errs32 = np.array(errs), np.array(errs32)
     log(f"c3: per-amplitude rel err max {errs.max():.2e} median {np.median(errs):.2e} "
-        f"(fp32 MFMA: max {errs32.max():.2e} median {np.median(errs32):.2e}); "
+        f"(plain fp32: max {errs32.max():.2e} median {np.median(errs32):.2e}); "
         f"per circuit normwise {', '.join(f'{x:.2e}' for x in norm_errs)}; "
         f"c2 slices {slice_err:.2e}")
     return {
@@ -964,7 +968,7 @@ def run_c3(args):
         "value": round(flops / (ms * 1e-3) / 1e12, 3),
         "unit": "TFLOP/s",
         "ms_per_step": round(ms, 3),
-        "dtype": f"c64 ({SPLIT_LABEL[args.split]} MFMA on MFMA-bound steps, fp32 MFMA elsewhere)",
+        "dtype": f"c64 ({SPLIT_LABEL[args.split]} MFMA on MFMA-bound steps, fp32 as six BF16 products elsewhere)",
         "config": {"workload": "c3: uneven batch in one hipGraph launch: 24 amplitudes of a "
                                "5x5 depth-14, 16 of a 6x6 depth-12 and 24 of a 6x7 depth-10 "
                                f"seeded grid circuit, plus {n_exec * per_exec} slices of the "
@@ -1050,7 +1054,7 @@ def run_c4(args):
         "value": round(1e3 / ms, 3),
         "unit": "gradients/s",
         "ms_per_step": round(ms, 3),
-        "dtype": "c64 (FP32 MFMA / VALU per step), gradient accumulated in FP64",
+        "dtype": "c64 (FP32 as six BF16 products / VALU per step), gradient accumulated in FP64",
         "config": {"workload": "c4: |<b|C(theta)|0>|^2 and its gradient for all fSim angles "
                                "of a seeded 6x6-qubit depth-10 grid circuit (angles ~ U(0, 2 pi)); "
                                "a step is one forward + adjoint evaluation",
