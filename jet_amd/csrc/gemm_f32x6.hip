@@ -1,14 +1,14 @@
 // gemm_f32x6.hip -- complex64 GEMM at FP32 accuracy on the BF16 matrix cores
 // (gfx950): the FP32 products of every precision mode.
 //
-// Each FP32 value is the sum of three BF16 pieces, 2^24 x = h + m + l (rounded
+// Each FP32 value is the sum of three BF16 pieces, 2^16 x = h + m + l (rounded
 // to nearest: 3 x 8 significant bits, so the sum is exact; unscaled, the pieces
-// of values under 2^-110 would fall below BF16's smallest normal), and a real
-// product keeps the six terms hh, hm, mh, hl, lh, mm; the dropped ones are below
-// 2^-24 of it.  Values from 2^103 on and sums from 2^79 on leave the scaled
-// range, and with infinities and NaN their outputs are computed again with the
-// FP32 instruction.  The scaling is one VALU instruction per value (4096^3 2380 ->
-// 2420 us, 64x32 tiles 3% more).
+// of values under 2^-110 would fall below BF16's smallest subnormal), and a
+// real product keeps the six terms hh, hm, mh, hl, lh, mm; the dropped ones are
+// below 2^-24 of it.  Values from 2^111 on and sums from 2^95 on leave the scaled
+// range, and with infinities and NaN their 32x32 blocks are computed again with
+// the FP32 instruction (all of 4096^3 10.8 ms).  The scaling is one VALU
+// instruction per value (4096^3 2380 -> 2405 us, 64x32 tiles 3% more).
 //
 // Four real products make 24 v_mfma_f32_32x32x16_bf16 per 32x32
 // block and 16 k: at BF16's rate (16 times FP32's on the same matrix cores)
@@ -67,10 +67,11 @@ __device__ __forceinline__ float high_bf16(uint32_t p)
     return __uint_as_float(p & 0xffff0000u);
 }
 
-// 2^24 x = h + m + l, each rounded to nearest: 24 significant bits, so the sum is
-// exact, and no piece of any FP32 number is below BF16's smallest normal.
-// Sums of products carry 2^48 until they are stored.
-constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;
+// 2^16 x = h + m + l, each rounded to nearest: 24 significant bits, so the sum is
+// exact, and the last bit of any FP32 number is at least BF16's smallest
+// subnormal, which the conversions and the products keep.  Sums of products
+// carry 2^32 until they are stored.
+constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l)
 {
     h = pack_bf16(a * kScale, b * kScale);

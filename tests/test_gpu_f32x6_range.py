@@ -37,14 +37,14 @@ def test_scaled_operands_are_bitwise_the_same(ctx, table, M, N, K, shift):  # no
     s = np.float32(2.0 ** shift)
     say(f"operands scaled by 2^{-shift}")
     want = _run(ctx, a.reshape(-1), b.reshape(-1), 1, M, N, K)
-    # columns of b at most 2^77, so that its values stay below 2^103
+    # columns of b at most 2^77, so that its values stay in the scaled range
     cap = np.float32(2.0 ** max(-100, min(shift, 76)))
     got = _run(ctx, (a / s).reshape(-1), (b * cap).reshape(-1), 1, M, N, K)
     ratio = np.float32(cap / s)
     assert np.array_equal(got, want * ratio)
 
 
-@pytest.mark.parametrize("rows,columns", [(103, -103), (126, -126), (126, 0), (60, 30), (50, 62)])
+@pytest.mark.parametrize("rows,columns", [(103, -103), (126, -126), (126, 0), (60, 30), (50, 62), (112, -112), (48, 48)])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_large_values(ctx, table, M, N, K, rows, columns):  # noqa: F811
     """Some rows and all columns scaled: the sums' range is left, FP32's is not."""
